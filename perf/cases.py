@@ -261,12 +261,6 @@ class _Pd:
         self.solver.Update(self.data, self.params)
         return {"X": self.X, "V": self.V, "XTilde": self.XTilde}
 
-    def __del__(self):
-        if hasattr(self, "solver"):
-            self.solver.close()
-        if self.sphere is not None:
-            self.sphere.close()
-
 
 class _Ipc:
     def __init__(self, case, seed):
@@ -290,10 +284,6 @@ class _Ipc:
         if not self.solver.Update(self.data, self.params):
             raise RuntimeError("the IPC step failed: %r" % self.solver.stats())
         return {"X": self.X, "V": self.V}
-
-    def __del__(self):
-        if hasattr(self, "solver"):
-            self.solver.close()
 
 
 class _Borrowed:
@@ -348,10 +338,6 @@ class _Coo:
         self.solver.Solve(self.n, self.b.data_ptr(), self.x.data_ptr(), self.vals.data_ptr(), self.vals.numel(),
                           self.rows.data_ptr(), self.cols.data_ptr())
         return {"x": self.x}
-
-    def __del__(self):
-        if hasattr(self, "solver"):
-            self.solver.close()
 
 
 def _coo_tol(case):

@@ -229,13 +229,24 @@ void BandCholesky<T>::factor(int n, const std::vector<int>& rowptr, const std::v
         throw Error(kFactorFailed, e.what());
     }
     const int bw = f.bw;
-    std::vector<T> ld((size_t)(bw + 1) * n);
-    for (int i = 0; i < n; ++i)
-        for (int d = 0; d <= bw; ++d) ld[(size_t)d * n + i] = (T)f.Lb[(size_t)i * (bw + 1) + d];
     const std::vector<int> sys = band_systems(n, rowptr, col, f.perm);
     n_ = n;
     bw_ = bw;
     nsys_ = (int)sys.size() - 1;
+    inverse_ = InverseOperator<T>();
+    if (InverseOperator<T>::suits(bw, sys)) {
+        try {
+            inverse_.setup(f, sys, stream);
+            return;
+        } catch (const Error& e) {  // no room for the inverse: the band solve needs far less
+            if (e.code != kOutOfMemory) throw;
+            (void)hipGetLastError();
+            inverse_ = InverseOperator<T>();
+        }
+    }
+    std::vector<T> ld((size_t)(bw + 1) * n);
+    for (int i = 0; i < n; ++i)
+        for (int d = 0; d <= bw; ++d) ld[(size_t)d * n + i] = (T)f.Lb[(size_t)i * (bw + 1) + d];
     ring_ = ring_rows(bw);
     ld_.alloc(ld.size());
     perm_.alloc(n);
@@ -253,6 +264,11 @@ void BandCholesky<T>::factor(int n, const std::vector<int>& rowptr, const std::v
 
 template <class T> void BandCholesky<T>::solve(const T* b, T* x, hipStream_t stream, const int* skip) const {
     SBS_REQUIRE(n_ > 0, "BandCholesky: solve before factor");
+    if (inverse_.ready()) {
+        inverse_.load_rhs(b, stream, skip);
+        inverse_.apply(x, stream, skip);
+        return;
+    }
     hipLaunchKernelGGL(band_solve_kernel<T>, dim3(24 * ceil_div((size_t)nsys_, 8)), dim3(kThreads),
                        lds_bytes<T>(ring_), stream, n_, bw_, ring_, nsys_, (const int*)sys_.get(), ld_.get(), perm_.get(),
                        b, x, ybuf_.get(), skip);

@@ -17,12 +17,16 @@
 //     wavefront with register broadcasts -- forward for L, backward for L^T;
 //     the band update reads the previous (next) bw rows' values from a ring
 //     of bw + 64 rows in LDS, so the limit is the bandwidth (up to the LDS a
-//     workgroup may use), not the number of rows.
+//     workgroup may use), not the number of rows;
+//   * where the product with the explicit inverse is faster than that chain
+//     of blocks (InverseOperator::suits), the factor only gives the inverse
+//     and a solve is that product.
 #pragma once
 
 #include <vector>
 
 #include "common.hpp"
+#include "direct_inverse.hpp"
 
 namespace sbs {
 
@@ -34,6 +38,10 @@ public:
     // x = A^-1 b for 3 interleaved right-hand sides; kernels return early
     // when *skip != 0 (device flag, may be null).
     void solve(const T* b, T* x, hipStream_t stream, const int* skip) const;
+    // The product with the explicit inverse, when that is how this factor is
+    // solved (null otherwise): the caller may write the right-hand side in its
+    // place and take the outer loop's end with it.
+    const InverseOperator<T>* inverse() const { return inverse_.ready() ? &inverse_ : nullptr; }
     int n() const { return n_; }
     int bandwidth() const { return bw_; }
     int systems() const { return nsys_; }
@@ -46,6 +54,7 @@ private:
     DevBuf<int> perm_;      // position i holds original row perm[i]
     DevBuf<int> sys_;       // first row of each independent system (nsys+1)
     DevBuf<T> ybuf_;        // forward-sweep result, 3 per row
+    InverseOperator<T> inverse_;
 };
 
 }  // namespace sbs

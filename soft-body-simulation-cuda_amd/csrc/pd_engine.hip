@@ -446,6 +446,22 @@ __global__ void rhs_kernel(int nv, RhsGather<T> g, T* __restrict__ out, const in
     st3(out, v, x, y, z);
 }
 
+// The same with component c of vertex v at out[c * stride + pos[v]]: the
+// right-hand side where the product with the inverse reads it.
+template <class T>
+__global__ void rhs_planes_kernel(int nv, RhsGather<T> g, const int* __restrict__ pos, int stride, T* __restrict__ out,
+                                  const int* __restrict__ skip) {
+    if (skip && *skip) return;
+    const unsigned v = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    if (v >= (unsigned)nv) return;
+    const int p = pos[v];
+    T x, y, z;
+    g.at(v, x, y, z);
+    out[p] = x;
+    out[(size_t)stride + p] = y;
+    out[2 * (size_t)stride + p] = z;
+}
+
 // Jacobi + Chebyshev global step (getErrorKern pdUtil.cu:195-214 and
 // chebyshevKern pdUtil.cu:216-226 fused per vertex).
 template <class T>
@@ -2308,6 +2324,18 @@ template <class T> void PdEngine<T>::enqueue_step(PdData<T>& data, const PdParam
                     hipLaunchKernelGGL(outer_decide_kernel, dim3(1), dim3(64), 0, stream_, (const double*)slots_.get(),
                                        nv_, params.tol, ctl, skip);
                 }
+            } else if (direct_ && direct_->inverse()) {
+                // the product with the inverse: it takes the outer loop's error
+                // and decision with it
+                const InverseOperator<T>* inv = direct_->inverse();
+                tick(kKRhs, true);
+                hipLaunchKernelGGL(rhs_planes_kernel<T>, dim3(vb), dim3(kTpb), 0, stream_, nv_, g, inv->pos(),
+                                   inv->stride(), inv->rhs(), skip);
+                tick(kKRhs, false);
+                tick(kKDirect, true);
+                inv->apply_outer(OuterStep<T>{sn_.get(), prev_.get(), &ctl->err, &ctl->outer_done, params.tol}, stream_,
+                                 skip);
+                tick(kKDirect, false);
             } else {
                 tick(kKRhs, true);
                 hipLaunchKernelGGL(rhs_kernel<T>, dim3(vb), dim3(kTpb), 0, stream_, nv_, g, rhs_.get(), skip);

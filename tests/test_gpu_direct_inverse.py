@@ -1,0 +1,49 @@
+"""The direct global solve by the product with the explicit inverse: sizes at
+the edges of its tiles (8 rows per workgroup, 4-value loads, 1,024 columns per
+pass) and scenes of several systems, against a dense FP64 solve of the
+exported matrix."""
+import numpy as np
+import pytest
+
+from sbs_amd import capi, mesh
+from sbs_amd.pd import PdSolver, SolverData, SolverParams, SolverType
+
+pytestmark = pytest.mark.gpu
+
+# vertices per body: 8, 12, 27, 120, 1,000 (a pass less 24), 1,056 (a pass and 32)
+SCENES = {"8": [(1, 1, 1)], "12": [(2, 1, 1)], "27": [(2, 2, 2)], "120": [(3, 4, 5)], "1000": [(9, 9, 9)],
+          "1056": [(10, 11, 7)], "three": [(2, 2, 2), (4, 3, 1), (1, 2, 1)]}
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("name", list(SCENES))
+def test_solve_against_dense(name, precision):
+    scene = mesh.make_scene([dict(nx=d[0], ny=d[1], nz=d[2], seed=3 + i, pin_top=True, origin=(3.0 * i, 0.0, 0.0))
+                             for i, d in enumerate(SCENES[name])])
+    data = SolverData(scene, precision)
+    pd = PdSolver(128, data)
+    pd.SetGlobalSolver(SolverType.CuSolverCholesky)
+    p = SolverParams(numIterations=2, dt=1.0 / 60.0, tol=0.0)
+    pd.Update(data, p)
+    ex = pd.export_system()
+    n = scene.nv
+    A = np.zeros((n, n))
+    for v in range(n):
+        A[v, ex["col"][ex["rowptr"][v]:ex["rowptr"][v + 1]]] = ex["val"][ex["rowptr"][v]:ex["rowptr"][v + 1]]
+    rng = np.random.default_rng(1)
+    b = (rng.normal(size=(n, 3)) * np.diag(A)[:, None]).astype(data.dtype)
+    db, dx = capi.DeviceArray.from_numpy(b), capi.DeviceArray(b.nbytes)
+    pd.solve(db.ptr, dx.ptr, p)
+    x = dx.download(data.dtype, (n, 3)).astype(np.float64)
+    inv = np.linalg.inv(A)
+    ref = inv @ b.astype(np.float64)
+    # each entry of the inverse and each product is rounded once, and at most
+    # n / 1024 + 24 sums stand between a product and the result; in FP64 the
+    # factor's own error (condition number times the unit roundoff) adds to it
+    u = np.finfo(data.dtype).eps / 2
+    bound = (3 + n / 1024 + 24) * u * (np.abs(inv) @ np.abs(b.astype(np.float64)))
+    if precision == 64:
+        bound = bound + 1e-12 * np.abs(ref).max()
+    assert np.all(np.abs(x - ref) <= bound)
+    pd.close()
+    data.free()

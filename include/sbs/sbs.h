@@ -401,7 +401,7 @@ typedef struct SbsIpcParams {
     double dhat;          /* barrier distance (queries kept while d^2 <= dhat)  */
     double tol;           /* Newton stop: |p|_inf / dt < tol                    */
     int max_iterations;   /* Newton iterations per step (failure beyond)        */
-    double lin_tol;       /* Jacobi-PCG: |r| <= lin_tol |g|                     */
+    double lin_tol;       /* PCG: |r| <= lin_tol |g|                     */
     int lin_max_iter;
 } SbsIpcParams;
 
@@ -435,7 +435,8 @@ int sbs_ipc_update(SbsIpc* h, SbsIpcData* data, const SbsIpcParams* params, int*
 int sbs_ipc_set_elastic(SbsIpc* h, int model);
 int sbs_ipc_reset(SbsIpc* h);
 /* Linear solver of the Newton system.  Every type that converges to the
- * solution (0, 1, 2) runs Jacobi-PCG to lin_tol; 3 (plain Jacobi iteration)
+ * solution (0, 1, 2) runs PCG to lin_tol, preconditioned by the diagonal and
+ * by inverted blocks of the vertices in contact; 3 (plain Jacobi iteration)
  * is rejected. */
 int sbs_ipc_set_linear_solver(SbsIpc* h, int solver_type);
 int sbs_ipc_set_stream(SbsIpc* h, void* hip_stream);

@@ -1,5 +1,5 @@
 // FP64 IPC step on gfx950: energies, gradients, element Hessians with the
-// positive-definite projection, matrix-free Jacobi-PCG and the Newton loop.
+// positive-definite projection, assembled block-Jacobi PCG and the Newton loop.
 // Reference citations are per kernel; see ipc_engine.hpp for the layout.
 #include <algorithm>
 #include <cfloat>
@@ -21,7 +21,7 @@ namespace sbs {
 namespace {
 
 constexpr int kT = 256;   // threads per block of the per-element kernels
-constexpr int kQB = 16;   // queries per block of the barrier kernel (LDS: 2 x 144 doubles per query)
+constexpr int kQB = 32;   // queries per block of the barrier kernel (LDS: 144 doubles per query)
 constexpr double kG = 9.8;  // GravityEnergy::g (gravity.h:14)
 
 unsigned nblk(size_t n) { return (unsigned)std::max<size_t>(1, (n + kT - 1) / kT); }
@@ -581,70 +581,15 @@ __global__ void __launch_bounds__(kT) ipc_nh_kernel(int nt, const uint32_t* tet,
                 for (int k = 0; k < 3; ++k) atomicAdd(&diag[3 * (size_t)tv[a] + k], H[13 * (3 * a + k)]);
 }
 
-// makePD (matrix.h:441-518) on a 12x12 matrix held in LDS (entry (i, j) of
-// this thread at M[(12 i + j) * kQB + lane]): cyclic Jacobi over the pairs
-// p < q, rotations skipped when |a_pq| < 1e-9, at most 20 sweeps; eigenvalues
-// below 1e-6 raised to 1e-6; M <- V diag V^T.
-__device__ void make_pd_lds(double* M, double* V, int lane) {
-    auto m = [&](int i, int j) -> double& { return M[(12 * i + j) * kQB + lane]; };
-    auto v = [&](int i, int j) -> double& { return V[(12 * i + j) * kQB + lane]; };
-    for (int i = 0; i < 12; ++i)
-        for (int j = 0; j < 12; ++j) v(i, j) = i == j ? 1.0 : 0.0;
-    for (int sweep = 0; sweep < 20; ++sweep) {
-        bool converged = true;
-        for (int p = 0; p < 12; ++p)
-            for (int q = p + 1; q < 12; ++q) {
-                const double apq = m(p, q);
-                if (fabs(apq) < 1e-9) continue;
-                converged = false;
-                const double app = m(p, p), aqq = m(q, q);
-                const double theta = 0.5 * (aqq - app) / apq;
-                double t;
-                if (fabs(theta) > 1e10) t = 0.5 / theta;
-                else t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(1.0 + theta * theta));
-                const double c = 1.0 / sqrt(1.0 + t * t), s = t * c;
-                m(p, q) = 0.0;
-                m(q, p) = 0.0;
-                m(p, p) = c * c * app - 2.0 * s * c * apq + s * s * aqq;
-                m(q, q) = s * s * app + 2.0 * s * c * apq + c * c * aqq;
-                for (int k = 0; k < 12; ++k) {
-                    if (k == p || k == q) continue;
-                    const double akp = m(k, p), akq = m(k, q);
-                    m(k, p) = c * akp - s * akq;
-                    m(p, k) = m(k, p);
-                    m(k, q) = s * akp + c * akq;
-                    m(q, k) = m(k, q);
-                }
-                for (int k = 0; k < 12; ++k) {
-                    const double vkp = v(k, p), vkq = v(k, q);
-                    v(k, p) = c * vkp - s * vkq;
-                    v(k, q) = s * vkp + c * vkq;
-                }
-            }
-        if (converged) break;
-    }
-    double lamv[12];
-    for (int i = 0; i < 12; ++i) lamv[i] = fmax(m(i, i), 1e-6);
-    for (int i = 0; i < 12; ++i)
-        for (int j = i; j < 12; ++j) {
-            double s = 0.0;
-            for (int k = 0; k < 12; ++k) s += v(i, k) * lamv[k] * v(j, k);
-            m(i, j) = s;  // only the upper triangle is read back: rows below are still the input
-        }
-    for (int i = 1; i < 12; ++i)
-        for (int j = 0; j < i; ++j) m(i, j) = m(j, i);
-}
-
 // Barrier of one query (Barrier::gradHessianKern, barrier.cu:99-173),
 // scaled by coef: gradient coef b'(d) grad d into g (atomics), and with hq
-// the Hessian coef (b''(d) grad d grad d^T + b'(d) hess d), made positive
-// definite.  Queries with d > dhat^2 contribute nothing.
+// the Hessian coef (b''(d) grad d grad d^T + b'(d) hess d) into hq, made
+// positive definite by ipc_barrier_pd_kernel.  Queries with d > dhat^2
+// contribute nothing.
 __global__ void __launch_bounds__(kQB) ipc_barrier_kernel(long long nq, const QueryKey* qk, const int* dtype,
                                                           const double* qd, const double* X, double dhat, double kappa,
-                                                          double coef, const unsigned char* fixed, double* g,
-                                                          double* hq, double* diag) {
-    __shared__ double sM[144 * kQB];
-    __shared__ double sV[144 * kQB];
+                                                          double coef, double* g, double* hq) {
+    __shared__ double M[144 * kQB];
     const long long i = (long long)blockIdx.x * kQB + threadIdx.x;
     if (i >= nq) return;  // no barrier below
     const double d = qd[i];
@@ -654,7 +599,6 @@ __global__ void __launch_bounds__(kQB) ipc_barrier_kernel(long long nq, const Qu
     const uint32_t vv[4] = {k.v0, k.v1, k.v2, k.v3};
     const int lane = threadIdx.x;
     double gd[12];
-    double* M = sM;
     if (hq)
         for (int e = 0; e < 144; ++e) M[e * kQB + lane] = 0.0;
     ipc::distance_derivatives((int)k.type, dtype[i], P, gd, [&](int a, int b, const ipc::M3& blk, double sgn) {
@@ -666,18 +610,108 @@ __global__ void __launch_bounds__(kQB) ipc_barrier_kernel(long long nq, const Qu
     for (int j = 0; j < 12; ++j) atomicAdd(&g[3 * (size_t)vv[j / 3] + j % 3], coef * d1 * gd[j]);
     if (!hq) return;
     const double d2 = barrier_d2(d, dhat, kappa);
-    for (int a = 0; a < 12; ++a)
-        for (int b = 0; b < 12; ++b) {
-            double& e = M[(12 * a + b) * kQB + lane];
-            e = coef * (d2 * gd[a] * gd[b] + d1 * e);
-        }
-    make_pd_lds(M, sV, lane);
     double* H = hq + 144 * (size_t)i;
-    for (int e = 0; e < 144; ++e) H[e] = M[e * kQB + lane];
-    if (diag)
-        for (int a = 0; a < 4; ++a)
-            if (!fixed[vv[a]])
-                for (int r = 0; r < 3; ++r) atomicAdd(&diag[3 * (size_t)vv[a] + r], H[13 * (3 * a + r)]);
+    for (int a = 0; a < 12; ++a)
+        for (int b = 0; b < 12; ++b)
+            H[12 * a + b] = coef * (d2 * gd[a] * gd[b] + d1 * M[(12 * a + b) * kQB + lane]);
+}
+
+// makePD (matrix.h:441-518) of the active queries' Hessians in hq, and their
+// diagonal into the Jacobi diagonal of the free vertices: cyclic Jacobi over
+// the pairs p < q, rotations skipped when |a_pq| < 1e-9, at most 20 sweeps;
+// eigenvalues below 1e-6 raised to 1e-6; H <- V diag V^T.  The pairs keep
+// their order (what the skipped entries leave behind depends on it).  Sixteen
+// lanes work on a query, lane k < 12 on the entries of row and column k, with
+// the matrix in LDS: a rotation is one round of LDS reads, the angle (found
+// by every lane) and one round of writes.  That chain, 66 rotations a sweep,
+// bounds it: one query per thread took 803 us with the derivatives for the
+// 16^3 contact scene (22,536 queries), the two kernels now 44 + 316 us (a
+// tournament order of the pairs would be faster and was not kept: it ends
+// with other skipped entries, 1e-12 m from the reference order's step).
+constexpr int kPdLanes = 16;
+constexpr int kPdQueries = 64 / kPdLanes;
+constexpr int kPdLd = 13;  // row stride in LDS: rows and columns spread over the banks
+__global__ void __launch_bounds__(64) ipc_barrier_pd_kernel(long long nq, const QueryKey* __restrict__ qk,
+                                                            const double* __restrict__ qd, double dhat2,
+                                                            const unsigned char* __restrict__ fixed,
+                                                            double* __restrict__ hq, double* __restrict__ diag) {
+    __shared__ double sm[kPdQueries][12][kPdLd], sv[kPdQueries][12][kPdLd];
+    const int grp = threadIdx.x / kPdLanes, k = threadIdx.x % kPdLanes;
+    const long long i = (long long)blockIdx.x * kPdQueries + grp;
+    const bool live = i < nq && qd[i < nq ? i : 0] <= dhat2;
+    if (__ballot(live) == 0ull) return;  // the block is one wavefront
+    double(*m)[kPdLd] = sm[grp];
+    double(*v)[kPdLd] = sv[grp];
+    const bool mine = live && k < 12;
+    double* H = hq + 144 * (size_t)(live ? i : 0);
+    if (mine)
+        for (int j = 0; j < 12; ++j) {
+            m[k][j] = H[12 * k + j];
+            v[k][j] = j == k ? 1.0 : 0.0;
+        }
+    __syncthreads();
+    bool run = mine;
+    for (int sweep = 0; sweep < 20; ++sweep) {
+        bool moved = false;
+        for (int p = 0; p < 12; ++p)
+            for (int q = p + 1; q < 12; ++q) {
+                // (a block of one wavefront: LDS accesses keep their order)
+                double apq = 0.0, app = 0.0, aqq = 0.0, akp = 0.0, akq = 0.0, vkp = 0.0, vkq = 0.0;
+                if (run) {
+                    apq = m[p][q];
+                    app = m[p][p];
+                    aqq = m[q][q];
+                    akp = m[k][p];
+                    akq = m[k][q];
+                    vkp = v[k][p];
+                    vkq = v[k][q];
+                }
+                const bool turn = run && !(fabs(apq) < 1e-9);
+                if (__ballot(turn) == 0ull) continue;
+                __builtin_amdgcn_wave_barrier();
+                if (turn) {
+                    moved = true;
+                    // t = sign(theta) / (|theta| + sqrt(1 + theta^2)), theta = (a_qq - a_pp) / (2 a_pq)
+                    const double h = 0.5 * (aqq - app);
+                    const double den = fabs(h) + sqrt(h * h + apq * apq);
+                    const double t = (h == 0.0 || (h > 0.0) == (apq > 0.0) ? fabs(apq) : -fabs(apq)) / den;
+                    const double c = 1.0 / sqrt(1.0 + t * t), s = t * c;
+                    double np = c * akp - s * akq, nq_ = s * akp + c * akq;
+                    if (k == p) {
+                        np = c * c * app - 2.0 * s * c * apq + s * s * aqq;
+                        nq_ = 0.0;
+                    }
+                    if (k == q) {
+                        np = 0.0;
+                        nq_ = s * s * app + 2.0 * s * c * apq + c * c * aqq;
+                    }
+                    m[k][p] = np;
+                    m[p][k] = np;
+                    m[k][q] = nq_;
+                    m[q][k] = nq_;
+                    v[k][p] = c * vkp - s * vkq;
+                    v[k][q] = s * vkp + c * vkq;
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+        // a sweep without a rotation ends the query (its 12 lanes take the same decision)
+        run = run && moved;
+        if (__ballot(run) == 0ull) break;
+    }
+    __syncthreads();
+    if (!mine) return;
+    for (int j = 0; j < 12; ++j) {
+        // the product of entry (min, max) in both lanes, so H stays symmetric
+        const int r = j < k ? j : k, c = j < k ? k : j;
+        double s = 0.0;
+        for (int e = 0; e < 12; ++e) s += v[r][e] * fmax(m[e][e], 1e-6) * v[c][e];
+        H[12 * k + j] = s;
+        if (j == k && diag) {
+            const QueryKey q = qk[i];
+            const uint32_t vv = k < 3 ? q.v0 : k < 6 ? q.v1 : k < 9 ? q.v2 : q.v3;
+            if (!fixed[vv]) atomicAdd(&diag[3 * (size_t)vv + k % 3], s);
+        }
+    }
 }
 
 // DOFElimination (ipc.cu:55-80): zero gradient and identity row/column on fixed vertices.
@@ -688,23 +722,6 @@ __global__ void ipc_fix_kernel(int nv, const unsigned char* fixed, double* g, do
         g[3 * (size_t)v + k] = 0.0;
         if (diag) diag[3 * (size_t)v + k] = 1.0;
     }
-}
-
-// Start of a Jacobi-PCG solve (n = 3 N_v): x = 0, r = b, z = D^-1 b and the
-// block partials of r.z and r.r.
-__global__ void ipc_pcg_init_kernel(int n, const double* b, const double* diag, double* x, double* r, double* z,
-                                    double* parts) {
-    const int i = blockIdx.x * kT + threadIdx.x;
-    double v[2] = {0.0, 0.0};
-    if (i < n) {
-        const double ri = b[i], zi = ri / diag[i];
-        x[i] = 0.0;
-        r[i] = ri;
-        z[i] = zi;
-        v[0] = ri * zi;
-        v[1] = ri * ri;
-    }
-    block_sums<2>(v, parts);
 }
 
 // The tets' 12x12 Hessian blocks summed into 3x3 blocks per (vertex, vertex)
@@ -813,6 +830,170 @@ __global__ void ipc_contact_rows_kernel(int nv, const int* __restrict__ count, c
     }
     crow[v] = lo;
 }
+
+// Preconditioner blocks.  The contact terms are orders of magnitude stiffer
+// than the rest of H and couple the vertices of a query, which a diagonal
+// does not see: the diagonal alone needs 545 iterations to 1e-10 where the
+// two 16^3 cubes touch over 690 vertices, and 52 without the contact terms.
+// So the free vertices with contact entries are taken in Morton order of
+// their positions, kBlkVerts at a time, and H restricted to such a block is
+// inverted exactly (96 x 96); every other unknown keeps its diagonal.  210
+// iterations then (290 -> 76 for a 6x4x5 scene); blocks of 16, 32 and 64
+// vertices need 229, 210 and 164, and 32 is what fits a workgroup's LDS.
+constexpr int kBlkVerts = 32;
+constexpr int kBlkN = 3 * kBlkVerts;
+constexpr size_t kBlkLds = ((size_t)kBlkN * kBlkN + 4 * kBlkN) * sizeof(double);
+
+// Morton keys (21 bits per axis) of the positions in cells of the given size.
+__global__ void ipc_morton_kernel(int nv, const double* __restrict__ X, double inv_cell,
+                                  unsigned long long* __restrict__ key, int* __restrict__ id) {
+    const int v = blockIdx.x * kT + threadIdx.x;
+    if (v >= nv) return;
+    unsigned long long k = 0;
+    for (int a = 0; a < 3; ++a) {
+        const double c = fmin(fmax(floor(X[3 * (size_t)v + a] * inv_cell) + 1048576.0, 0.0), 2097151.0);
+        unsigned long long x = (unsigned long long)c;  // spread to every third bit
+        x = (x | (x << 32)) & 0x001f00000000ffffull;
+        x = (x | (x << 16)) & 0x001f0000ff0000ffull;
+        x = (x | (x << 8)) & 0x100f00f00f00f00full;
+        x = (x | (x << 4)) & 0x10c30c30c30c30c3ull;
+        x = (x | (x << 2)) & 0x1249249249249249ull;
+        k |= x << (2 - a);
+    }
+    key[v] = k;
+    id[v] = v;
+}
+
+// flag[i] = 1 where vertex order[i] is free and has contact entries.
+__global__ void ipc_block_flags_kernel(int nv, const int* __restrict__ order, const int* __restrict__ crow,
+                                       const unsigned char* __restrict__ fixed, int* __restrict__ flag) {
+    const int i = blockIdx.x * kT + threadIdx.x;
+    if (i >= nv) return;
+    const int v = order[i];
+    flag[i] = !fixed[v] && crow[v + 1] > crow[v];
+}
+// Their list, each vertex's place in it (-1: not in it), and its length.
+__global__ void ipc_block_list_kernel(int nv, const int* __restrict__ order, const int* __restrict__ flag,
+                                      const int* __restrict__ pos, int* __restrict__ list, int* __restrict__ slot,
+                                      int* __restrict__ count) {
+    const int i = blockIdx.x * kT + threadIdx.x;
+    if (i >= nv) return;
+    const int v = order[i];
+    slot[v] = flag[i] ? pos[i] : -1;
+    if (flag[i]) list[pos[i]] = v;
+    if (i == nv - 1) *count = pos[i] + flag[i];
+}
+
+// H restricted to block blockIdx.x, inverted by Gauss-Jordan without pivoting
+// (the block is symmetric positive definite), into binv (row-major; unused
+// places are identity).  An elastic Hessian need not be positive definite: a
+// block with a pivot that is not positive takes its diagonal instead.  The
+// matrix is assembled in LDS and then held in registers, 6 x 6 entries per
+// thread (rows ty + 16 i, columns tx + 16 j); a step passes the pivot's row
+// and column through LDS, double-buffered, so it costs one barrier and 36
+// products.  All blocks run side by side in 68 us; with the matrix left in
+// LDS it was 484 us.
+__global__ void __launch_bounds__(kT) ipc_block_invert_kernel(
+    const int* __restrict__ count, const int* __restrict__ list, const int* __restrict__ slot,
+    const long long* __restrict__ rowptr, const int* __restrict__ col, const double* __restrict__ val,
+    const int* __restrict__ crow, const int* __restrict__ ccol, const double* __restrict__ cval,
+    const double* __restrict__ mass, const double* __restrict__ hv, const double* __restrict__ diag,
+    double* __restrict__ binv) {
+    static_assert(kT == 256 && kBlkN == 96, "16 x 16 threads of 6 x 6 entries");
+    constexpr int kTile = kBlkN / 16;
+    extern __shared__ double A[];  // kBlkN x kBlkN, then two pivot rows and columns
+    double* srow = A + kBlkN * kBlkN;
+    double* scol = srow + 2 * kBlkN;
+    const int n = *count, b0 = blockIdx.x * kBlkVerts, nb = min(kBlkVerts, n - b0), tid = threadIdx.x;
+    if (nb <= 0) return;
+    for (int e = tid; e < kBlkN * kBlkN; e += kT) A[e] = e / kBlkN == e % kBlkN && e / kBlkN >= 3 * nb ? 1.0 : 0.0;
+    __syncthreads();
+    if (tid < 3 * nb) {  // one thread per row: its entries are added in a fixed order
+        const int v = list[b0 + tid / 3], r = tid % 3;
+        double* row = A + tid * kBlkN;
+        row[tid] += mass[v];
+        if (hv)
+            for (int c = 0; c < 3; ++c) row[tid - r + c] += hv[9 * (size_t)v + 3 * r + c];
+        for (long long k = rowptr[v]; k < rowptr[v + 1]; ++k) {
+            const int j = slot[col[k]] - b0;
+            if (j >= 0 && j < nb)
+                for (int c = 0; c < 3; ++c) row[3 * j + c] += val[9 * k + 3 * r + c];
+        }
+        for (int k = crow[v]; k < crow[v + 1]; ++k) {
+            const int j = slot[ccol[k]] - b0;
+            if (j >= 0 && j < nb)
+                for (int c = 0; c < 3; ++c) row[3 * j + c] += cval[9 * (size_t)k + 3 * r + c];
+        }
+    }
+    __syncthreads();
+    const int tx = tid & 15, ty = tid >> 4;
+    double a[kTile][kTile];
+#pragma unroll
+    for (int i = 0; i < kTile; ++i)
+#pragma unroll
+        for (int j = 0; j < kTile; ++j) a[i][j] = A[(ty + 16 * i) * kBlkN + tx + 16 * j];
+    bool bad = false;
+#pragma unroll
+    for (int pi = 0; pi < kTile; ++pi)
+        for (int pp = 0; pp < 16; ++pp) {
+            const int p = 16 * pi + pp;
+            double* pr = srow + (p & 1) * kBlkN;
+            double* pc = scol + (p & 1) * kBlkN;
+            if (ty == pp)
+#pragma unroll
+                for (int j = 0; j < kTile; ++j) pr[tx + 16 * j] = a[pi][j];
+            if (tx == pp)
+#pragma unroll
+                for (int i = 0; i < kTile; ++i) pc[ty + 16 * i] = a[i][pi];
+            __syncthreads();
+            const double d = pr[p];
+            bad = bad || !(d > 0.0);  // every thread sees the same pivots
+            const double inv = 1.0 / d;
+            double rv[kTile], cv[kTile];
+#pragma unroll
+            for (int j = 0; j < kTile; ++j) rv[j] = pr[tx + 16 * j] * inv;
+            if (tx == pp) rv[pi] = inv;
+#pragma unroll
+            for (int i = 0; i < kTile; ++i) cv[i] = pc[ty + 16 * i];
+            if (tx == pp)
+#pragma unroll
+                for (int i = 0; i < kTile; ++i) a[i][pi] = 0.0;
+#pragma unroll
+            for (int i = 0; i < kTile; ++i)
+#pragma unroll
+                for (int j = 0; j < kTile; ++j) a[i][j] -= cv[i] * rv[j];
+            if (ty == pp)
+#pragma unroll
+                for (int j = 0; j < kTile; ++j) a[pi][j] = rv[j];
+        }
+    // symmetrise through LDS
+#pragma unroll
+    for (int i = 0; i < kTile; ++i)
+#pragma unroll
+        for (int j = 0; j < kTile; ++j) A[(ty + 16 * i) * kBlkN + tx + 16 * j] = a[i][j];
+    __syncthreads();
+    double* out = binv + (size_t)blockIdx.x * kBlkN * kBlkN;
+#pragma unroll
+    for (int i = 0; i < kTile; ++i)
+#pragma unroll
+        for (int j = 0; j < kTile; ++j) {
+            const int r = ty + 16 * i, c = tx + 16 * j;
+            double x = 0.5 * (a[i][j] + A[c * kBlkN + r]);
+            if (bad) x = r != c ? 0.0 : r < 3 * nb ? 1.0 / diag[3 * (size_t)list[b0 + r / 3] + r % 3] : 1.0;
+            out[r * kBlkN + c] = x;
+        }
+}
+
+// The blocks of a solve: none when verts is 0.
+struct BlockView {
+    int verts = 0;                // vertices in blocks
+    const int* list = nullptr;    // their ids
+    const int* slot = nullptr;    // per vertex its place, -1: its diagonal
+    const double* inv = nullptr;  // kBlkN x kBlkN per block
+};
+constexpr int kBlkHalf = 2;                      // threads per unknown of a block
+constexpr int kBlkPer = kBlkN / kBlkHalf;        // products per thread
+static_assert(kBlkN * kBlkHalf <= kT, "one workgroup per preconditioner block");
 
 // Jacobi-PCG on H p = g in two launches per iteration (n = 3 N_v).  The
 // scalars stay on the device: out = [rz0, rr, pq, alpha, beta, |b|, rz (even
@@ -963,19 +1144,94 @@ __global__ void __launch_bounds__(kT) ipc_pcg_prod_kernel(
     block_sums<1>(pq, parts);
 }
 
+// The unknown of this thread in the launches that apply the preconditioner:
+// the first blocks workgroups take a block each (kBlkHalf threads per
+// unknown, the first of them its owner), the others kT unknowns each, without
+// those in blocks.  Returns -1 for a thread without one.
+__device__ __forceinline__ int precond_unknown(const BlockView& B, int blocks, int n, bool& in_block) {
+    in_block = (int)blockIdx.x < blocks;
+    if (in_block) {
+        const int u = threadIdx.x % kBlkN, p = (int)blockIdx.x * kBlkVerts + u / 3;
+        return threadIdx.x < kBlkN && p < B.verts ? 3 * B.list[p] + u % 3 : -1;
+    }
+    const int i = ((int)blockIdx.x - blocks) * kT + threadIdx.x;
+    return i < n && (blocks == 0 || B.slot[i / 3] < 0) ? i : -1;
+}
+// This thread's kBlkPer entries of the block's inverse (symmetric, so row
+// `unknown` is read as a column: consecutive threads, consecutive entries).
+__device__ __forceinline__ void precond_load(const BlockView& B, double (&bv)[kBlkPer]) {
+    const int u = threadIdx.x % kBlkN, h = threadIdx.x / kBlkN;
+    if (h >= kBlkHalf) return;
+    const double* inv = B.inv + (size_t)blockIdx.x * kBlkN * kBlkN + (size_t)h * kBlkPer * kBlkN + u;
+#pragma unroll
+    for (int j = 0; j < kBlkPer; ++j) bv[j] = inv[(size_t)j * kBlkN];
+}
+// z = B r in a block's workgroup (r: this thread's unknown, 0 without one).
+__device__ __forceinline__ double precond_apply(const double (&bv)[kBlkPer], double r) {
+    __shared__ double sr[kBlkN], sz[kBlkHalf][kBlkN];
+    const int u = threadIdx.x % kBlkN, h = threadIdx.x / kBlkN;
+    if (h == 0) sr[u] = r;
+    __syncthreads();
+    if (h < kBlkHalf) {
+        double s = 0.0;
+#pragma unroll
+        for (int j = 0; j < kBlkPer; ++j) s += bv[j] * sr[h * kBlkPer + j];
+        sz[h][u] = s;
+    }
+    __syncthreads();
+    double z = 0.0;
+    if (h == 0)
+#pragma unroll
+        for (int k = 0; k < kBlkHalf; ++k) z += sz[k][u];
+    return z;
+}
+
+// Start of a solve (n = 3 N_v): x = 0, r = b, z = M^-1 b and the block
+// partials of r.z and r.r.
+__global__ void __launch_bounds__(kT) ipc_pcg_init_kernel(int n, BlockView B, int blocks, const double* __restrict__ b,
+                                                          const double* __restrict__ diag, double* __restrict__ x,
+                                                          double* __restrict__ r, double* __restrict__ z,
+                                                          double* __restrict__ parts) {
+    bool in_block;
+    const int i = precond_unknown(B, blocks, n, in_block);
+    double ri = 0.0, zi = 0.0;
+    if (i >= 0) ri = b[i];
+    if (in_block) {
+        double bv[kBlkPer];
+        precond_load(B, bv);
+        zi = precond_apply(bv, ri);
+    } else if (i >= 0) {
+        zi = ri / diag[i];
+    }
+    double v[2] = {0.0, 0.0};
+    if (i >= 0) {
+        x[i] = 0.0;
+        r[i] = ri;
+        z[i] = zi;
+        v[0] = ri * zi;
+        v[1] = ri * ri;
+    }
+    block_sums<2>(v, parts);
+}
+
 // Update launch of iteration it: alpha = rz_it / p.q, x += alpha p,
-// r -= alpha q, z = D^-1 r and the block partials of r.z and r.r.  H not positive along p
-// finishes the solve with the iterate kept.
-__global__ void __launch_bounds__(kT) ipc_pcg_update_kernel(int n, int nb_prod, const double* __restrict__ prod_parts,
-                                                            int it, const double* __restrict__ p,
+// r -= alpha q, z = M^-1 r and the block partials of r.z and r.r.  H not
+// positive along p finishes the solve with the iterate kept.  A block's
+// inverse (73 KB) is requested before the stop word and the partial sums.
+__global__ void __launch_bounds__(kT) ipc_pcg_update_kernel(int n, BlockView B, int blocks, int nb_prod,
+                                                            const double* __restrict__ prod_parts, int it,
+                                                            const double* __restrict__ p,
                                                             const double* __restrict__ q,
                                                             const double* __restrict__ diag, double* __restrict__ x,
                                                             double* __restrict__ r, double* __restrict__ z,
                                                             double* __restrict__ upd_parts, double* __restrict__ out,
                                                             int* __restrict__ ctl) {
-    const int i = blockIdx.x * kT + threadIdx.x;
+    bool in_block;
+    const int i = precond_unknown(B, blocks, n, in_block);
+    double bv[kBlkPer];
+    if (in_block) precond_load(B, bv);
     double pi = 0.0, qi = 0.0, ri = 0.0, di = 1.0, xi = 0.0;
-    if (i < n) {
+    if (i >= 0) {
         pi = p[i];
         qi = q[i];
         ri = r[i];
@@ -1000,11 +1256,11 @@ __global__ void __launch_bounds__(kT) ipc_pcg_update_kernel(int n, int nb_prod, 
         out[2] = pq;
         out[3] = al;
     }
+    ri -= al * qi;
+    const double zi = in_block ? precond_apply(bv, ri) : ri / di;
     double v[2] = {0.0, 0.0};
-    if (i < n) {
+    if (i >= 0) {
         x[i] = xi + al * pi;
-        ri = ri - al * qi;
-        const double zi = ri / di;
         r[i] = ri;
         z[i] = zi;
         v[0] = ri * zi;
@@ -1057,6 +1313,17 @@ IpcEngine::IpcEngine(const IpcData& data) {
         }
         for (int v = 0; v < nv_; ++v)
             if (deg[v] > 0) area[v] /= deg[v];
+        {   // Morton cells of half the bounding box's edge per cube root of the vertex count
+            double lo[3] = {X[0], X[1], X[2]}, hi[3] = {X[0], X[1], X[2]};
+            for (int v = 0; v < nv_; ++v)
+                for (int k = 0; k < 3; ++k) {
+                    lo[k] = std::min(lo[k], X[3 * (size_t)v + k]);
+                    hi[k] = std::max(hi[k], X[3 * (size_t)v + k]);
+                }
+            const double ext = std::max({hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]});
+            const double cell = 0.5 * ext / std::cbrt((double)nv_);
+            inv_cell_ = cell > 0.0 && std::isfinite(cell) ? 1.0 / cell : 1.0;
+        }
         area_.alloc(nv_);
         SBS_HIP(hipMemcpy(area_.get(), area.data(), area.size() * sizeof(double), hipMemcpyHostToDevice));
         if (ntri_ > 0) {
@@ -1080,6 +1347,13 @@ IpcEngine::IpcEngine(const IpcData& data) {
     pcg_ctl_.alloc(2);
     pcg_parts_.alloc(2 * (size_t)nblk(n3));
     prod_parts_.alloc(nblk((size_t)kRowLanes * n3));
+    vkey_.alloc(nv_); vkey_s_.alloc(nv_); vid_.alloc(nv_); order_.alloc(nv_);
+    blk_flag_.alloc(nv_); blk_pos_.alloc(nv_); blk_list_.alloc(nv_); blk_slot_.alloc(nv_);
+    blk_count_.alloc(1);
+    SBS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&ipc_block_invert_kernel),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBlkLds));
+    SBS_HIP(hipHostMalloc((void**)&host_blk_, sizeof(int), hipHostMallocDefault));
+    host_blk_[0] = 0;
     SBS_HIP(hipHostMalloc((void**)&host_, 8 * sizeof(double), hipHostMallocDefault));
     SBS_HIP(hipHostMalloc((void**)&host_ctl_, 2 * sizeof(int), hipHostMallocDefault));
     hipLaunchKernelGGL(ipc_precompute_kernel, dim3(nblk(nt_)), dim3(kT), 0, stream_, nt_, data.Tet,
@@ -1144,6 +1418,7 @@ void IpcEngine::build_rows(const std::vector<uint32_t>& tet) {
 IpcEngine::~IpcEngine() {
     if (host_) (void)hipHostFree(host_);
     if (host_ctl_) (void)hipHostFree(host_ctl_);
+    if (host_blk_) (void)hipHostFree(host_blk_);
 }
 
 void IpcEngine::set_stream(hipStream_t s) {
@@ -1255,11 +1530,15 @@ void IpcEngine::gradient(const double* X, bool hessian, double kap) {
                        (const double*)d_.XTilde, d_.mass, h2, g_.get(), hessian ? diag_.get() : nullptr);
     elastic(X, h2, hessian);
     body_gradient(X, h2, hessian);
-    if (nq_ > 0)
+    if (nq_ > 0) {
         hipLaunchKernelGGL(ipc_barrier_kernel, dim3((unsigned)((nq_ + kQB - 1) / kQB)), dim3(kQB), 0, stream_, nq_,
                            col_->queries(), (const int*)qtype_.get(), (const double*)qd_.get(), X, p_.dhat, kap, h2,
-                           (const unsigned char*)fixed_.get(), g_.get(), hessian ? hq_.get() : nullptr,
-                           hessian ? diag_.get() : nullptr);
+                           g_.get(), hessian ? hq_.get() : nullptr);
+        if (hessian)
+            hipLaunchKernelGGL(ipc_barrier_pd_kernel, dim3((unsigned)((nq_ + kPdQueries - 1) / kPdQueries)), dim3(64), 0,
+                               stream_, nq_, col_->queries(), (const double*)qd_.get(), p_.dhat * p_.dhat,
+                               (const unsigned char*)fixed_.get(), hq_.get(), diag_.get());
+    }
     if (hessian)
         hipLaunchKernelGGL(ipc_fix_kernel, dim3(nblk(nv_)), dim3(kT), 0, stream_, nv_,
                            (const unsigned char*)fixed_.get(), g_.get(), diag_.get());
@@ -1318,7 +1597,7 @@ void IpcEngine::update_kappa(const double* X) {
     if (nq_ > 0)
         hipLaunchKernelGGL(ipc_barrier_kernel, dim3((unsigned)((nq_ + kQB - 1) / kQB)), dim3(kQB), 0, stream_, nq_,
                            col_->queries(), (const int*)qtype_.get(), (const double*)qd_.get(), X, p_.dhat, 1.0, h2,
-                           (const unsigned char*)fixed_.get(), g_.get(), (double*)nullptr, (double*)nullptr);
+                           g_.get(), (double*)nullptr);
     SBS_HIP(hipGetLastError());
     const double gb = nq_ > 0 ? max_abs(g_.get(), n3) : 0.0;
     kappa_ = gb > 1e-9 ? std::max(100.0, ge / gb) : 100.0;
@@ -1332,12 +1611,18 @@ void IpcEngine::update_kappa(const double* X) {
 int IpcEngine::solve() {
     constexpr int kPcgChunk = 16;
     const int n = 3 * nv_;
-    const unsigned nb = nblk(n), nrb = nblk((size_t)kRowLanes * n);
+    BlockView B;
+    int blocks = 0;
+    if (blk_verts_ > 0) {
+        B = BlockView{blk_verts_, blk_list_.get(), blk_slot_.get(), blk_inv_.get()};
+        blocks = (blk_verts_ + kBlkVerts - 1) / kBlkVerts;
+    }
+    const unsigned nb = nblk(n) + (unsigned)blocks, nrb = nblk((size_t)kRowLanes * n);
     double* out = out_.get();  // [0] rz0, [1] rr, [2] pq, [3] alpha, [4] beta, [5] |b|, [6..7] rz by parity
     int* ctl = pcg_ctl_.get();
     double* upd_parts = pcg_parts_.get();
     double* prod_parts = prod_parts_.get();
-    hipLaunchKernelGGL(ipc_pcg_init_kernel, dim3(nb), dim3(kT), 0, stream_, n, (const double*)g_.get(),
+    hipLaunchKernelGGL(ipc_pcg_init_kernel, dim3(nb), dim3(kT), 0, stream_, n, B, blocks, (const double*)g_.get(),
                        (const double*)diag_.get(), p_dir_.get(), r_.get(), z_.get(), upd_parts);
     hipLaunchKernelGGL(sum_parts_kernel<2>, dim3(1), dim3(kT), 0, stream_, (int)nb, (const double*)upd_parts, out);
     SBS_HIP(hipMemcpyAsync(host_, out, 2 * sizeof(double), hipMemcpyDeviceToHost, stream_));
@@ -1362,16 +1647,19 @@ int IpcEngine::solve() {
                            (const double*)z_.get(), (const double*)dir[it & 1], dir[(it + 1) & 1], q_.get(), (int)nb,
                            (const double*)upd_parts, it, p_.lin_max_iter, p_.lin_tol, prod_parts, out, ctl);
     };
+    const size_t ord = pcg_solve_++;
+    const int guess = ord < pcg_seen_.size() ? pcg_seen_[ord] : pcg_seen_.empty() ? 0 : pcg_seen_.back();
     for (int launched = 0; launched < p_.lin_max_iter;) {
-        // the first check after 9/10 of the previous solve's iterations, then
-        // every kPcgChunk or launched/8 (a check costs the GPU ~30 us idle, a
-        // launch after the solve finished ~2.5 us)
-        const int want = launched == 0 ? std::max(kPcgChunk, pcg_last_ * 9 / 10) : std::max(kPcgChunk, launched / 8);
+        // the first check after 9/10 of the iterations that the same solve of
+        // the previous step took (the previous solve where that step had
+        // fewer), then every kPcgChunk or launched/8 (a check costs the GPU
+        // ~30 us idle, a launch after the solve finished ~2.5 us)
+        const int want = launched == 0 ? std::max(kPcgChunk, guess * 9 / 10) : std::max(kPcgChunk, launched / 8);
         const int chunk = std::min(want, p_.lin_max_iter - launched);
         for (int j = 0; j < chunk; ++j) {
             const int it = launched + j;
             product(it);
-            hipLaunchKernelGGL(ipc_pcg_update_kernel, dim3(nb), dim3(kT), 0, stream_, n, (int)nrb,
+            hipLaunchKernelGGL(ipc_pcg_update_kernel, dim3(nb), dim3(kT), 0, stream_, n, B, blocks, (int)nrb,
                                (const double*)prod_parts, it, (const double*)dir[(it + 1) & 1], (const double*)q_.get(),
                                (const double*)diag_.get(), p_dir_.get(), r_.get(), z_.get(), upd_parts, out, ctl);
         }
@@ -1382,7 +1670,8 @@ int IpcEngine::solve() {
         SBS_HIP(hipStreamSynchronize(stream_));
         if (host_ctl_[0]) break;
     }
-    pcg_last_ = host_ctl_[1];
+    if (ord < pcg_seen_.size()) pcg_seen_[ord] = host_ctl_[1];
+    else if (ord == pcg_seen_.size() && ord < kPcgSeen) pcg_seen_.push_back(host_ctl_[1]);
     return host_ctl_[1];
 }
 
@@ -1436,6 +1725,50 @@ void IpcEngine::assemble_contact() {
     SBS_HIP(hipGetLastError());
 }
 
+// The vertices of the preconditioner's blocks: free, with contact entries, in
+// Morton order of the positions (sorted once per step).  Their number lands in
+// host_blk_ by the next wait for the stream.
+void IpcEngine::list_blocks(const double* X) {
+    const unsigned vb = nblk(nv_);
+    size_t b1 = 0, b2 = 0;
+    SBS_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, b1, vkey_.get(), vkey_s_.get(), vid_.get(), order_.get(), nv_, 0,
+                                               63, stream_));
+    SBS_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, b2, blk_flag_.get(), blk_pos_.get(), nv_, stream_));
+    if (std::max(b1, b2) > ctmp_bytes_) {
+        ctmp_bytes_ = std::max(b1, b2);
+        ctmp_.alloc(ctmp_bytes_);
+    }
+    if (!ordered_) {
+        hipLaunchKernelGGL(ipc_morton_kernel, dim3(vb), dim3(kT), 0, stream_, nv_, X, inv_cell_, vkey_.get(),
+                           vid_.get());
+        SBS_HIP(hipcub::DeviceRadixSort::SortPairs(ctmp_.get(), b1, vkey_.get(), vkey_s_.get(), vid_.get(),
+                                                   order_.get(), nv_, 0, 63, stream_));
+        ordered_ = true;
+    }
+    hipLaunchKernelGGL(ipc_block_flags_kernel, dim3(vb), dim3(kT), 0, stream_, nv_, (const int*)order_.get(),
+                       (const int*)crow_.get(), (const unsigned char*)fixed_.get(), blk_flag_.get());
+    SBS_HIP(hipcub::DeviceScan::ExclusiveSum(ctmp_.get(), b2, blk_flag_.get(), blk_pos_.get(), nv_, stream_));
+    hipLaunchKernelGGL(ipc_block_list_kernel, dim3(vb), dim3(kT), 0, stream_, nv_, (const int*)order_.get(),
+                       (const int*)blk_flag_.get(), (const int*)blk_pos_.get(), blk_list_.get(), blk_slot_.get(),
+                       blk_count_.get());
+    SBS_HIP(hipGetLastError());
+    SBS_HIP(hipMemcpyAsync(host_blk_, blk_count_.get(), sizeof(int), hipMemcpyDeviceToHost, stream_));
+}
+
+// The inverses of the blk_verts_ listed vertices' blocks.
+void IpcEngine::invert_blocks() {
+    const size_t blocks = ((size_t)blk_verts_ + kBlkVerts - 1) / kBlkVerts, need = blocks * kBlkN * kBlkN;
+    if (need > blk_inv_.n) blk_inv_.alloc(need + need / 4);
+    const size_t np = 2 * ((size_t)nblk(3 * (size_t)nv_) + blocks);
+    if (np > pcg_parts_.n) pcg_parts_.alloc(np);
+    hipLaunchKernelGGL(ipc_block_invert_kernel, dim3((unsigned)blocks), dim3(kT), kBlkLds, stream_,
+                       (const int*)blk_count_.get(), (const int*)blk_list_.get(), (const int*)blk_slot_.get(),
+                       (const long long*)row_ptr_.get(), (const int*)row_col_.get(), (const double*)row_val_.get(),
+                       (const int*)crow_.get(), (const int*)cbcol_.get(), (const double*)cval_.get(), d_.mass,
+                       hv_live_ ? (const double*)hv_.get() : nullptr, (const double*)diag_.get(), blk_inv_.get());
+    SBS_HIP(hipGetLastError());
+}
+
 // SearchDirection (ipc.cu:230-239): gradient and Hessian at X, elimination,
 // p = H^-1 g; false when the gradient holds NaN or Inf.
 bool IpcEngine::search_direction(const double* X) {
@@ -1444,10 +1777,16 @@ bool IpcEngine::search_direction(const double* X) {
                        (const int*)row_of_.get(), (const int*)row_col_.get(), (const long long*)contrib_ptr_.get(),
                        (const uint32_t*)contrib_.get(), (const double*)ht_.get(), (const unsigned char*)fixed_.get(),
                        row_val_.get());
-    if (nq_ > 0) assemble_contact();
+    const bool contact = nq_ > 0;
+    if (contact) {
+        assemble_contact();
+        list_blocks(X);
+    }
     SBS_HIP(hipGetLastError());
-    const double gm = max_abs(g_.get(), 3 * (size_t)nv_);
+    const double gm = max_abs(g_.get(), 3 * (size_t)nv_);  // waits: the block count has arrived too
     if (!std::isfinite(gm)) return false;
+    blk_verts_ = contact ? host_blk_[0] : 0;
+    if (blk_verts_ > 0) invert_blocks();
     stats_.linear_iterations += solve();
     return true;
 }
@@ -1458,6 +1797,8 @@ bool IpcEngine::step(IpcData& data, const IpcParams& p) {
     const double h = p.dt;
     const int n3 = 3 * nv_;
     const unsigned vb = nblk(n3);
+    ordered_ = false;
+    pcg_solve_ = 0;
     stats_.newton_iterations = 0;
     stats_.line_search_halvings = 0;
     stats_.linear_iterations = 0;

@@ -97,6 +97,8 @@ private:
     void build_rows(const std::vector<uint32_t>& tet);
     int solve();
     void assemble_contact();
+    void list_blocks(const double* X);
+    void invert_blocks();
     double reduce_sum(const double* parts, int n);
     double max_abs(const double* v, size_t n);
     double body_step(const double* X, const double* p);
@@ -146,7 +148,17 @@ private:
     DevBuf<double> pcg_parts_;              // PCG block partials of r.z and r.r
     DevBuf<double> prod_parts_;             // PCG block partials of p.q
     int* host_ctl_ = nullptr;               // its pinned copy
-    int pcg_last_ = 0;                      // iterations of the previous solve (when to check first)
+    // the preconditioner's blocks of contact vertices (see ipc_block_invert_kernel)
+    double inv_cell_ = 1.0;                 // 1 / Morton cell
+    bool ordered_ = false;                  // order_ holds this step's vertex order
+    DevBuf<unsigned long long> vkey_, vkey_s_;
+    DevBuf<int> vid_, order_, blk_flag_, blk_pos_, blk_list_, blk_slot_, blk_count_;
+    DevBuf<double> blk_inv_;                // 96 x 96 per block
+    int blk_verts_ = 0;                     // vertices in blocks of this solve
+    int* host_blk_ = nullptr;               // their number (pinned)
+    static constexpr size_t kPcgSeen = 64;
+    std::vector<int> pcg_seen_;             // iterations of the last step's solves, in order (when to check first)
+    size_t pcg_solve_ = 0;                  // solves of this step so far
 };
 
 }  // namespace sbs

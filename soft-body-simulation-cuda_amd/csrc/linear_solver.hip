@@ -14,7 +14,7 @@ namespace sbs {
 namespace {
 
 constexpr int kTpbL = 256;
-constexpr int kCheck = 16;  // iterations launched between host reads of the control word
+constexpr int kCheck = 16;  // fewest iterations launched between host reads of the control word
 
 struct LinCtl {
     double rho[2];   // r.z of iteration k, by parity of k
@@ -42,20 +42,30 @@ __device__ __forceinline__ void block_sum_to(double v, double* parts) {
     }
 }
 
-// Sum of nb partials in index order: every block of a launch forms the same
-// value (wave 0 strides the partials, then a fixed-order wave reduction).
-__device__ __forceinline__ double total_of(const double* parts, int nb) {
-    __shared__ double tot;
-    if (threadIdx.x < 64) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < nb; i += 64) s += parts[i];
-        s = wave_sum(s);
-        if (threadIdx.x == 0) tot = s;
+// Sums of NQ arrays of nb partials: every block of a launch forms the same
+// values (thread t adds partials t, t + kTpbL, ..., then the wavefronts'
+// totals in index order).  The loads can be issued ahead of the sums.
+template <int NQ> __device__ __forceinline__ void load_partials(const double* const (&parts)[NQ], int nb, double (&s)[NQ]) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) s[q] = 0.0;
+    for (int i = threadIdx.x; i < nb; i += kTpbL)
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) s[q] += parts[q][i];
+}
+template <int NQ> __device__ __forceinline__ void totals_of(double (&s)[NQ]) {
+    __shared__ double red[NQ][kTpbL / 64];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const double w = wave_total(s[q]);
+        if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = w;
     }
     __syncthreads();
-    const double t = tot;
-    __syncthreads();
-    return t;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        s[q] = 0.0;
+#pragma unroll
+        for (int w = 0; w < kTpbL / 64; ++w) s[q] += red[q][w];
+    }
 }
 
 __global__ void ctl_reset_kernel(LinCtl* ctl, long long* nruns) {
@@ -128,10 +138,29 @@ __global__ void inv_diag_kernel(int n, const int* rowptr, const int* colidx, con
     dinv[r] = (T)1 / d;
 }
 
-template <class T> __device__ __forceinline__ T csr_row(const int* rowptr, const int* colidx, const T* val, const T* v, int r) {
-    T acc = 0;
-    for (int e = rowptr[r]; e < rowptr[r + 1]; ++e) acc += val[e] * v[colidx[e]];
-    return acc;
+// Rows are shared by kLanes lanes: lane l of a row takes its entries l,
+// l + kLanes, ... (consecutive lanes read consecutive entries), and the lanes'
+// sums are added as a tree.  A block holds kTpbL / kLanes rows.
+template <int kLanes, class T> __device__ __forceinline__ T lane_sum(T v) {
+#pragma unroll
+    for (int o = 1; o < kLanes; o <<= 1) v += __shfl_xor(v, o);
+    return v;
+}
+constexpr int kRowBatch = 4;  // entries of a lane whose loads are in flight together
+template <class T> struct RowPart {
+    int c[kRowBatch];
+    T m[kRowBatch];  // 0 past the row's end
+};
+template <int kLanes, class T>
+__device__ __forceinline__ void load_part(const int* __restrict__ colidx, const T* __restrict__ val, int e, int e1,
+                                          RowPart<T>& p) {
+#pragma unroll
+    for (int j = 0; j < kRowBatch; ++j) {
+        const int k = e + j * kLanes, kc = k < e1 ? k : e1 - 1;
+        p.c[j] = colidx[kc];
+        const T m = val[kc];
+        p.m[j] = k < e1 ? m : (T)0;
+    }
 }
 
 // x0 = guess (r = b - A x0) or 0 (r = b); z = D^-1 r; partials of r.r, r.z
@@ -143,7 +172,11 @@ __global__ void pcg_start_kernel(int n, const T* b, const T* guess, T* x, T* r, 
     double rr = 0.0, rz = 0.0;
     if (i < n) {
         T ri = b[i];
-        if (guess) ri -= csr_row(rowptr, colidx, val, guess, i);
+        if (guess) {
+            T acc = 0;
+            for (int e = rowptr[i]; e < rowptr[i + 1]; ++e) acc += val[e] * guess[colidx[e]];
+            ri -= acc;
+        }
         const T zi = dinv[i] * ri;
         x[i] = guess ? guess[i] : (T)0;
         r[i] = ri;
@@ -155,37 +188,103 @@ __global__ void pcg_start_kernel(int n, const T* b, const T* guess, T* x, T* r, 
     block_sum_to(rz, prz);
 }
 
-// Iteration k, part 1: the stop tests at the loop top (||r|| < tol, then
-// |r.z| < 1e-15), beta = rho_k / rho_{k-1}, p = z + beta p (p = z at k = 0).
+// The stop tests of iteration k (||r|| < tol, then |r.z| < 1e-15) and beta =
+// rho_k / rho_{k-1}, formed by every block from the totals rr = r.r and rho =
+// r.z of the update launch; block 0 records them.  Returns true when the solve
+// stops here.
+__device__ __forceinline__ bool pcg_direction(int k, double tol, double rr, double rho, LinCtl* ctl, double& beta) {
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    if (sqrt(rr) < tol || fabs(rho) < 1e-15) {
+        if (lead) {
+            ctl->done = 1;
+            ctl->iters = k;
+        }
+        return true;
+    }
+    beta = k == 0 ? 0.0 : rho / ctl->rho[(k - 1) & 1];
+    if (lead) ctl->rho[k & 1] = rho;
+    return false;
+}
+
+// Iteration k, part 1 when there is no room for a second direction: p = z +
+// beta p in place (p = z at k = 0).
 template <class T>
 __global__ void pcg_dir_kernel(int n, int k, int nb, double tol, const double* prr, const double* prz, const T* z,
                                T* p, LinCtl* ctl) {
     if (block_done(ctl)) return;
-    const double rr = total_of(prr, nb), rho = total_of(prz, nb);
-    if (sqrt(rr) < tol || fabs(rho) < 1e-15) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            ctl->done = 1;
-            ctl->iters = k;
-        }
-        return;
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) ctl->rho[k & 1] = rho;
-    const T beta = k == 0 ? (T)0 : (T)(rho / ctl->rho[(k - 1) & 1]);
+    double s[2];
+    load_partials<2>({prr, prz}, nb, s);
+    totals_of<2>(s);
+    double beta;
+    if (pcg_direction(k, tol, s[0], s[1], ctl, beta)) return;
     const int i = blockIdx.x * kTpbL + threadIdx.x;
-    if (i < n) p[i] = k == 0 ? z[i] : z[i] + beta * p[i];
+    if (i < n) p[i] = k == 0 ? z[i] : z[i] + (T)beta * p[i];
 }
 
-// Iteration k, part 2: q = A p and the partials of p.q.
-template <class T>
-__global__ void pcg_spmv_kernel(int n, const int* rowptr, const int* colidx, const T* val, const T* p, T* q,
-                                double* ppq, const LinCtl* ctl) {
+// Iteration k, part 2: q = A p and the partials of p.q.  With kForm the
+// direction is formed here too: p_k = z + beta p_{k-1} by one expression
+// wherever it is read (the row's own entry, stored to pnew, and the columns),
+// so an iteration is two launches.  A launch is a chain of memory round trips
+// (row bounds, entries, the columns' values; the stop word; the partials), so
+// all but the last of them are requested before the stop word is looked at.
+// With one thread per row the entries of neighbouring threads lie a row
+// apart: 16,416 rows of 41 entries in FP64 took 17.9 us (and 4.4 us for the
+// direction), this form 6.0 us.
+template <int kLanes, bool kForm, class T>
+__global__ void __launch_bounds__(kTpbL) pcg_spmv_kernel(int n, int k, int nb, double tol, const double* prr,
+                                                         const double* prz, const int* __restrict__ rowptr,
+                                                         const int* __restrict__ colidx, const T* __restrict__ val,
+                                                         const T* __restrict__ z, const T* __restrict__ pold,
+                                                         T* __restrict__ pnew, T* __restrict__ q, double* ppq,
+                                                         LinCtl* ctl) {
+    const bool first = k == 0;
+    const int i = (blockIdx.x * kTpbL + threadIdx.x) / kLanes, l = threadIdx.x % kLanes;
+    const bool live = i < n;
+    const int e0 = live ? rowptr[i] : 0, e1 = live ? rowptr[i + 1] : 0;
+    double tot[2];
+    if (kForm) load_partials<2>({prr, prz}, nb, tot);
+    T zi = 0, pi = 0;
+    if (live && l == 0) {
+        if (kForm) zi = z[i];
+        if (!kForm || !first) pi = pold[i];
+    }
+    RowPart<T> part;
+    T zc[kRowBatch], pc[kRowBatch];
+    auto fetch = [&](int e) {
+        load_part<kLanes>(colidx, val, e, e1, part);
+#pragma unroll
+        for (int j = 0; j < kRowBatch; ++j) {
+            if (kForm) zc[j] = z[part.c[j]];
+            pc[j] = kForm && first ? (T)0 : pold[part.c[j]];
+        }
+    };
+    const bool any = e0 + l < e1;
+    if (any) fetch(e0 + l);
     if (block_done(ctl)) return;
-    const int i = blockIdx.x * kTpbL + threadIdx.x;
+    double bt = 0.0;
+    if (kForm) {
+        totals_of<2>(tot);
+        if (pcg_direction(k, tol, tot[0], tot[1], ctl, bt)) return;
+    }
+    const T beta = (T)bt;
+    auto dir = [&](T zv, T pv) -> T { return !kForm ? pv : first ? zv : zv + beta * pv; };
+    T acc = 0;
+    if (any)
+        for (int e = e0 + l;;) {
+#pragma unroll
+            for (int j = 0; j < kRowBatch; ++j)
+                if (e + j * kLanes < e1) acc += part.m[j] * dir(zc[j], pc[j]);
+            e += kLanes * kRowBatch;
+            if (e >= e1) break;
+            fetch(e);
+        }
+    acc = lane_sum<kLanes>(acc);
     double pq = 0.0;
-    if (i < n) {
-        const T qi = csr_row(rowptr, colidx, val, p, i);
-        q[i] = qi;
-        pq = (double)p[i] * (double)qi;
+    if (live && l == 0) {
+        const T pv = dir(zi, pi);
+        if (kForm) pnew[i] = pv;
+        q[i] = acc;
+        pq = (double)pv * (double)acc;
     }
     block_sum_to(pq, ppq);
 }
@@ -193,17 +292,27 @@ __global__ void pcg_spmv_kernel(int n, const int* rowptr, const int* colidx, con
 // Iteration k, part 3: alpha = rho / p.q, x += alpha p, r -= alpha q, then
 // z = D^-1 r and the partials of iteration k+1 (other parity).
 template <class T>
-__global__ void pcg_update_kernel(int n, int k, int nb, const double* ppq, const T* p, const T* q, T* x, T* r, T* z,
+__global__ void pcg_update_kernel(int n, int k, int nb_prod, const double* ppq, const T* p, const T* q, T* x, T* r, T* z,
                                   const T* dinv, double* prr_next, double* prz_next, LinCtl* ctl) {
-    if (block_done(ctl)) return;
-    const double pq = total_of(ppq, nb);
-    const T alpha = (T)(ctl->rho[k & 1] / pq);
+    double tot[1];
+    load_partials<1>({ppq}, nb_prod, tot);
     const int i = blockIdx.x * kTpbL + threadIdx.x;
+    T xi = 0, pi = 0, ri = 0, qi = 0, di = 0;
+    if (i < n) {
+        xi = x[i];
+        pi = p[i];
+        ri = r[i];
+        qi = q[i];
+        di = dinv[i];
+    }
+    if (block_done(ctl)) return;
+    totals_of<1>(tot);
+    const T alpha = (T)(ctl->rho[k & 1] / tot[0]);
     double rr = 0.0, rz = 0.0;
     if (i < n) {
-        x[i] += alpha * p[i];
-        const T ri = r[i] - alpha * q[i];
-        const T zi = dinv[i] * ri;
+        x[i] = xi + alpha * pi;
+        ri -= alpha * qi;
+        const T zi = di * ri;
         r[i] = ri;
         z[i] = zi;
         rr = (double)ri * (double)ri;
@@ -212,6 +321,16 @@ __global__ void pcg_update_kernel(int n, int k, int nb, const double* ppq, const
     block_sum_to(rr, prr_next);
     block_sum_to(rz, prz_next);
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl->iters = k + 1;
+}
+
+constexpr int kMaxLanes = 32;  // lanes per row of the product at most
+// Lanes per row: a lane keeps 4 to 8 entries of a mean row (an elasticity row
+// of 41 entries, 152 iterations of 16,416 rows: 4 lanes 2,175 us a solve, 8
+// 2,185, 16 2,223; with one thread per row 4,700).
+int lanes_for(int n, long long nnz) {
+    int l = 1;
+    while (l < kMaxLanes && 8ll * l * n <= nnz) l *= 2;
+    return l;
 }
 
 // Workspace layout (each piece 256-byte aligned).
@@ -226,6 +345,11 @@ template <class T> struct Layout {
     void* tmp;
     size_t tmp_bytes;
     size_t total;
+    // The sort's arrays (keys to vals_sorted, contiguous) are free once the
+    // rows stand: the second direction and the product's partials live there
+    // where they fit, so the workspace is no larger for them.
+    T* p2 = nullptr;
+    double* ppq_rows = nullptr;
 
     Layout(char* base, int n, long long nz, size_t tmp_b) {
         size_t off = 0;
@@ -256,6 +380,12 @@ template <class T> struct Layout {
         tmp = take(tmp_b);
         tmp_bytes = tmp_b;
         total = off;
+        const size_t second = align256((size_t)n * sizeof(T));
+        const size_t partials = align256((size_t)nblk((size_t)n * kMaxLanes) * sizeof(double));
+        if (base && second + partials <= (size_t)((char*)uvals - base)) {
+            p2 = (T*)base;
+            ppq_rows = (double*)(base + second);
+        }
     }
 };
 
@@ -367,19 +497,47 @@ int CooPcgSolver<T>::solve_in(int n, const T* b, T* x, const T* A, long long nz,
     SBS_HIP(hipStreamSynchronize(stream));
     SBS_REQUIRE(!hc.bad_index, "LinearSolver::Solve: a row or column index is outside [0, N)");
     nnz_ = hc.nnz;
+    const int lanes = L.p2 ? lanes_for(n, hc.nnz) : 1;
+    const int nbp = (int)nblk((size_t)n * lanes);
+    double* ppq = L.p2 ? L.ppq_rows : L.ppq;
+    const bool form = L.p2 != nullptr;
+    T* dir[2] = {L.p, form ? L.p2 : L.p};
+    // product of iteration k: reads the direction of k - 1 (or, without room
+    // for two, the direction that pcg_dir_kernel has just formed)
+    auto product = [&](int k, const double* prr, const double* prz) {
+        auto launch = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(nbp), dim3(kTpbL), 0, stream, n, k, nb, tol_, prr, prz,
+                               (const int*)L.rowptr, (const int*)L.colidx, (const T*)L.uvals, (const T*)L.z,
+                               (const T*)dir[(k + 1) & 1], dir[k & 1], L.q, ppq, L.ctl);
+        };
+        if (!form) {
+            hipLaunchKernelGGL(pcg_dir_kernel<T>, dim3(nb), dim3(kTpbL), 0, stream, n, k, nb, tol_, prr, prz,
+                               (const T*)L.z, L.p, L.ctl);
+            launch(pcg_spmv_kernel<1, false, T>);
+            return;
+        }
+        switch (lanes) {
+            case 1: launch(pcg_spmv_kernel<1, true, T>); break;
+            case 2: launch(pcg_spmv_kernel<2, true, T>); break;
+            case 4: launch(pcg_spmv_kernel<4, true, T>); break;
+            case 8: launch(pcg_spmv_kernel<8, true, T>); break;
+            case 16: launch(pcg_spmv_kernel<16, true, T>); break;
+            default: launch(pcg_spmv_kernel<32, true, T>); break;
+        }
+    };
     int k = 0;
     while (k < max_iter_) {
-        const int chunk = std::min(kCheck, max_iter_ - k);
+        // a look at the control word leaves the GPU idle for about 30 us, an
+        // iteration launched after the solve has stopped costs 5: the first
+        // look after 9/10 of this solver's previous count, then every quarter
+        // of what has been launched
+        const int want = k == 0 ? std::max(kCheck, last_iters_ * 9 / 10) : std::max(kCheck, k / 4);
+        const int chunk = std::min(want, max_iter_ - k);
         for (int j = 0; j < chunk; ++j, ++k) {
             const int par = k & 1;
-            hipLaunchKernelGGL(pcg_dir_kernel<T>, dim3(nb), dim3(kTpbL), 0, stream, n, k, nb, tol_,
-                               (const double*)(L.prr + par * nb), (const double*)(L.prz + par * nb), (const T*)L.z,
-                               L.p, L.ctl);
-            hipLaunchKernelGGL(pcg_spmv_kernel<T>, dim3(nb), dim3(kTpbL), 0, stream, n, (const int*)L.rowptr,
-                               (const int*)L.colidx, (const T*)L.uvals, (const T*)L.p, L.q, L.ppq,
-                               (const LinCtl*)L.ctl);
-            hipLaunchKernelGGL(pcg_update_kernel<T>, dim3(nb), dim3(kTpbL), 0, stream, n, k, nb,
-                               (const double*)L.ppq, (const T*)L.p, (const T*)L.q, x, L.r, L.z, (const T*)L.dinv,
+            product(k, L.prr + par * nb, L.prz + par * nb);
+            hipLaunchKernelGGL(pcg_update_kernel<T>, dim3(nb), dim3(kTpbL), 0, stream, n, k, nbp, (const double*)ppq,
+                               (const T*)dir[k & 1], (const T*)L.q, x, L.r, L.z, (const T*)L.dinv,
                                L.prr + (1 - par) * nb, L.prz + (1 - par) * nb, L.ctl);
         }
         SBS_HIP(hipGetLastError());
@@ -387,6 +545,7 @@ int CooPcgSolver<T>::solve_in(int n, const T* b, T* x, const T* A, long long nz,
         SBS_HIP(hipStreamSynchronize(stream));
         if (hc.done) break;
     }
+    last_iters_ = hc.iters;
     return hc.iters;
 }
 

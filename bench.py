@@ -253,8 +253,8 @@ def batched_scene(nbodies: int = 1024, seed: int = 0):
 
 def batched_measure(steps: int, warmup: int, sample: int, fp64_check: bool = True, polar: bool = False):
     """The 1024 uneven bodies on the batched solver (every body its own
-    Jacobi-PCG + Chebyshev, one workgroup per body, one launch per size class,
-    workgroup sizes from the autotuner at the first update), against one
+    Jacobi-PCG + Chebyshev, one workgroup per body and solve,
+    the workgroup size from the autotuner at the first update), against one
     PdSolver per body (the plain FP32 per-body form) on a sample of the bodies,
     extrapolated to all of them; accuracy against an FP64 batched run of the
     same steps (FP64 batched is parity-tested against the FP64 oracle per body)."""

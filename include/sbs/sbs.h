@@ -60,10 +60,9 @@ extern "C" {
 /* Batched bodies: every connected body of the scene (the bodies the
  * reference's DataLoader concatenates, dataLoader.cu:292-378) is solved on its
  * own -- its own Jacobi-PCG (alpha, beta and stop test per body,
- * pcgJacobi.cu:89-173) + Chebyshev -- with one workgroup per body running the
- * whole step in one persistent launch per body-size class; the classes'
- * workgroup sizes come from an autotuner run at the first batched update
- * (SbsSolverParams.batch_autotune).  Results equal one PdSolver per body with
+ * pcgJacobi.cu:89-173) + Chebyshev -- with one workgroup per body running each
+ * global solve; the workgroup size comes from an autotuner run at the first
+ * batched update (SbsSolverParams.batch_autotune).  Results equal one PdSolver per body with
  * SBS_SOLVER_PCG and pcg_chebyshev.  moreDBC is not taken. */
 #define SBS_SOLVER_BATCHED_PCG 5
 
@@ -121,9 +120,9 @@ typedef struct SbsSolverParams {
                              caps; no collision handling, perf or kernel timing).  On MI355X
                              a replay costs what the eager launches cost (64^3 cube: 248 vs
                              256 steps/s; 8^3: 660 vs 654), so 0 is the usual choice */
-    int batch_autotune;   /* SBS_SOLVER_BATCHED_PCG: 1 times the workgroup sizes of each
-                             body-size class at the first batched update (state unchanged);
-                             0 keeps one thread per 16 tets of the class's largest body */
+    int batch_autotune;   /* SBS_SOLVER_BATCHED_PCG: 1 times a step with each workgroup
+                             size at the first batched update (state unchanged); 0 keeps
+                             half a thread per vertex of the largest body */
     int polar_rotation;   /* FP32 local step: 0 takes each element's rotation from the TR1690
                              SVD as the reference does (computeLocal, pdUtil.cu:112-125);
                              1 from Newton's polar iteration R <- (R + R^-T)/2, 5 steps,
@@ -222,7 +221,8 @@ int sbs_pd_export_system(SbsPd* pd, void* c, void* diagA, void* diagL, void* V0,
 typedef struct SbsCollision SbsCollision;
 /* Batched solver of the handle (after an update with SBS_SOLVER_BATCHED_PCG):
  * bodies and size classes; per class info = {min tets, max tets, bodies,
- * threads per workgroup} and the tuner's (threads, ms per step) pairs; per
+ * threads per workgroup} and the tuner's (threads, ms per step) pairs (the
+ * launches, and so the tuner's choice, are shared by the classes); per
  * body 6 ints {vertices, tets, PCG iterations, solves, most iterations of one
  * solve, solves stopped by pcg_max_iter} accumulated over the updates. */
 int sbs_pd_batch_info(SbsPd* pd, int* num_bodies, int* num_classes);

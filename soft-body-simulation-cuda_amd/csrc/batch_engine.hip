@@ -1,46 +1,53 @@
-// Batched PD step: one workgroup per body runs the whole step; see
-// batch_engine.hpp.  Per body and outer iteration i (pdSolver.cu:164-205 with
+// Batched PD step: per body and outer iteration i (pdSolver.cu:164-205 with
 // the Jacobi-PCG global solve, as the PCG global step of pd_engine):
-//   computeLocal (pdUtil.cu:97-145) per tet, its 4 corner forces into `force`;
-//   b = c sn_old + the forces of the vertex's corners, pinned rows
-//   overwritten with DBCX 1e6/h^2 (pdUtil.cu:147-178);
+//   computeLocal (pdUtil.cu:97-145) over the tet chunks of all bodies (one
+//   workgroup per chunk, see local_chunk);
+//   b = c sn_old + the vertex's partial forces, pinned rows overwritten with
+//   DBCX 1e6/h^2 (pdUtil.cu:147-178);
 //   Jacobi-PCG warm-started from sn, per component stopping when
 //   ||D^-1 r_k|| <= max(tol ||D^-1 r_0||, floor ||D^-1 b||);
-//   the Chebyshev recurrence (pdSolver.cu:196-198, pdUtil.cu:216-226).
-// Reductions are block reductions in a fixed order (DPP inside a wavefront,
-// then the wavefront totals in index order), so a body's result does not
-// depend on the other bodies or on scheduling.
+//   the Chebyshev recurrence (pdSolver.cu:196-198, pdUtil.cu:216-226);
+// the last three by one workgroup per body in one launch.  Reductions are
+// block reductions in a fixed order, so a body's result does not depend on the
+// other bodies or on scheduling.  See batch_engine.hpp.
 #include "batch_engine.hpp"
 
 #include <algorithm>
 #include <numeric>
+#include <type_traits>
 
-#include "svd3.hpp"
+#include "halo_tiles.hpp"
+#include "local_chunk.hpp"
 
 namespace sbs {
 namespace {
 
 constexpr int kMaxWaves = 16;  // 1024-thread workgroups at most
+constexpr int kTpbB = 256;     // threads of the per-vertex kernels
+constexpr int kMaxNarrow = 65535 / 3 - 1;  // vertices of a body whose columns fit 16 bits
+constexpr int kFixedPlaces = 6;  // from this many rows per thread on, workgroups have 1,024 threads
+constexpr int kBufferFlags = 0x00020000;  // raw buffer descriptor: 32-bit data format, no swizzle
+constexpr int kRegWidth = 16;  // widest matrix row kept in registers
 
 template <class T> struct BatchArgs {
-    const int* body_list;
-    const int* vptr;
-    const int* tptr;
-    const int* eptr;
-    const int* ew;
-    const uint32_t* perm;
-    const uint4* tets;
-    const T* dminv;
-    const T* w;
-    const int* inc_ptr;
-    const uint32_t* inc;
-    const uint32_t* ecol;
+    const int* vptr;      // first vertex of each body
+    const int* eptr;      // first matrix entry
+    const int* ew;        // entries per row
+    const int* orig;      // the caller's number of the body
+    const int* vbody;     // body of each vertex
+    const uint32_t* perm; // vertex -> caller's vertex
+    const uint16_t* ecol; // 3 x the column's place in the body
+    const uint32_t* ecol_wide;  // the same for bodies past the 16 bits
     const T* eval;
     const T* diagA;
+    const T* dinv;
     const T* c0;
     const T* mass;
     const T* dbc;
-    const T* origin;  // 3 per body: the body's local origin
+    const T* origin;      // 3 per body: the body's local origin
+    int nv;
+    const int* vent_ptr;  // partial forces of vertex i: [vent_ptr[i], vent_ptr[i + 1])
+    const T* partial;
     T* X;
     T* V;
     T* XT;
@@ -48,19 +55,15 @@ template <class T> struct BatchArgs {
     T* sn;
     T* sn_old;
     T* prev;
-    T* x;
+    T* x;                 // vectors of the bodies whose rows do not fit the registers
     T* r;
     T* p;
     T* q;
-    T* force;
     int* stats;
-    int iters;
     int max_iter;
     int write_x;
-    int polar;  // rotation by Newton's polar iteration (FP32)
     T dt;
     T gravity;
-    T rho;
     T wdbc;
     T tol2;
     T floor2;
@@ -73,302 +76,421 @@ template <class T> __device__ __forceinline__ T cheb(T x, T s, T prev, T omega) 
     return fma(damped - prev, omega, prev);
 }
 
-// Block sum of NQ doubles returned to every thread: DPP wavefront totals,
-// then the wavefront totals added in index order.  `buf` alternates between
-// two LDS buffers from one reduction to the next, so one barrier suffices.
-template <int NQ> __device__ __forceinline__ void block_sum(double (&v)[NQ], double* buf) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+// Block sums of the three components of NG quantities: component c of
+// quantity g ends in every lane of row c of each wavefront (t[g]).  A
+// wavefront's totals go to LDS by rows (wave_rows4), one read per quantity
+// gives a row all wavefronts' totals of its component, and one 16-lane sum
+// finishes it; with a full wavefront sum and one LDS read per wavefront and
+// value the reductions were most of a small body's iteration.  `live`: the
+// wavefront has rows (uniform; the others' values are 0 and only wait).
+// `buf` alternates between two LDS buffers from one reduction to the next, so
+// one barrier suffices.
+template <int NG> __device__ __forceinline__ void block_rows(const double (&v)[NG][3], double (&t)[NG], double* buf, bool live) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6, row = lane >> 4, s = lane & 15;
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) v[k] = wave_total(v[k]);
-    if (lane == 0)
-#pragma unroll
-        for (int k = 0; k < NQ; ++k) buf[wv * NQ + k] = v[k];
+    for (int g = 0; g < NG; ++g) {
+        const double w = live ? wave_rows4(v[g][0], v[g][1], v[g][2], 0.0) : 0.0;
+        if (s == 0) buf[(4 * g + row) * kMaxWaves + wv] = w;
+    }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) {
-        double s = 0.0;
-        for (int j = 0; j < nw; ++j) s += buf[j * NQ + k];
-        v[k] = s;
+    for (int g = 0; g < NG; ++g) t[g] = row16_total(s < nw ? buf[(4 * g + row) * kMaxWaves + s] : 0.0);
+}
+// A value of lanes 0, 16 and 32 (components 0, 1, 2) as three uniform values.
+__device__ __forceinline__ void from_rows(float v, float (&o)[3]) {
+    o[0] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
+    o[1] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 16));
+    o[2] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
+}
+__device__ __forceinline__ void from_rows(double v, double (&o)[3]) {
+    o[0] = readlane_f64<0>(v);
+    o[1] = readlane_f64<16>(v);
+    o[2] = readlane_f64<32>(v);
+}
+
+// Prologue (pdSolver.cu:154-162): s_n = x + h v +
+// f_ext / c, sn_old, prev.  Every vector of a body is held relative to its
+// origin o (the step is translation invariant: L o = 0, so A (y + o) = b
+// becomes A y = b - c o), so FP32 rounds offsets of the body's size, not of
+// its distance from the world origin.
+template <class T> __global__ void __launch_bounds__(kTpbB) batch_begin_kernel(BatchArgs<T> a) {
+    const int i = (int)(blockIdx.x * kTpbB + threadIdx.x);
+    if (i >= a.nv) return;
+    const uint32_t g = a.perm[i];
+    const T* o = a.origin + 3 * (size_t)a.vbody[i];
+    const T fy = -a.gravity * a.mass[i], inv = (T)1 / a.c0[i], dt = a.dt;
+    const T s0 = (a.X[3 * (size_t)g] - o[0]) + dt * a.V[3 * (size_t)g];
+    const T s1 = (a.X[3 * (size_t)g + 1] - o[1]) + dt * a.V[3 * (size_t)g + 1] + inv * fy;
+    const T s2 = (a.X[3 * (size_t)g + 2] - o[2]) + dt * a.V[3 * (size_t)g + 2];
+    for (T* out : {a.sn, a.sn_old, a.prev}) {
+        out[3 * (size_t)i] = s0;
+        out[3 * (size_t)i + 1] = s1;
+        out[3 * (size_t)i + 2] = s2;
     }
 }
 
-// Entries j0 .. j0 + NB - 1 of row il of a body's ELL matrix
-// (positions past the row's width repeat its last entry; the caller skips
-// them), requested together so their latencies overlap.
-template <class T> constexpr int kRowBatch = sizeof(T) == 4 ? 8 : 4;  // FP64: within the 128 registers
-template <class T, int NB = kRowBatch<T>>
-__device__ __forceinline__ void row_entries(const BatchArgs<T>& a, size_t ebase, int nrow, int il, int width, int j0,
-                                            uint32_t (&uu)[NB], T (&vv)[NB]) {
+// updateVelPos (pdUtil.cu:180-193) and X <- XTilde (pdSolver.cu:227).
+template <class T> __global__ void __launch_bounds__(kTpbB) batch_end_kernel(BatchArgs<T> a) {
+    const int i = (int)(blockIdx.x * kTpbB + threadIdx.x);
+    if (i >= a.nv) return;
+    const T dt_inv = (T)1 / a.dt;
+    const uint32_t g = a.perm[i];
+    const T* o = a.origin + 3 * (size_t)a.vbody[i];
 #pragma unroll
-    for (int jj = 0; jj < NB; ++jj) {
-        const int j = j0 + jj < width ? j0 + jj : width - 1;
-        const size_t e = ebase + (size_t)j * nrow + il;
-        uu[jj] = a.ecol[e];
-        vv[jj] = a.eval[e];
+    for (int k = 0; k < 3; ++k) {
+        const T n = a.sn[3 * (size_t)i + k];
+        const size_t j = 3 * (size_t)g + k;
+        a.V[j] = (n - (a.XT[j] - o[k])) * dt_inv;
+        const T xa = n + o[k];
+        a.XT[j] = xa;
+        if (a.write_x) a.X[j] = xa;
     }
 }
 
-// kLdsP: the PCG search direction of the body lives in LDS (3 values per
-// vertex of the class's largest body), so the product's neighbour reads are
-// LDS reads instead of L2 round trips; the values are the same.
-template <class T, bool kLdsP>
-__global__ void __launch_bounds__(1024) batch_step_kernel(BatchArgs<T> a, int first) {
-    __shared__ double red[2][kMaxWaves * 9];
-    extern __shared__ __align__(16) unsigned char dyn_lds[];
-    int rb = 0;
-    const int b = a.body_list[first + blockIdx.x];
-    const int v0 = a.vptr[b], v1 = a.vptr[b + 1], t0 = a.tptr[b], t1 = a.tptr[b + 1];
-    T* const lp = reinterpret_cast<T*>(dyn_lds);
-    const size_t pbase = 3 * (size_t)v0;
-    // entry j (3 per vertex, global numbering) of the search direction
-    auto P = [&](size_t j) -> T& { return kLdsP ? lp[j - pbase] : a.p[j]; };
-    const int nrow = v1 - v0, width = a.ew[b];
-    const size_t ebase = (size_t)a.eptr[b];
-    const int B = blockDim.x, tid = threadIdx.x;
-    const T dt = a.dt;
-    // Every vector of the body is held relative to its origin o (the step is
-    // translation invariant: L o = 0, so A (y + o) = b becomes A y = b - c o),
-    // so FP32 rounds offsets of the body's size, not of its distance from the
-    // world origin.
-    const T o[3] = {a.origin[3 * b], a.origin[3 * b + 1], a.origin[3 * b + 2]};
+template <class T>
+__global__ void __launch_bounds__(kChunkTets) batch_local_kernel(
+    int nt, const uint2* __restrict__ lidx, const int* __restrict__ chunk_vptr,
+    const uint32_t* __restrict__ chunk_verts, const uint32_t* __restrict__ entry_pos,
+    const uint16_t* __restrict__ inc_codes, const uint16_t* __restrict__ inc_end, const T* __restrict__ dminv,
+    const T* __restrict__ w, const T* __restrict__ q, T* __restrict__ partial, int flags) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    local_chunk<T>(xcd_block(blockIdx.x, gridDim.x), nt, lidx, chunk_vptr, chunk_verts, entry_pos, inc_codes, inc_end,
+                   dminv, w, partial, flags, smem_raw, [&](int, uint32_t g, T& x, T& y, T& z) {
+        x = q[3 * (size_t)g];
+        y = q[3 * (size_t)g + 1];
+        z = q[3 * (size_t)g + 2];
+    });
+}
 
-    // prologue (pdSolver.cu:154-162): s_n = x + h v + f_ext / c, sn_old, prev
-    for (int i = v0 + tid; i < v1; i += B) {
-        const uint32_t g = a.perm[i];
+template <class T> constexpr int kPairBatch = sizeof(T) == 4 ? 4 : 2;  // pairs of matrix entries in flight per row
+
+// Right-hand side, PCG solve and Chebyshev step of one body (a workgroup).
+// The body's rows are dealt to the threads, row
+// k blockDim + tid to the thread's place k < K, and r and q of a row stay in
+// registers for the whole solve (the diagonal and x too where they are few:
+// !kXg); with kRegs the row's matrix entries as well, read once per solve.
+// K = 0 keeps the vectors in memory and takes any number of rows.  With kLds
+// the search direction lives in LDS (first the iterate, for A x), so the
+// product's neighbour reads are LDS reads.  Matrix entries are stored in
+// pairs (two values, two 16-bit columns: a load of 8 and one of 4 bytes for
+// FP32), since a load costs its lanes' addresses whatever its width.  What
+// bounds it: instructions for small bodies (an iteration of a 280-row body
+// took 2.6 us, 700 instructions a wavefront of which the reductions were 280),
+// LDS reads and the matrix from L2 for the largest.
+template <class T, int K, bool kRegs, bool kLds, bool kXg, bool kWide = false>
+__device__ __forceinline__ void batch_solve_body(const BatchArgs<T>& a, int b, int v0, int n, int width, T omega, T* lp,
+                                                 double (*red)[12 * kMaxWaves]) {
+    static_assert(K > 0 || (!kRegs && kXg), "vectors in memory: no matrix in registers");
+    static_assert(!kWide || (K == 0 && !kLds), "wide bodies keep their vectors in memory");
+    constexpr int KR = K > 0 ? K : 1;
+    constexpr bool kDiag = K > 0 && K * sizeof(T) <= 16;  // the diagonal and its inverse in registers
+    typedef T V2 __attribute__((ext_vector_type(2)));
+    const size_t ebase = (size_t)__builtin_amdgcn_readfirstlane(a.eptr[b]);
+    // rows k B + tid: with the k B part in a uniform base and the thread's part a
+    // 32-bit byte offset, a load needs one address register for all places
+    const int B = K >= kFixedPlaces ? 1024 : blockDim.x;
+    const unsigned tid = threadIdx.x;
+    const int lane = tid & 63, row = lane >> 4, comp = row < 3 ? row : 2;
+    const bool live = (int)(tid & ~63u) < n;  // the wavefront has rows
+    const int places = K > 0 ? K : (n + B - 1) / B;
+    const T o[3] = {a.origin[3 * (size_t)b], a.origin[3 * (size_t)b + 1], a.origin[3 * (size_t)b + 2]};
+    T rr[KR][3], qr[KR][3], xr[kXg ? 1 : KR][3], da[kDiag ? KR : 1], dr[kDiag ? KR : 1];
+    // (with many rows per thread: one row's loads at a time, all rows' would spill)
+    auto fence = [] {
+        if constexpr (K >= kFixedPlaces) __builtin_amdgcn_sched_barrier(0);
+    };
+    const unsigned o1 = tid * (unsigned)sizeof(T), o3 = 3 * o1;
+    auto elem = [](auto* base, unsigned byte, int c) -> auto& {
+        using E = std::remove_pointer_t<decltype(base)>;
+        using Bytes = std::conditional_t<std::is_const_v<E>, const char, char>;
+        return reinterpret_cast<E*>(reinterpret_cast<Bytes*>(base) + byte)[c];
+    };
+    // (readfirstlane where a base is used: hoisted out of the iterations, the
+    // places' addresses would take more registers than their vectors)
+    auto at = [&](int k) -> size_t { return (size_t)__builtin_amdgcn_readfirstlane(v0 + k * B); };
+    auto vec = [&](T (&reg)[KR][3], T* mem, int k, int c) -> T& {
+        if constexpr (K > 0) return reg[k][c];
+        else return elem(mem + 3 * at(k), o3, c);
+    };
+    auto X = [&](int k, int c) -> T& {
+        if constexpr (kXg) return elem(a.x + 3 * at(k), o3, c);
+        else return xr[k][c];
+    };
+    auto diag = [&](int k) -> T {
+        if constexpr (kDiag) return da[k];
+        else return elem(a.diagA + at(k), o1, 0);
+    };
+    auto dinv = [&](int k) -> T {
+        if constexpr (kDiag) return dr[k];
+        else return elem(a.dinv + at(k), o1, 0);
+    };
+    // entry j (3 per row) of the vector whose neighbours are read
+    T* const pm = kLds ? lp : a.p + 3 * (size_t)v0;
+    auto P = [&](int k, int c) -> T& { return (pm + 3 * (size_t)k * B)[3 * tid + c]; };
+    // pair j2 of the row in place k: values and 3 x columns.  Buffer loads: the
+    // body's base in a descriptor, the pair's and place's part a scalar offset,
+    // the thread's one register for all of them (address arithmetic per load
+    // was most of the product's instructions, and spilled).
+    const unsigned entries = (unsigned)width * (unsigned)n;
+    const auto rval = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.eval) + ebase, 0, (int)(entries * sizeof(T)),
+                                                        kBufferFlags);
+    const auto rcol = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.ecol) + ebase, 0, (int)(entries * 2),
+                                                        kBufferFlags);
+    auto pair = [&](int j2, int k, V2& m, unsigned& c0, unsigned& c1) {
+        const unsigned at2 = 2u * ((unsigned)j2 * (unsigned)n + (unsigned)(k * B));
+        if constexpr (kWide) {
+            const size_t e = ebase + at2 + 2 * (size_t)tid;
+            m = *reinterpret_cast<const V2*>(a.eval + e);
+            const uint2 c = *reinterpret_cast<const uint2*>(a.ecol_wide + e);
+            c0 = c.x;
+            c1 = c.y;
+        } else {
+            if constexpr (sizeof(T) == 4)
+                m = __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b64(rval, 2 * o1, at2 * sizeof(T), 0));
+            else
+                m = __builtin_bit_cast(V2, __builtin_amdgcn_raw_buffer_load_b128(rval, 2 * o1, at2 * sizeof(T), 0));
+            const unsigned c = __builtin_amdgcn_raw_buffer_load_b32(rcol, 4 * tid, at2 * 2, 0);
+            c0 = c & 0xffffu;
+            c1 = c >> 16;
+        }
+    };
+    const int pairs = width / 2;  // rows are padded to whole pairs
+    V2 mv[kRegs ? KR : 1][kRegWidth / 2];
+    unsigned mc[kRegs ? KR : 1][kRegWidth / 2];
+    if constexpr (kRegs) {
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+            const bool own = k * B + (int)tid < n;
+#pragma unroll
+            for (int j = 0; j < kRegWidth / 2; ++j) {
+                mv[k][j] = V2{(T)0, (T)0};
+                mc[k][j] = 0;
+                if (j < pairs && own) {
+                    unsigned c0, c1;
+                    pair(j, k, mv[k][j], c0, c1);
+                    mc[k][j] = c0 | (c1 << 16);
+                }
+            }
+        }
+    }
+    // y += the off-diagonal entries of row (place k) times pm
+    auto product = [&](int k, T (&y)[3]) {
+        auto add = [&](const V2& m, unsigned c0, unsigned c1) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) y[c] += m.x * pm[c0 + c];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) y[c] += m.y * pm[c1 + c];
+        };
+        if constexpr (kRegs) {
+#pragma unroll
+            for (int j = 0; j < kRegWidth / 2; ++j)
+                if (j < pairs) add(mv[k][j], mc[k][j] & 0xffffu, mc[k][j] >> 16);
+        } else {
+            // whole batches, then the rest one pair at a time (no clamped loads)
+            auto batch = [&](int j0, auto count) {
+                constexpr int NB = decltype(count)::value;
+                V2 m[NB];
+                unsigned c0[NB], c1[NB];
+#pragma unroll
+                for (int j = 0; j < NB; ++j) pair(j0 + j, k, m[j], c0[j], c1[j]);
+#pragma unroll
+                for (int j = 0; j < NB; ++j) add(m[j], c0[j], c1[j]);
+            };
+            constexpr int NB = kPairBatch<T>;
+            int j0 = 0;
+#pragma unroll 1
+            for (; j0 + NB <= pairs; j0 += NB) batch(j0, std::integral_constant<int, NB>());
+#pragma unroll 1
+            for (; j0 < pairs; ++j0) batch(j0, std::integral_constant<int, 1>());
+        }
+    };
+#define SBS_ROWS(k) _Pragma("unroll") for (int k = 0; k < places; ++k) if (fence(), k * B + (int)tid < n)
+    SBS_ROWS(k) {
+        if constexpr (kDiag) {
+            da[k] = elem(a.diagA + at(k), o1, 0);
+            dr[k] = elem(a.dinv + at(k), o1, 0);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const T s = elem(a.sn + 3 * at(k), o3, c);
+            P(k, c) = s;
+            X(k, c) = s;
+        }
+    }
+    __syncthreads();
+    // right-hand side and the PCG start: x = sn, r = b - A x
+    double acc[3][3] = {};  // r.z, z.z, (D^-1 b)^2 per component
+    SBS_ROWS(k) {
+        const size_t i = at(k) + tid;
         const T cv = a.c0[i];
-        const T fy = -a.gravity * a.mass[i];
-        const T inv = (T)1 / cv;
-        const T s0 = (a.X[3 * (size_t)g] - o[0]) + dt * a.V[3 * (size_t)g];
-        const T s1 = (a.X[3 * (size_t)g + 1] - o[1]) + dt * a.V[3 * (size_t)g + 1] + inv * fy;
-        const T s2 = (a.X[3 * (size_t)g + 2] - o[2]) + dt * a.V[3 * (size_t)g + 2];
-        T* sn = a.sn + 3 * (size_t)i;
-        T* so = a.sn_old + 3 * (size_t)i;
-        T* pv = a.prev + 3 * (size_t)i;
-        sn[0] = s0; sn[1] = s1; sn[2] = s2;
-        so[0] = s0; so[1] = s1; so[2] = s2;
-        pv[0] = s0; pv[1] = s1; pv[2] = s2;
+        T bv[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) bv[c] = cv * a.sn_old[3 * i + c];
+        const int e0 = a.vent_ptr[i], e1 = a.vent_ptr[i + 1];
+        for (int e = e0; e < e1; e += 4) {
+            T f[4][3];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) f[j][c] = a.partial[3 * (size_t)min(e + j, e1 - 1) + c];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (e + j < e1)
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) bv[c] += f[j][c];
+        }
+        if (a.dbc[i] > (T)0) {
+            // DBCX wdbc - c o (translation of b = DBCX wdbc by A o = c o):
+            // (DBCX - o) wdbc - (c - wdbc) o, where both differences are
+            // exact (nearby values), so nothing cancels
+            const uint32_t g = a.perm[i];
+            const T cw = cv - a.wdbc;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) bv[c] = (a.DBCX[3 * (size_t)g + c] - o[c]) * a.wdbc - cw * o[c];
+        }
+        const T dA = diag(k), di = dinv(k);
+        T Ax[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) Ax[c] = dA * P(k, c);
+        product(k, Ax);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const T rk = bv[c] - Ax[c];
+            const T zk = di * rk;
+            const T dbk = di * bv[c];
+            vec(rr, a.r, k, c) = rk;
+            acc[0][c] += (double)(rk * zk);
+            acc[1][c] += (double)(zk * zk);
+            acc[2][c] += (double)(dbk * dbk);
+        }
     }
-    __syncthreads();
-    int it_total = 0, solves = 0, max_solve = 0, cut = 0;
-    T omega = 1;
-    for (int i_outer = 0; i_outer < a.iters; ++i_outer) {
-        // computeLocal (R form, as the direct and PCG global steps use it)
-        for (int t = t0 + tid; t < t1; t += B) {
-            const uint4 tv = a.tets[t];
-            const T* m = a.dminv + 9 * (size_t)t;
-            T mm[9];
+    __syncthreads();  // the iterate has been read
+    SBS_ROWS(k) {
 #pragma unroll
-            for (int k = 0; k < 9; ++k) mm[k] = m[k];
-            const T* q0 = a.sn + 3 * (size_t)tv.x;
-            const T* q1 = a.sn + 3 * (size_t)tv.y;
-            const T* q2 = a.sn + 3 * (size_t)tv.z;
-            const T* q3 = a.sn + 3 * (size_t)tv.w;
-            T F[3][3];
+        for (int c = 0; c < 3; ++c) P(k, c) = dinv(k) * vec(rr, a.r, k, c);
+    }
+    // the scalars of component c in every lane of row c
+    double tot[3];
+    block_rows<3>(acc, tot, red[0], live);
+    int rb = 1;
+    T rz = (T)tot[0];
+    const T thr = max(a.tol2 * (T)tot[1], a.floor2 * (T)tot[2]);
+    bool act = (T)tot[1] > thr && row < 3;
+    int it = 0;
+    for (; it < a.max_iter && __ballot(act) != 0ull; ++it) {
+        // q = A p and p.q (p of every row was completed before the last barrier)
+        double pq[1][3] = {};
+        SBS_ROWS(k) {
+            const T dA = diag(k);
+            T y[3], pv[3];
 #pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                const T x0 = q0[r];
-                const T d0 = q1[r] - x0, d1 = q2[r] - x0, d2 = q3[r] - x0;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) F[r][k] = d0 * mm[k] + d1 * mm[3 + k] + d2 * mm[6 + k];
+            for (int c = 0; c < 3; ++c) {
+                pv[c] = P(k, c);
+                y[c] = dA * pv[c];
             }
-            T P[3][3];
-            pd_projection(F, false, P, a.polar != 0);
-            const T ww = a.w[t];
-            T* f = a.force + 12 * (size_t)t;
+            product(k, y);
 #pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                const T f1 = ww * (P[r][0] * mm[0] + P[r][1] * mm[1] + P[r][2] * mm[2]);
-                const T f2 = ww * (P[r][0] * mm[3] + P[r][1] * mm[4] + P[r][2] * mm[5]);
-                const T f3 = ww * (P[r][0] * mm[6] + P[r][1] * mm[7] + P[r][2] * mm[8]);
-                f[r] = -(f1 + f2 + f3);
-                f[3 + r] = f1;
-                f[6 + r] = f2;
-                f[9 + r] = f3;
+            for (int c = 0; c < 3; ++c) {
+                vec(qr, a.q, k, c) = y[c];
+                pq[0][c] += (double)(pv[c] * y[c]);
             }
         }
-        __syncthreads();
-        // right-hand side and the PCG start: x = sn, r = b - A x, p = z = D^-1 r
-        double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // r.z, z.z, (D^-1 b)^2 per component
-        for (int i = v0 + tid; i < v1; i += B) {
-            T bv[3];
-            const T cv = a.c0[i];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) bv[k] = cv * a.sn_old[3 * (size_t)i + k];
-            // the vertex's corner forces in incidence order, kRowBatch requested together
-            const int e0 = a.inc_ptr[i], e1 = a.inc_ptr[i + 1];
-            for (int eb = e0; eb < e1; eb += kRowBatch<T>) {
-                T fv[kRowBatch<T>][3];
-#pragma unroll
-                for (int jj = 0; jj < kRowBatch<T>; ++jj) {
-                    const uint32_t code = a.inc[eb + jj < e1 ? eb + jj : e1 - 1];
-                    const T* f = a.force + 12 * (size_t)(code >> 2) + 3 * (code & 3u);
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) fv[jj][k] = f[k];
-                }
-#pragma unroll
-                for (int jj = 0; jj < kRowBatch<T>; ++jj)
-                    if (eb + jj < e1)
-#pragma unroll
-                        for (int k = 0; k < 3; ++k) bv[k] += fv[jj][k];
-            }
-            if (a.dbc[i] > (T)0) {
-                // DBCX wdbc - c o (translation of b = DBCX wdbc by A o = c o):
-                // (DBCX - o) wdbc - (c - wdbc) o, where both differences are
-                // exact (nearby values), so nothing cancels
-                const uint32_t g = a.perm[i];
-                const T cw = cv - a.wdbc;
-#pragma unroll
-                for (int k = 0; k < 3; ++k) bv[k] = (a.DBCX[3 * (size_t)g + k] - o[k]) * a.wdbc - cw * o[k];
-            }
-            const T dA = a.diagA[i], di = (T)1 / dA;
-            T Ax[3];
-            const T* xs = a.sn + 3 * (size_t)i;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) Ax[k] = dA * xs[k];
-            const int il = i - v0;
-            for (int j0 = 0; j0 < width; j0 += kRowBatch<T>) {
-                uint32_t uu[kRowBatch<T>];
-                T vv[kRowBatch<T>];
-                row_entries(a, ebase, nrow, il, width, j0, uu, vv);
-                T xu[kRowBatch<T>][3];
-#pragma unroll
-                for (int jj = 0; jj < kRowBatch<T>; ++jj)
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) xu[jj][k] = a.sn[3 * (size_t)uu[jj] + k];
-#pragma unroll
-                for (int jj = 0; jj < kRowBatch<T>; ++jj)
-                    if (j0 + jj < width)
-#pragma unroll
-                        for (int k = 0; k < 3; ++k) Ax[k] += vv[jj] * xu[jj][k];
-            }
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const T rk = bv[k] - Ax[k];
-                const T zk = di * rk;
-                const T dbk = di * bv[k];
-                a.x[3 * (size_t)i + k] = xs[k];
-                a.r[3 * (size_t)i + k] = rk;
-                P(3 * (size_t)i + k) = zk;
-                acc[k] += (double)(rk * zk);
-                acc[3 + k] += (double)(zk * zk);
-                acc[6 + k] += (double)(dbk * dbk);
-            }
-        }
-        block_sum<9>(acc, red[rb]);
+        double tp[1];
+        block_rows<1>(pq, tp, red[rb], live);
         rb ^= 1;
-        T rz[3], thr[3];
-        bool act[3];
+        T alpha[3];
+        from_rows(act && tp[0] != 0.0 ? rz / (T)tp[0] : (T)0, alpha);
+        // x += alpha p, r -= alpha q, z = D^-1 r
+        double nz[2][3] = {};
+        SBS_ROWS(k) {
+            const T di = dinv(k);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            rz[k] = (T)acc[k];
-            const T zz = (T)acc[3 + k];
-            thr[k] = max(a.tol2 * zz, a.floor2 * (T)acc[6 + k]);
-            act[k] = zz > thr[k];
+            for (int c = 0; c < 3; ++c) {
+                X(k, c) += alpha[c] * P(k, c);
+                T& rv = vec(rr, a.r, k, c);
+                const T rk = rv - alpha[c] * vec(qr, a.q, k, c);
+                const T zk = di * rk;
+                rv = rk;
+                nz[0][c] += (double)(rk * zk);
+                nz[1][c] += (double)(zk * zk);
+            }
         }
-        int it = 0;
-        for (; it < a.max_iter && (act[0] || act[1] || act[2]); ++it) {
-            // q = A p and p.q (p of every row was completed before the last barrier)
-            double pq[3] = {0, 0, 0};
-            for (int i = v0 + tid; i < v1; i += B) {
-                const T dA = a.diagA[i];
-                const T pi[3] = {P(3 * (size_t)i), P(3 * (size_t)i + 1), P(3 * (size_t)i + 2)};
-                T qv[3] = {dA * pi[0], dA * pi[1], dA * pi[2]};
-                const int il = i - v0;
-                for (int j0 = 0; j0 < width; j0 += kRowBatch<T>) {
-                    uint32_t uu[kRowBatch<T>];
-                    T vv[kRowBatch<T>];
-                    row_entries(a, ebase, nrow, il, width, j0, uu, vv);
+        double tn[2];
+        block_rows<2>(nz, tn, red[rb], live);
+        rb ^= 1;
+        T beta[3];
+        from_rows(act && rz != (T)0 ? (T)tn[0] / rz : (T)0, beta);
+        rz = (T)tn[0];
+        SBS_ROWS(k) {
+            const T di = dinv(k);
 #pragma unroll
-                    for (int jj = 0; jj < kRowBatch<T>; ++jj)
-                        if (j0 + jj < width)
-#pragma unroll
-                            for (int k = 0; k < 3; ++k) qv[k] += vv[jj] * P(3 * (size_t)uu[jj] + k);
-                }
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    a.q[3 * (size_t)i + k] = qv[k];
-                    pq[k] += (double)(pi[k] * qv[k]);
-                }
-            }
-            block_sum<3>(pq, red[rb]);
-            rb ^= 1;
-            T alpha[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) alpha[k] = (act[k] && pq[k] != 0.0) ? rz[k] / (T)pq[k] : (T)0;
-            // x += alpha p, r -= alpha q, z = D^-1 r (kept in q: this row's q is used up)
-            double nz[6] = {0, 0, 0, 0, 0, 0};
-            for (int i = v0 + tid; i < v1; i += B) {
-                const T di = (T)1 / a.diagA[i];
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const size_t j = 3 * (size_t)i + k;
-                    const T pk = P(j), qk = a.q[j];
-                    a.x[j] += alpha[k] * pk;
-                    const T rk = a.r[j] - alpha[k] * qk;
-                    const T zk = di * rk;
-                    a.r[j] = rk;
-                    a.q[j] = zk;
-                    nz[k] += (double)(rk * zk);
-                    nz[3 + k] += (double)(zk * zk);
-                }
-            }
-            block_sum<6>(nz, red[rb]);
-            rb ^= 1;
-            T beta[3];
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                beta[k] = (act[k] && rz[k] != (T)0) ? (T)nz[k] / rz[k] : (T)0;
-                rz[k] = (T)nz[k];
-            }
-            for (int i = v0 + tid; i < v1; i += B)
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const size_t j = 3 * (size_t)i + k;
-                    P(j) = a.q[j] + beta[k] * P(j);
-                }
-#pragma unroll
-            for (int k = 0; k < 3; ++k) act[k] = act[k] && (T)nz[3 + k] > thr[k];
-            __syncthreads();
+            for (int c = 0; c < 3; ++c) P(k, c) = di * vec(rr, a.r, k, c) + beta[c] * P(k, c);
         }
-        it_total += it;
-        ++solves;
-        max_solve = it > max_solve ? it : max_solve;
-        cut += (act[0] || act[1] || act[2]) ? 1 : 0;
-        // Chebyshev (omega = 1 for i <= 10, then the semi-iteration's schedule)
-        if (i_outer <= 10) omega = 1;
-        else if (i_outer == 11) omega = (T)2 / ((T)2 - a.rho * a.rho);
-        else omega = (T)4 / ((T)4 - a.rho * a.rho * omega);
-        for (int i = v0 + tid; i < v1; i += B)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const size_t j = 3 * (size_t)i + k;
-                const T s = a.sn[j];
-                const T n = cheb(a.x[j], s, a.prev[j], omega);
-                a.prev[j] = s;
-                a.sn[j] = n;
-            }
+        act = act && (T)tn[1] > thr;
         __syncthreads();
     }
-    // updateVelPos (pdUtil.cu:180-193) and X <- XTilde (pdSolver.cu:227)
-    const T dt_inv = (T)1 / dt;
-    for (int i = v0 + tid; i < v1; i += B) {
-        const uint32_t g = a.perm[i];
+    // Chebyshev (omega = 1 for i <= 10, then the semi-iteration's schedule)
+    SBS_ROWS(k) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const T n = a.sn[3 * (size_t)i + k];
-            const size_t j = 3 * (size_t)g + k;
-            a.V[j] = (n - (a.XT[j] - o[k])) * dt_inv;
-            const T xa = n + o[k];
-            a.XT[j] = xa;
-            if (a.write_x) a.X[j] = xa;
+        for (int c = 0; c < 3; ++c) {
+            T* const sn = a.sn + 3 * at(k);
+            T* const prev = a.prev + 3 * at(k);
+            T& sv = elem(sn, o3, c);
+            T& pv = elem(prev, o3, c);
+            const T s = sv, nx = cheb(X(k, c), s, pv, omega);
+            pv = s;
+            sv = nx;
         }
     }
+#undef SBS_ROWS
+    const bool cut = __ballot(act) != 0ull;
     if (tid == 0) {
-        int* st = a.stats + 4 * (size_t)b;
-        st[0] += it_total;
-        st[1] += solves;
-        st[2] = max(st[2], max_solve);
-        st[3] += cut;
+        int* st = a.stats + 4 * (size_t)a.orig[b];
+        st[0] += it;
+        st[1] += 1;
+        st[2] = max(st[2], it);
+        st[3] += cut ? 1 : 0;
+    }
+}
+
+// One workgroup per body, the largest bodies first; the instance by the rows
+// per thread (uniform).  All bodies go in one launch: with a launch per size
+// class on a stream of its own the classes' launches ran one after the other
+// more often than side by side (256 bodies of 3..20 hexes per axis: 4.4 ms a
+// step, this form 3.17; 1,024 bodies 7.2 and 6.3).
+template <class T>
+__global__ void __launch_bounds__(1024) batch_solve_kernel(BatchArgs<T> a, unsigned lds_values, T omega) {
+    __shared__ double red[2][12 * kMaxWaves];
+    extern __shared__ __align__(16) unsigned char dyn_lds[];
+    T* const lp = reinterpret_cast<T*>(dyn_lds);
+    const int b = blockIdx.x;
+    // (uniform values said to be so: addresses then have scalar bases)
+    const int v0 = __builtin_amdgcn_readfirstlane(a.vptr[b]);
+    const int n = __builtin_amdgcn_readfirstlane(a.vptr[b + 1]) - v0;
+    const int width = __builtin_amdgcn_readfirstlane(a.ew[b]);
+    const int places = (n + (int)blockDim.x - 1) / (int)blockDim.x;
+    const bool regs = width <= kRegWidth;
+    if (n > kMaxNarrow) {
+        batch_solve_body<T, 0, false, false, true, true>(a, b, v0, n, width, omega, lp, red);
+    } else if (3u * (unsigned)n > lds_values) {
+        batch_solve_body<T, 0, false, false, true>(a, b, v0, n, width, omega, lp, red);
+    } else if (places <= 1 && regs) {
+        batch_solve_body<T, 1, true, true, false>(a, b, v0, n, width, omega, lp, red);
+    } else if (places <= 2 && regs && sizeof(T) == 4) {
+        if constexpr (sizeof(T) == 4)
+            batch_solve_body<T, 2, true, true, false>(a, b, v0, n, width, omega, lp, red);
+    } else if (places <= 2) {
+        batch_solve_body<T, 2, false, true, false>(a, b, v0, n, width, omega, lp, red);
+    } else if (places <= 4) {
+        batch_solve_body<T, 4, false, true, (sizeof(T) > 4)>(a, b, v0, n, width, omega, lp, red);
+    } else if (places <= 6 && blockDim.x == 1024 && sizeof(T) == 4) {
+        if constexpr (sizeof(T) == 4)
+            batch_solve_body<T, 6, false, true, true>(a, b, v0, n, width, omega, lp, red);
+    } else if (places <= 10 && blockDim.x == 1024 && sizeof(T) == 4) {
+        if constexpr (sizeof(T) == 4)
+            batch_solve_body<T, 10, false, true, true>(a, b, v0, n, width, omega, lp, red);
+    } else {
+        batch_solve_body<T, 0, false, true, true>(a, b, v0, n, width, omega, lp, red);
     }
 }
 
@@ -402,146 +524,171 @@ template <class T> BatchEngine<T>::BatchEngine(const BatchSystem<T>& s) {
             const int a = find((int)s.tets[4 * (size_t)t]), b = find((int)s.tets[4 * (size_t)t + k]);
             if (a != b) parent[std::max(a, b)] = std::min(a, b);
         }
-    std::vector<int> body_of_root(nv_, -1), body(nv_);
+    std::vector<int> body_of_root(nv_, -1), number(nv_);
     nb_ = 0;
     for (int v = 0; v < nv_; ++v) {  // bodies numbered by their first vertex
         const int r = find(v);
         if (body_of_root[r] < 0) body_of_root[r] = nb_++;
-        body[v] = body_of_root[r];
+        number[v] = body_of_root[r];
     }
+    verts_h_.assign(nb_, 0);
+    tets_h_.assign(nb_, 0);
+    for (int v = 0; v < nv_; ++v) verts_h_[number[v]]++;
+    for (int t = 0; t < nt_; ++t) tets_h_[number[s.tets[4 * (size_t)t]]]++;
+    // bodies are held largest first (a launch's workgroups start in that
+    // order); the reported classes end at the rows that one, two and four
+    // places of 1,024 threads take, and where columns need 32 bits
+    std::vector<int> order(nb_);  // place -> the caller's number
+    std::iota(order.begin(), order.end(), 0);
+    std::sort(order.begin(), order.end(),
+              [&](int x, int y) { return verts_h_[x] != verts_h_[y] ? verts_h_[x] > verts_h_[y] : x < y; });
+    max_verts_ = verts_h_[order[0]];
+    const int bounds[] = {0, 1024, 2048, 4096, kMaxNarrow, 0x7fffffff};
+    for (int c = 0; c < 5; ++c) {
+        BatchClass bc;
+        for (int b = 0; b < nb_; ++b) {
+            if (verts_h_[b] <= bounds[c] || verts_h_[b] > bounds[c + 1]) continue;
+            bc.min_tets = bc.bodies ? std::min(bc.min_tets, tets_h_[b]) : tets_h_[b];
+            bc.max_tets = std::max(bc.max_tets, tets_h_[b]);
+            ++bc.bodies;
+        }
+        if (bc.bodies) cls_.push_back(bc);
+    }
+    set_threads(round64((max_verts_ + 1) / 2));  // until the tuner chooses
+    std::vector<int> place(nb_);
+    for (int k = 0; k < nb_; ++k) place[order[k]] = k;
     // internal vertex order: body by body, caller order inside a body
-    vptr_h_.assign(nb_ + 1, 0);
-    for (int v = 0; v < nv_; ++v) vptr_h_[body[v] + 1]++;
-    for (int b = 0; b < nb_; ++b) vptr_h_[b + 1] += vptr_h_[b];
+    std::vector<int> vptr(nb_ + 1, 0);
+    for (int k = 0; k < nb_; ++k) vptr[k + 1] = vptr[k] + verts_h_[order[k]];
     std::vector<uint32_t> perm(nv_);
-    std::vector<int> inv(nv_), fill(vptr_h_.begin(), vptr_h_.end() - 1);
+    std::vector<int> inv(nv_), vbody(nv_), fill(vptr.begin(), vptr.end() - 1);
     for (int v = 0; v < nv_; ++v) {
-        const int i = fill[body[v]]++;
+        const int k = place[number[v]], i = fill[k]++;
         perm[i] = (uint32_t)v;
         inv[v] = i;
+        vbody[i] = k;
     }
-    // internal tet order: body by body, caller order inside a body
-    tptr_h_.assign(nb_ + 1, 0);
-    for (int t = 0; t < nt_; ++t) tptr_h_[body[s.tets[4 * (size_t)t]] + 1]++;
-    for (int b = 0; b < nb_; ++b) tptr_h_[b + 1] += tptr_h_[b];
-    std::vector<int> tfill(tptr_h_.begin(), tptr_h_.end() - 1);
-    std::vector<uint4> tets(std::max(nt_, 1));
-    std::vector<T> dminv(9 * (size_t)std::max(nt_, 1)), w(std::max(nt_, 1));
-    for (int t = 0; t < nt_; ++t) {
-        const int j = tfill[body[s.tets[4 * (size_t)t]]]++;
-        const uint32_t* tv = &s.tets[4 * (size_t)t];
-        tets[j] = make_uint4((unsigned)inv[tv[0]], (unsigned)inv[tv[1]], (unsigned)inv[tv[2]], (unsigned)inv[tv[3]]);
-        for (int k = 0; k < 9; ++k) dminv[9 * (size_t)j + k] = s.dminv[9 * (size_t)t + k];
-        w[j] = s.w[t];
-    }
-    // corner incidences per internal vertex, ascending internal tet
-    std::vector<int> inc_ptr(nv_ + 1, 0);
-    for (int j = 0; j < nt_; ++j) {
-        inc_ptr[tets[j].x + 1]++; inc_ptr[tets[j].y + 1]++; inc_ptr[tets[j].z + 1]++; inc_ptr[tets[j].w + 1]++;
-    }
-    for (int i = 0; i < nv_; ++i) inc_ptr[i + 1] += inc_ptr[i];
-    std::vector<uint32_t> inc(std::max(inc_ptr[nv_], 1));
-    std::vector<int> ifill(inc_ptr.begin(), inc_ptr.end() - 1);
-    for (int j = 0; j < nt_; ++j) {
-        const unsigned c[4] = {tets[j].x, tets[j].y, tets[j].z, tets[j].w};
-        for (int k = 0; k < 4; ++k) inc[ifill[c[k]]++] = ((uint32_t)j << 2) | (uint32_t)k;
-    }
-    // per-body ELL of the off-diagonal entries (column-major inside the body,
-    // padded with the row's own column and value 0); per-vertex constants
+    // per-body ELL of the off-diagonal entries, in pairs (entries 2 j and
+    // 2 j + 1 of a row side by side, pair-major inside the body, padded with
+    // the row's own place and value 0); per-vertex constants
     std::vector<int> eptr(nb_ + 1, 0), ew(nb_, 0);
-    std::vector<T> diagA(nv_), c0(nv_), mass(nv_), dbc(nv_);
+    std::vector<T> diagA(nv_), dinv(nv_), c0(nv_), mass(nv_), dbc(nv_);
     for (int i = 0; i < nv_; ++i) {
         const int v = (int)perm[i];
         diagA[i] = s.diagA[v];
         c0[i] = s.c0[v];
         mass[i] = s.mass[v];
         dbc[i] = s.dbc[v];
-        ew[body[v]] = std::max(ew[body[v]], s.rowptr[v + 1] - s.rowptr[v] - 1);
+        dinv[i] = (T)1 / s.diagA[v];
+        ew[vbody[i]] = std::max(ew[vbody[i]], s.rowptr[v + 1] - s.rowptr[v] - 1);
     }
-    for (int b = 0; b < nb_; ++b) eptr[b + 1] = eptr[b] + ew[b] * (vptr_h_[b + 1] - vptr_h_[b]);
-    std::vector<uint32_t> ecol(std::max(eptr[nb_], 1));
-    std::vector<T> eval(std::max(eptr[nb_], 1), (T)0);
+    // whole pairs; whole batches of pairs where the rows are read in every
+    // iteration (a body past the rows that fit the registers)
     for (int b = 0; b < nb_; ++b) {
-        const int n = vptr_h_[b + 1] - vptr_h_[b];
+        const int unit = vptr[b + 1] - vptr[b] > (int)(8192 / sizeof(T)) ? 2 * kPairBatch<T> : 2;
+        ew[b] = (ew[b] + unit - 1) / unit * unit;
+    }
+    size_t entries = 0;
+    bool wide = false;
+    for (int b = 0; b < nb_; ++b) {
+        const size_t n = (size_t)(vptr[b + 1] - vptr[b]);
+        wide = wide || n > (size_t)kMaxNarrow;
+        entries += n * (size_t)ew[b];
+        SBS_REQUIRE(entries < ((size_t)1 << 31), "batched PD: scene too large");
+        eptr[b + 1] = (int)entries;
+    }
+    std::vector<uint16_t> ecol(std::max<size_t>(entries, 1));
+    std::vector<uint32_t> ecol_wide(wide ? entries : 0);
+    std::vector<T> eval(std::max<size_t>(entries, 1), (T)0);
+    for (int b = 0; b < nb_; ++b) {
+        const int n = vptr[b + 1] - vptr[b];
+        auto place_of = [&](int j, int il) { return (size_t)eptr[b] + 2 * ((size_t)(j / 2) * n + il) + (j & 1); };
+        auto set_col = [&](size_t pos, int col) {
+            if (n > kMaxNarrow) ecol_wide[pos] = (uint32_t)(3 * col);
+            else ecol[pos] = (uint16_t)(3 * col);
+        };
         for (int il = 0; il < n; ++il) {
-            const int i = vptr_h_[b] + il, v = (int)perm[i];
+            const int v = (int)perm[vptr[b] + il];
             int j = 0;
             for (int e = s.rowptr[v]; e < s.rowptr[v + 1]; ++e) {
                 if (s.col[e] == v) continue;
-                const size_t pos = (size_t)eptr[b] + (size_t)j * n + il;
-                ecol[pos] = (uint32_t)inv[s.col[e]];
+                const size_t pos = place_of(j, il);
+                set_col(pos, inv[s.col[e]] - vptr[b]);
                 eval[pos] = s.val[e];
                 ++j;
             }
-            for (; j < ew[b]; ++j) {
-                const size_t pos = (size_t)eptr[b] + (size_t)j * n + il;
-                ecol[pos] = (uint32_t)i;
-                eval[pos] = 0;
-            }
+            for (; j < ew[b]; ++j) set_col(place_of(j, il), il);
         }
     }
-    SBS_REQUIRE(eptr[nb_] >= 0 && (size_t)nt_ * 4 < (1ull << 32), "batched PD: scene too large");
     // each body's origin: the rest position of its first vertex
     std::vector<T> origin(3 * (size_t)nb_);
     for (int b = 0; b < nb_; ++b)
-        for (int k = 0; k < 3; ++k) origin[3 * (size_t)b + k] = s.x0[3 * (size_t)perm[vptr_h_[b]] + k];
+        for (int k = 0; k < 3; ++k) origin[3 * (size_t)b + k] = s.x0[3 * (size_t)perm[vptr[b]] + k];
     upload(origin_, origin);
-    upload(vptr_, vptr_h_);
-    upload(tptr_, tptr_h_);
+    upload(vptr_, vptr);
     upload(eptr_, eptr);
     upload(ew_, ew);
+    upload(orig_, order);
+    upload(vbody_, vbody);
     upload(perm_, perm);
-    upload(tets_, tets);
-    upload(dminv_, dminv);
-    upload(w_, w);
-    upload(inc_ptr_, inc_ptr);
-    upload(inc_, inc);
     upload(ecol_, ecol);
+    if (wide) upload(ecol_wide_, ecol_wide);
     upload(eval_, eval);
     upload(diagA_, diagA);
+    upload(dinv_, dinv);
     upload(c0_, c0);
     upload(mass_, mass);
     upload(dbc_, dbc);
     const size_t n3 = 3 * (size_t)nv_;
     sn_.alloc(n3); sn_old_.alloc(n3); prev_.alloc(n3); x_.alloc(n3); r_.alloc(n3); p_.alloc(n3); q_.alloc(n3);
-    force_.alloc(12 * (size_t)std::max(nt_, 1));
     stats_.alloc(4 * (size_t)nb_);
     reset_stats();
-    // size classes by tet count (factor 4 apart from 1,024 tets), largest bodies first
-    const int bounds[] = {0, 1024, 4096, 16384, 1 << 30};
-    std::vector<int> list;
-    for (int c = 0; c < 4; ++c) {
-        std::vector<int> mem;
-        for (int b = 0; b < nb_; ++b) {
-            const int nt = tptr_h_[b + 1] - tptr_h_[b];
-            if (nt >= bounds[c] && nt < bounds[c + 1]) mem.push_back(b);
+    // the tets in chunks: body by body, along a Morton curve of the
+    // rest centroids inside a body
+    std::vector<std::vector<int>> tets_of(nb_);
+    for (int t = 0; t < nt_; ++t) tets_of[place[number[s.tets[4 * (size_t)t]]]].push_back(t);
+    std::vector<int> seq;
+    std::vector<std::pair<uint32_t, int>> key;
+    for (int b = 0; b < nb_; ++b) {
+        double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+        for (int i = vptr[b]; i < vptr[b + 1]; ++i)
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = std::min(lo[k], (double)s.x0[3 * (size_t)perm[i] + k]);
+                hi[k] = std::max(hi[k], (double)s.x0[3 * (size_t)perm[i] + k]);
+            }
+        key.clear();
+        for (int t : tets_of[b]) {
+            double cen[3] = {0, 0, 0};
+            for (int j = 0; j < 4; ++j)
+                for (int k = 0; k < 3; ++k) cen[k] += 0.25 * (double)s.x0[3 * (size_t)s.tets[4 * (size_t)t + j] + k];
+            key.emplace_back(morton_code(cen, lo, hi), t);
         }
-        if (mem.empty()) continue;
-        std::sort(mem.begin(), mem.end(), [&](int x, int y) {
-            const int a = tptr_h_[x + 1] - tptr_h_[x], b2 = tptr_h_[y + 1] - tptr_h_[y];
-            return a != b2 ? a > b2 : x < y;
-        });
-        BatchClass bc;
-        bc.min_tets = tptr_h_[mem.back() + 1] - tptr_h_[mem.back()];
-        bc.max_tets = tptr_h_[mem.front() + 1] - tptr_h_[mem.front()];
-        bc.bodies = (int)mem.size();
-        for (int b : mem) bc.max_verts = std::max(bc.max_verts, vptr_h_[b + 1] - vptr_h_[b]);
-        bc.threads = round64(bc.max_tets / 16);  // until the tuner chooses
-        cls_first_.push_back((int)list.size());
-        list.insert(list.end(), mem.begin(), mem.end());
-        cls_.push_back(bc);
+        std::sort(key.begin(), key.end());
+        for (const auto& q : key) seq.push_back(q.second);
     }
-    upload(body_list_, list);
-    for (size_t c = 0; c < cls_.size(); ++c) {
-        hipStream_t st;
-        SBS_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
-        streams_.push_back(st);
+    const int nt = (int)seq.size();
+    std::vector<uint32_t> tv(4 * (size_t)nt);
+    std::vector<T> dm(9 * (size_t)nt), w(nt);
+    for (int i = 0; i < nt; ++i) {
+        const size_t t = (size_t)seq[i];
+        for (int j = 0; j < 4; ++j) tv[4 * (size_t)i + j] = (uint32_t)(inv[s.tets[4 * t + j]]);
+        for (int k = 0; k < 9; ++k) dm[(size_t)k * nt + i] = s.dminv[9 * t + k];
+        w[i] = s.w[t];
     }
-    for (size_t k = 0; k < cls_.size() + 1; ++k) {
-        hipEvent_t e;
-        SBS_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        events_.push_back(e);
-    }
+    const ChunkLists ch = build_chunk_lists(nv_, tv);
+        chunks_ = ch.chunks;
+    local_lds_ = chunk_lds_bytes<T>(ch.max_verts);
+    SBS_REQUIRE(local_lds_ <= 64 * 1024, "batched PD: chunk vertex list exceeds LDS");
+    upload(lidx_, ch.lidx);
+    upload(chunk_vptr_, ch.vptr);
+    upload(chunk_verts_, ch.verts);
+    upload(entry_pos_, ch.pos);
+    upload(inc_codes_, ch.inc_codes);
+    upload(inc_end_, ch.inc_end);
+    upload(vent_ptr_, ch.vert_ptr);
+    upload(dminv_, dm);
+    upload(w_, w);
+    partial_.alloc(std::max<size_t>(3 * ch.verts.size(), 1));
     // LDS a workgroup may take for the search direction: the device's per-block
     // limit less the kernel's static 2.3 KB (64 KB unless it reports more)
     int dev = 0, lim = 0;
@@ -549,16 +696,16 @@ template <class T> BatchEngine<T>::BatchEngine(const BatchSystem<T>& s) {
     if (hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || lim <= 0)
         lim = 64 * 1024;
     lds_p_limit_ = (size_t)lim - 4096;
-    SBS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&batch_step_kernel<T, true>),
+    SBS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&batch_solve_kernel<T>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_p_limit_));
-}
-
-template <class T> BatchEngine<T>::~BatchEngine() {
-    for (auto s : streams_) {
-        (void)hipStreamSynchronize(s);
-        (void)hipStreamDestroy(s);
+    // the largest body whose direction fits
+    for (int k = 0; k < nb_; ++k) {
+        const size_t need = 3 * (size_t)verts_h_[order[k]] * sizeof(T);
+        if (need <= lds_p_limit_) {
+            solve_lds_ = need;
+            break;
+        }
     }
-    for (auto e : events_) (void)hipEventDestroy(e);
 }
 
 template <class T> void BatchEngine<T>::reset_stats() {
@@ -574,8 +721,8 @@ template <class T> std::vector<BatchBody> BatchEngine<T>::body_stats() {
     SBS_HIP(hipMemcpy(h.data(), stats_.get(), h.size() * sizeof(int), hipMemcpyDeviceToHost));
     std::vector<BatchBody> out(nb_);
     for (int b = 0; b < nb_; ++b) {
-        out[b].verts = vptr_h_[b + 1] - vptr_h_[b];
-        out[b].tets = tptr_h_[b + 1] - tptr_h_[b];
+        out[b].verts = verts_h_[b];
+        out[b].tets = tets_h_[b];
         out[b].iterations = h[4 * b];
         out[b].solves = h[4 * b + 1];
         out[b].max_per_solve = h[4 * b + 2];
@@ -584,30 +731,40 @@ template <class T> std::vector<BatchBody> BatchEngine<T>::body_stats() {
     return out;
 }
 
+template <class T> void BatchEngine<T>::set_threads(int threads) {
+    threads_ = threads;
+    for (BatchClass& c : cls_) c.threads = threads;
+}
+
 template <class T>
-void BatchEngine<T>::launch_class(int c, T* X, T* V, T* XT, const T* DBCX, const BatchParams& p, hipStream_t s,
-                                  int threads) {
+void BatchEngine<T>::step(T* X, T* V, T* XT, const T* DBCX, const BatchParams& p, hipStream_t stream) {
+    SBS_REQUIRE(p.iterations >= 0 && p.pcg_max_iter >= 1 && p.dt > 0, "batched PD: invalid parameters");
+    launch_step(X, V, XT, DBCX, p, stream, threads_);
+}
+
+template <class T>
+void BatchEngine<T>::launch_step(T* X, T* V, T* XT, const T* DBCX, const BatchParams& p, hipStream_t s, int threads) {
     SBS_REQUIRE(threads >= 64 && threads <= 64 * kMaxWaves && threads % 64 == 0,
                 "batched PD: workgroup size must be a multiple of 64 up to 1024");
     BatchArgs<T> a;
-    a.body_list = body_list_.get();
     a.vptr = vptr_.get();
-    a.tptr = tptr_.get();
     a.eptr = eptr_.get();
     a.ew = ew_.get();
+    a.orig = orig_.get();
+    a.vbody = vbody_.get();
     a.perm = perm_.get();
-    a.tets = tets_.get();
-    a.dminv = dminv_.get();
-    a.w = w_.get();
-    a.inc_ptr = inc_ptr_.get();
-    a.inc = inc_.get();
     a.ecol = ecol_.get();
+    a.ecol_wide = ecol_wide_.get();
     a.eval = eval_.get();
     a.diagA = diagA_.get();
+    a.dinv = dinv_.get();
     a.c0 = c0_.get();
     a.mass = mass_.get();
     a.dbc = dbc_.get();
     a.origin = origin_.get();
+    a.nv = nv_;
+    a.vent_ptr = vent_ptr_.get();
+    a.partial = partial_.get();
     a.X = X;
     a.V = V;
     a.XT = XT;
@@ -619,44 +776,33 @@ void BatchEngine<T>::launch_class(int c, T* X, T* V, T* XT, const T* DBCX, const
     a.r = r_.get();
     a.p = p_.get();
     a.q = q_.get();
-    a.force = force_.get();
     a.stats = stats_.get();
-    a.iters = p.iterations;
     a.max_iter = p.pcg_max_iter;
     a.write_x = p.write_x ? 1 : 0;
-    a.polar = p.polar ? 1 : 0;
     a.dt = (T)p.dt;
     a.gravity = (T)p.gravity;
-    a.rho = (T)p.rho;
     const T dt_inv = (T)1 / (T)p.dt;
     a.wdbc = (T)1e6 * (dt_inv * dt_inv);
     a.tol2 = (T)(p.pcg_tol * p.pcg_tol);
     a.floor2 = (T)(p.pcg_floor * p.pcg_floor);
-    const size_t lds = 3 * (size_t)cls_[c].max_verts * sizeof(T);
-    if (lds <= lds_p_limit_)
-        hipLaunchKernelGGL((batch_step_kernel<T, true>), dim3(cls_[c].bodies), dim3(threads), lds, s, a,
-                           cls_first_[c]);
-    else
-        hipLaunchKernelGGL((batch_step_kernel<T, false>), dim3(cls_[c].bodies), dim3(threads), 0, s, a,
-                           cls_first_[c]);
+    const unsigned vb = ceil_div((size_t)nv_, kTpbB);
+    hipLaunchKernelGGL(batch_begin_kernel<T>, dim3(vb), dim3(kTpbB), 0, s, a);
+    const T rho = (T)p.rho;
+    T omega = 1;
+    for (int i = 0; i < p.iterations; ++i) {
+        if (chunks_ > 0)
+            hipLaunchKernelGGL(batch_local_kernel<T>, dim3(chunks_), dim3(kChunkTets), local_lds_, s, nt_, lidx_.get(),
+                               chunk_vptr_.get(), chunk_verts_.get(), entry_pos_.get(), inc_codes_.get(),
+                               inc_end_.get(), dminv_.get(), w_.get(), (const T*)sn_.get(), partial_.get(),
+                               p.polar ? kLocalPolar : 0);
+        if (i <= 10) omega = 1;
+        else if (i == 11) omega = (T)2 / ((T)2 - rho * rho);
+        else omega = (T)4 / ((T)4 - rho * rho * omega);
+        hipLaunchKernelGGL(batch_solve_kernel<T>, dim3(nb_), dim3(threads), solve_lds_, s, a,
+                           (unsigned)(solve_lds_ / sizeof(T)), omega);
+    }
+    hipLaunchKernelGGL(batch_end_kernel<T>, dim3(vb), dim3(kTpbB), 0, s, a);
     SBS_HIP(hipGetLastError());
-}
-
-template <class T>
-void BatchEngine<T>::step(T* X, T* V, T* XT, const T* DBCX, const BatchParams& p, hipStream_t stream) {
-    SBS_REQUIRE(p.iterations >= 0 && p.pcg_max_iter >= 1 && p.dt > 0, "batched PD: invalid parameters");
-    if (cls_.size() == 1) {
-        launch_class(0, X, V, XT, DBCX, p, stream, cls_[0].threads);
-        return;
-    }
-    // fork: every class on its own stream, joined back into `stream`
-    SBS_HIP(hipEventRecord(events_[0], stream));
-    for (size_t c = 0; c < cls_.size(); ++c) {
-        SBS_HIP(hipStreamWaitEvent(streams_[c], events_[0], 0));
-        launch_class((int)c, X, V, XT, DBCX, p, streams_[c], cls_[c].threads);
-        SBS_HIP(hipEventRecord(events_[c + 1], streams_[c]));
-    }
-    for (size_t c = 0; c < cls_.size(); ++c) SBS_HIP(hipStreamWaitEvent(stream, events_[c + 1], 0));
 }
 
 template <class T>
@@ -666,38 +812,33 @@ void BatchEngine<T>::autotune(const T* X, const T* V, const T* DBCX, const Batch
     hipEvent_t e0, e1;
     SBS_HIP(hipEventCreate(&e0));
     SBS_HIP(hipEventCreate(&e1));
-    const int cand[] = {64, 128, 256, 512, 1024};
-    for (size_t c = 0; c < cls_.size(); ++c) {
-        cls_[c].tried.clear();
-        double best = 1e300;
-        int best_t = cls_[c].threads;
-        for (int th : cand) {
-            if (th > 64 && th / 2 >= round64(cls_[c].max_tets)) continue;  // more threads than tets: no gain
-            double ms_best = 1e300;
-            for (int rep = 0; rep < 3; ++rep) {  // one warm-up, then the faster of two
-                SBS_HIP(hipMemcpyAsync(xc.get(), X, n3 * sizeof(T), hipMemcpyDeviceToDevice, stream));
-                SBS_HIP(hipMemcpyAsync(vc.get(), V, n3 * sizeof(T), hipMemcpyDeviceToDevice, stream));
-                SBS_HIP(hipMemcpyAsync(tc.get(), X, n3 * sizeof(T), hipMemcpyDeviceToDevice, stream));
-                SBS_HIP(hipEventRecord(e0, stream));
-                launch_class((int)c, xc.get(), vc.get(), tc.get(), DBCX, p, stream, th);
-                SBS_HIP(hipEventRecord(e1, stream));
-                SBS_HIP(hipEventSynchronize(e1));
-                float ms = 0;
-                SBS_HIP(hipEventElapsedTime(&ms, e0, e1));
-                if (rep > 0) ms_best = std::min(ms_best, (double)ms);
-            }
-            cls_[c].tried.emplace_back(th, ms_best);
-            if (ms_best < best) {
-                best = ms_best;
-                best_t = th;
-            }
+    std::vector<std::pair<int, double>> tried;
+    double best = 1e300;
+    int best_t = threads_;
+    for (int th : {64, 128, 256, 512, 1024}) {
+        if (th > 64 && th / 2 >= round64(max_verts_)) continue;              // more threads than rows: no gain
+        if (th < 1024 && (max_verts_ + th - 1) / th > 4) continue;           // rows would leave the registers
+        double ms_best = 1e300;
+        for (int rep = 0; rep < 3; ++rep) {  // one warm-up, then the faster of two
+            SBS_HIP(hipMemcpyAsync(xc.get(), X, n3 * sizeof(T), hipMemcpyDeviceToDevice, stream));
+            SBS_HIP(hipMemcpyAsync(vc.get(), V, n3 * sizeof(T), hipMemcpyDeviceToDevice, stream));
+            SBS_HIP(hipMemcpyAsync(tc.get(), X, n3 * sizeof(T), hipMemcpyDeviceToDevice, stream));
+            SBS_HIP(hipEventRecord(e0, stream));
+            launch_step(xc.get(), vc.get(), tc.get(), DBCX, p, stream, th);
+            SBS_HIP(hipEventRecord(e1, stream));
+            SBS_HIP(hipEventSynchronize(e1));
+            float ms = 0;
+            SBS_HIP(hipEventElapsedTime(&ms, e0, e1));
+            if (rep > 0) ms_best = std::min(ms_best, (double)ms);
         }
-        // the classes share the CUs when they run together: of the sizes within
-        // 5% of the fastest, the smallest workgroup leaves the most room
-        for (const auto& tm : cls_[c].tried)
-            if (tm.second <= 1.05 * best && tm.first < best_t) best_t = tm.first;
-        cls_[c].threads = best_t;
+        tried.emplace_back(th, ms_best);
+        if (ms_best < best) {
+            best = ms_best;
+            best_t = th;
+        }
     }
+    for (BatchClass& c : cls_) c.tried = tried;
+    set_threads(best_t);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     reset_stats();

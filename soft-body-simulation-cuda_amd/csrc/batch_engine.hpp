@@ -1,11 +1,15 @@
 // Batched PD step for many independent bodies on gfx950: every body advances
 // with its own Jacobi-PCG global solve (its own alpha, beta and stop test,
-// pcgJacobi.cu:134-135 applied per body) inside one persistent launch per
-// body-size class, one workgroup per body running the whole step: the
-// prologue, the local/global iterations (computeLocal, the right-hand side,
-// the PCG solve, the Chebyshev recurrence) and updateVelPos
-// (pdSolver.cu:141-208).  The classes launch on their own streams, so a
-// captured step is one graph with a branch per class.
+// pcgJacobi.cu:134-135 applied per body).  The step (pdSolver.cu:141-208) is a
+// sequence of launches over all bodies: the prologue, then per local/global
+// iteration computeLocal over the tet chunks of all bodies (so the tets of the
+// largest body spread over the CUs) and one launch with a workgroup per body
+// that gathers the right-hand side, runs the whole PCG solve and applies the
+// Chebyshev recurrence, then updateVelPos.  One stream, so a captured step is
+// a chain.  (One workgroup running a body's whole step, local step included,
+// was bound by the largest body's chain: 256 bodies of 3..20 hexes per axis,
+// 10 iterations, 10.5-12.9 ms a step; this form 3.17 ms;
+// 1,024 such bodies 19.3 -> 6.3 ms.)
 //
 // Bodies are the connected components of the tet mesh (the reference's
 // DataLoader concatenates bodies, dataLoader.cu:292-378; they stay
@@ -18,9 +22,9 @@
 // rather than of its distance from the world origin; dot products accumulate
 // in FP64.
 //
-// Tile choice: the workgroup size of each class (64..1024 threads) comes from
-// an autotuner that times one step of the class with every candidate on a
-// copy of the state at prepare.
+// Tile choice: the workgroup size (64..1024 threads, shared by all bodies)
+// comes from an autotuner that times one step with every candidate on a copy
+// of the state at prepare.
 #pragma once
 
 #include <memory>
@@ -35,9 +39,9 @@ struct BatchBody {
     int verts = 0, tets = 0, iterations = 0, solves = 0, max_per_solve = 0, unconverged = 0;
 };
 
+// Bodies by size, for reports: the classes share the launches.
 struct BatchClass {
     int min_tets = 0, max_tets = 0, bodies = 0, threads = 0;  // threads per workgroup chosen by the tuner
-    int max_verts = 0;                                        // vertices of the class's largest body
     std::vector<std::pair<int, double>> tried;               // (threads, ms of one step) the tuner measured
 };
 
@@ -64,11 +68,10 @@ struct BatchParams {
 template <class T> class BatchEngine {
 public:
     explicit BatchEngine(const BatchSystem<T>& sys);
-    ~BatchEngine();
-    // One step of every body on `stream` (and the class streams joined back
-    // into it); X, V, XTilde and DBCX are the caller's arrays.
+    // One step of every body on `stream`; X, V, XTilde and DBCX are the caller's
+    // arrays.
     void step(T* X, T* V, T* XTilde, const T* DBCX, const BatchParams& p, hipStream_t stream);
-    // Chooses each class's workgroup size by timing one step per candidate on
+    // Chooses the workgroup size by timing one step per candidate on
     // copies of X, V, XTilde (the caller's state is not changed).
     void autotune(const T* X, const T* V, const T* DBCX, const BatchParams& p, hipStream_t stream);
     int num_bodies() const { return nb_; }
@@ -78,22 +81,28 @@ public:
     void reset_stats();
 
 private:
-    void launch_class(int c, T* X, T* V, T* XTilde, const T* DBCX, const BatchParams& p, hipStream_t s, int threads);
+    void launch_step(T* X, T* V, T* XTilde, const T* DBCX, const BatchParams& p, hipStream_t s, int threads);
+    void set_threads(int threads);
 
-    int nv_ = 0, nt_ = 0, nb_ = 0;
-    std::vector<int> vptr_h_, tptr_h_;
+    int nv_ = 0, nt_ = 0, nb_ = 0, max_verts_ = 0, threads_ = 256;
+    std::vector<int> verts_h_, tets_h_;  // per body, the caller's order
+    // the tets in chunks
+    int chunks_ = 0;
+    size_t local_lds_ = 0;               // of a chunk's workgroup
+    DevBuf<uint2> lidx_;
+    DevBuf<int> chunk_vptr_, vent_ptr_;
+    DevBuf<uint32_t> chunk_verts_, entry_pos_;
+    DevBuf<uint16_t> inc_codes_, inc_end_;
+    DevBuf<T> dminv_, w_, partial_;
     size_t lds_p_limit_ = 0;  // largest search direction (bytes) a workgroup keeps in LDS
-    DevBuf<int> vptr_, tptr_, eptr_, ew_, body_list_;
-    DevBuf<uint32_t> perm_, ecol_, inc_;
-    DevBuf<int> inc_ptr_;
-    DevBuf<uint4> tets_;
-    DevBuf<T> dminv_, w_, eval_, diagA_, c0_, mass_, dbc_, origin_;
-    DevBuf<T> sn_, sn_old_, prev_, x_, r_, p_, q_, force_;
+    size_t solve_lds_ = 0;    // of the largest body that fits
+    DevBuf<int> vptr_, eptr_, ew_, orig_, vbody_;
+    DevBuf<uint32_t> perm_, ecol_wide_;
+    DevBuf<uint16_t> ecol_;
+    DevBuf<T> eval_, diagA_, dinv_, c0_, mass_, dbc_, origin_;
+    DevBuf<T> sn_, sn_old_, prev_, x_, r_, p_, q_;
     DevBuf<int> stats_;
     std::vector<BatchClass> cls_;
-    std::vector<int> cls_first_;      // offset of each class's bodies in body_list_
-    std::vector<hipStream_t> streams_;
-    std::vector<hipEvent_t> events_;  // fork + one join per class
 };
 
 }  // namespace sbs

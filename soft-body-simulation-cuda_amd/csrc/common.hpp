@@ -153,4 +153,31 @@ __device__ __forceinline__ double wave_total(double v) {
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// a + its other half-wavefront's value in lanes 0..31, b + its other half's in
+// lanes 32..63: one swap of halves per 32 bits and one add for two quantities.
+__device__ __forceinline__ double fold_halves(double a, double b) {
+    const unsigned long long x = (unsigned long long)__double_as_longlong(a);
+    const unsigned long long y = (unsigned long long)__double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+           __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+// The same with neighbouring rows of 16 lanes: a's sums in rows 0 and 2, b's in
+// rows 1 and 3.
+__device__ __forceinline__ double fold_rows(double a, double b) {
+    const unsigned long long x = (unsigned long long)__double_as_longlong(a);
+    const unsigned long long y = (unsigned long long)__double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return __longlong_as_double((long long)(((unsigned long long)hi[0] << 32) | lo[0])) +
+           __longlong_as_double((long long)(((unsigned long long)hi[1] << 32) | lo[1]));
+}
+// Sums of four doubles over the wavefront, quantity r in every lane of row r
+// of 16 lanes: 21 instructions for the four, where a wave_total each takes
+// 18.  Every lane of the wavefront must be active.
+__device__ __forceinline__ double wave_rows4(double q0, double q1, double q2, double q3) {
+    return row16_total(fold_rows(fold_halves(q0, q2), fold_halves(q1, q3)));
+}
+
 }  // namespace sbs

@@ -10,6 +10,7 @@
 #include "dense_refine.hpp"
 #include "direct_solver.hpp"
 #include "halo_tiles.hpp"
+#include "local_chunk.hpp"
 #include "pd_engine.hpp"
 #include "batch_engine.hpp"
 #include "svd3.hpp"
@@ -266,11 +267,6 @@ __global__ void __launch_bounds__(kTpb) fem_precompute_kernel(int nt, const T* _
     v0[i] = vol;
     w[i] = fabs(vol) * mu[t];
     if (v0_out) v0_out[t] = vol;
-}
-
-template <class T> __device__ __forceinline__ void load_dminv(const T* __restrict__ dminv, int nt, unsigned t, T (&m)[9]) {
-#pragma unroll
-    for (int k = 0; k < 9; ++k) m[k] = dminv[(size_t)k * nt + t];
 }
 
 // ---------------------------------------------------------------------------
@@ -816,14 +812,6 @@ template <class T> __device__ __forceinline__ PcgStep pcg_state(const PcgArgs<T>
 #define SBS_ITER_BATCH 4
 #endif
 constexpr int kIterBatch = SBS_ITER_BATCH;  // neighbours in flight per row in the iteration kernel
-// Unroll of the local step's per-vertex incidence sums: the LDS reads of
-// several incidences are in flight together (the sum keeps its order).
-#ifndef SBS_GATHER_UNROLL
-#define SBS_GATHER_UNROLL 2
-#endif
-#define SBS_PRAGMA(x) _Pragma(#x)
-#define SBS_UNROLL(n) SBS_PRAGMA(unroll n)
-
 // One PCG iteration.  Everything that does not depend on alpha_i, beta_i is
 // issued first: the row's own values and the three neighbour sums
 //   Yr = sum m D^-1 r_i,  Yw = sum m D^-1 w_i,  Ys = sum m D^-1 s_{i-1}
@@ -948,19 +936,9 @@ __global__ void __launch_bounds__(kTpb) pcg_finish_kernel(PcgArgs<T> a, int L, i
 
 // ---------------------------------------------------------------------------
 // computeLocal (src/simulation/solver/projective/pdUtil.cu:97-145), one
-// workgroup per chunk of kChunkTets Morton-ordered tets:
-//   1. the chunk's vertices (a sorted list) are staged from q into LDS, with
-//      the chunk's incidence list (per vertex, the (tet, corner) pairs that
-//      touch it, in tet order);
-//   2. one thread per tet: F = Ds Dm^-1, 3x3 SVD in registers, R (or R - F),
-//      the 4 corner forces of w R Dm^-T G^T written to LDS (plain stores);
-//   3. one thread per chunk vertex sums its incidences in list order (the
-//      three components together, each code decoded once) and writes the
-//      chunk's partial force for that vertex at the vertex's slot of the
-//      vertex-major partial array.
-// No atomics anywhere, so the result is deterministic; float atomics on LDS
-// serialise on the shared corners of neighbouring tets and were the
-// bottleneck of the scatter form.
+// workgroup per chunk of kChunkTets Morton-ordered tets (see local_chunk).
+// Float atomics on LDS serialise on the shared corners of neighbouring tets
+// and were the bottleneck of the scatter form.
 //
 // With kFold the kernel also finishes the previous PCG solve (instead of a
 // finish launch of its own): block 0 evaluates that solve's last stop test and
@@ -981,10 +959,6 @@ template <class T> struct FoldIn {
     T omega;
 };
 
-// flags of the local step
-constexpr int kLocalResidual = 1;  // P = R - F (Jacobi mode) instead of R
-constexpr int kLocalPolar = 2;     // FP32: rotation by Newton's polar iteration (SVD fallback)
-
 template <class T, bool kFold>
 __global__ void __launch_bounds__(kChunkTets) local_chunk_kernel(
     int nt, const uint2* __restrict__ lidx, const int* __restrict__ chunk_vptr,
@@ -1003,16 +977,10 @@ __global__ void __launch_bounds__(kChunkTets) local_chunk_kernel(
         for (int i = threadIdx.x; i < zero_n; i += kChunkTets) zero_slots[i] = 0.0;
     }
     const unsigned c = xcd_block(blockIdx.x, gridDim.x);
-    const int e0 = chunk_vptr[c], nu = chunk_vptr[c + 1] - e0;
-    T* fs = reinterpret_cast<T*>(smem_raw);                    // [12][kChunkTets] corner forces
-    T* qs = fs + 12 * kChunkTets;                              // [nu][3] staged q
-    uint16_t* codes = reinterpret_cast<uint16_t*>(qs + 3 * (size_t)nu);  // [4 kChunkTets] tet<<2 | corner
-    uint16_t* ends = codes + 4 * kChunkTets;                   // [nu] end of each vertex's incidences
-    for (int i = threadIdx.x; i < nu; i += kChunkTets) {
-        const uint32_t g = chunk_verts[e0 + i];
-        T x, y, z;
+    local_chunk<T>(c, nt, lidx, chunk_vptr, chunk_verts, entry_pos, inc_codes, inc_end, dminv, w, partial, flags,
+                   smem_raw, [&](int e, uint32_t g, T& x, T& y, T& z) {
         if (kFold) {
-            const uint32_t rw = fold.rows[e0 + i];
+            const uint32_t rw = fold.rows[e];
             T v[3], sv[3], pv[3];
             ld3(fold.x, rw & 0x7fffffffu, v[0], v[1], v[2]);
             ld3(fold.sn_in, g, sv[0], sv[1], sv[2]);
@@ -1026,60 +994,7 @@ __global__ void __launch_bounds__(kChunkTets) local_chunk_kernel(
         } else {
             ld3(q, g, x, y, z);
         }
-        qs[3 * i] = x; qs[3 * i + 1] = y; qs[3 * i + 2] = z;
-        ends[i] = inc_end[e0 + i];
-    }
-    {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(inc_codes) + (size_t)c * (2 * kChunkTets);
-        uint32_t* dst = reinterpret_cast<uint32_t*>(codes);
-        for (int k = threadIdx.x; k < 2 * kChunkTets; k += kChunkTets) dst[k] = src[k];
-    }
-    __syncthreads();
-    const unsigned t = c * kChunkTets + threadIdx.x;
-    if (t < (unsigned)nt) {
-        const uint2 li = lidx[t];
-        const unsigned l0 = li.x & 0xffffu, l1 = li.x >> 16, l2 = li.y & 0xffffu, l3 = li.y >> 16;
-        T m[9];
-        load_dminv(dminv, nt, t, m);
-        const T ww = w[t];
-        T F[3][3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            const T x0 = qs[3 * l0 + r];
-            const T d0 = qs[3 * l1 + r] - x0, d1 = qs[3 * l2 + r] - x0, d2 = qs[3 * l3 + r] - x0;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) F[r][k] = d0 * m[k] + d1 * m[3 + k] + d2 * m[6 + k];
-        }
-        T P[3][3];
-        pd_projection(F, (flags & kLocalResidual) != 0, P, (flags & kLocalPolar) != 0);
-#pragma unroll
-        for (int r = 0; r < 3; ++r) {
-            // column j of w P Dm^-T is w P (row j of Dm^-1); corner 0 gets minus their sum
-            const T f1 = ww * (P[r][0] * m[0] + P[r][1] * m[1] + P[r][2] * m[2]);
-            const T f2 = ww * (P[r][0] * m[3] + P[r][1] * m[4] + P[r][2] * m[5]);
-            const T f3 = ww * (P[r][0] * m[6] + P[r][1] * m[7] + P[r][2] * m[8]);
-            fs[(0 * 3 + r) * kChunkTets + threadIdx.x] = -(f1 + f2 + f3);
-            fs[(1 * 3 + r) * kChunkTets + threadIdx.x] = f1;
-            fs[(2 * 3 + r) * kChunkTets + threadIdx.x] = f2;
-            fs[(3 * 3 + r) * kChunkTets + threadIdx.x] = f3;
-        }
-    }
-    __syncthreads();
-    // one thread per chunk vertex sums all three components, so each
-    // incidence code is read and decoded once
-    for (int i = threadIdx.x; i < nu; i += kChunkTets) {
-        const int k1 = ends[i];
-        T a0 = 0, a1 = 0, a2 = 0;
-        SBS_UNROLL(SBS_GATHER_UNROLL)
-        for (int k = i ? ends[i - 1] : 0; k < k1; ++k) {
-            const unsigned code = codes[k];
-            const T* f = fs + (code & 3u) * 3 * kChunkTets + (code >> 2);
-            a0 += f[0];
-            a1 += f[kChunkTets];
-            a2 += f[2 * kChunkTets];
-        }
-        st3(partial, entry_pos[e0 + i], a0, a1, a2);  // vertex-major: the consumers read contiguously
-    }
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -1561,65 +1476,18 @@ template <class T> void PdEngine<T>::build_chunks(const std::vector<double>& X0h
     std::sort(key.begin(), key.end());
     tet_perm_.resize(nt_);
     for (int i = 0; i < nt_; ++i) tet_perm_[i] = (int)(key[i] & 0xffffffffu);
-    nchunks_ = (nt_ + kChunkTets - 1) / kChunkTets;
-    std::vector<int> cvptr(nchunks_ + 1, 0);
-    std::vector<uint32_t> cverts;
-    cverts.reserve((size_t)nt_ * 2);
-    std::vector<uint2> lidx(nt_);
-    std::vector<uint32_t> tmp;
-    std::vector<int> cnt(4 * kChunkTets);
-    std::vector<uint16_t> inc_end;
-    inc_end.reserve((size_t)nt_ * 2);
-    std::vector<uint16_t> inc_codes((size_t)((nt_ + kChunkTets - 1) / kChunkTets) * 4 * kChunkTets, 0);
-    chunk_max_verts_ = 0;
-    for (int c = 0; c < nchunks_; ++c) {
-        const int t0 = c * kChunkTets, t1 = std::min(nt_, t0 + kChunkTets);
-        tmp.clear();
-        for (int i = t0; i < t1; ++i)
-            for (int j = 0; j < 4; ++j) tmp.push_back(host_tets_[4 * (size_t)tet_perm_[i] + j]);
-        std::sort(tmp.begin(), tmp.end());
-        tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
-        chunk_max_verts_ = std::max(chunk_max_verts_, (int)tmp.size());
-        std::fill(cnt.begin(), cnt.end(), 0);
-        for (int i = t0; i < t1; ++i) {
-            uint32_t l[4];
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t g = host_tets_[4 * (size_t)tet_perm_[i] + j];
-                l[j] = (uint32_t)(std::lower_bound(tmp.begin(), tmp.end(), g) - tmp.begin());
-                cnt[l[j]]++;
-            }
-            lidx[i] = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
-        }
-        // incidence list of the chunk: per local vertex, (tet << 2 | corner) in tet order
-        const size_t nloc = tmp.size();
-        std::vector<int> pos(nloc + 1, 0);
-        for (size_t k = 0; k < nloc; ++k) pos[k + 1] = pos[k] + cnt[k];
-        for (size_t k = 0; k < nloc; ++k) inc_end.push_back((uint16_t)pos[k + 1]);
-        uint16_t* codes = &inc_codes[(size_t)c * 4 * kChunkTets];
-        for (int i = t0; i < t1; ++i)
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t word = j < 2 ? lidx[i].x : lidx[i].y;
-                const uint32_t lv = (j & 1) ? word >> 16 : word & 0xffffu;
-                codes[pos[lv]++] = (uint16_t)(((i - t0) << 2) | j);
-            }
-        cverts.insert(cverts.end(), tmp.begin(), tmp.end());
-        cvptr[c + 1] = (int)cverts.size();
-    }
-    nentries_ = cverts.size();
-    // vertex -> entries
-    std::vector<int> vptr(nv_ + 1, 0);
-    for (uint32_t g : cverts) vptr[g + 1]++;
-    for (int v = 0; v < nv_; ++v) vptr[v + 1] += vptr[v];
-    std::vector<uint32_t> vent(nentries_);
-    std::vector<int> fill(vptr.begin(), vptr.end() - 1);
-    for (size_t e = 0; e < nentries_; ++e) vent[fill[cverts[e]]++] = (uint32_t)e;
-    std::vector<uint32_t> epos(nentries_);  // entry -> its slot in vertex-major order
-    for (size_t j = 0; j < nentries_; ++j) epos[vent[j]] = (uint32_t)j;
-    host_cverts_ = cverts;
-    host_vptr_ = vptr;
+    std::vector<uint32_t> ordered(4 * (size_t)nt_);
+    for (int i = 0; i < nt_; ++i)
+        for (int j = 0; j < 4; ++j) ordered[4 * (size_t)i + j] = host_tets_[4 * (size_t)tet_perm_[i] + j];
+    const ChunkLists ch = build_chunk_lists(nv_, ordered);
+    nchunks_ = ch.chunks;
+    chunk_max_verts_ = ch.max_verts;
+    nentries_ = ch.verts.size();
+    host_cverts_ = ch.verts;
+    host_vptr_ = ch.vert_ptr;
     host_first_.assign(nentries_, 0);
     for (int v = 0; v < nv_; ++v)
-        if (vptr[v + 1] > vptr[v]) host_first_[vent[vptr[v]]] = 1;
+        if (ch.vert_ptr[v + 1] > ch.vert_ptr[v]) host_first_[ch.entry[ch.vert_ptr[v]]] = 1;
     tet_perm_d_.alloc(nt_);
     tet_lidx_.alloc(nt_);
     chunk_vptr_.alloc(nchunks_ + 1);
@@ -1627,16 +1495,16 @@ template <class T> void PdEngine<T>::build_chunks(const std::vector<double>& X0h
     vent_ptr_.alloc(nv_ + 1);
     entry_pos_.alloc(nentries_);
     partial_f_.alloc(3 * nentries_);
-    inc_codes_.alloc(inc_codes.size());
-    inc_end_.alloc(std::max<size_t>(1, inc_end.size()));
-    SBS_HIP(hipMemcpy(inc_codes_.get(), inc_codes.data(), inc_codes.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
-    SBS_HIP(hipMemcpy(inc_end_.get(), inc_end.data(), inc_end.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+    inc_codes_.alloc(ch.inc_codes.size());
+    inc_end_.alloc(std::max<size_t>(1, ch.inc_end.size()));
+    SBS_HIP(hipMemcpy(inc_codes_.get(), ch.inc_codes.data(), ch.inc_codes.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+    SBS_HIP(hipMemcpy(inc_end_.get(), ch.inc_end.data(), ch.inc_end.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
     SBS_HIP(hipMemcpy(tet_perm_d_.get(), tet_perm_.data(), nt_ * sizeof(int), hipMemcpyHostToDevice));
-    SBS_HIP(hipMemcpy(tet_lidx_.get(), lidx.data(), nt_ * sizeof(uint2), hipMemcpyHostToDevice));
-    SBS_HIP(hipMemcpy(chunk_vptr_.get(), cvptr.data(), cvptr.size() * sizeof(int), hipMemcpyHostToDevice));
-    SBS_HIP(hipMemcpy(chunk_verts_.get(), cverts.data(), nentries_ * sizeof(uint32_t), hipMemcpyHostToDevice));
-    SBS_HIP(hipMemcpy(vent_ptr_.get(), vptr.data(), vptr.size() * sizeof(int), hipMemcpyHostToDevice));
-    SBS_HIP(hipMemcpy(entry_pos_.get(), epos.data(), nentries_ * sizeof(uint32_t), hipMemcpyHostToDevice));
+    SBS_HIP(hipMemcpy(tet_lidx_.get(), ch.lidx.data(), nt_ * sizeof(uint2), hipMemcpyHostToDevice));
+    SBS_HIP(hipMemcpy(chunk_vptr_.get(), ch.vptr.data(), ch.vptr.size() * sizeof(int), hipMemcpyHostToDevice));
+    SBS_HIP(hipMemcpy(chunk_verts_.get(), ch.verts.data(), nentries_ * sizeof(uint32_t), hipMemcpyHostToDevice));
+    SBS_HIP(hipMemcpy(vent_ptr_.get(), ch.vert_ptr.data(), ch.vert_ptr.size() * sizeof(int), hipMemcpyHostToDevice));
+    SBS_HIP(hipMemcpy(entry_pos_.get(), ch.pos.data(), nentries_ * sizeof(uint32_t), hipMemcpyHostToDevice));
 }
 
 // Sliced-ELL structure of the off-diagonal scalar pattern, built on the host
@@ -1857,7 +1725,7 @@ template <class T> void PdEngine<T>::direct_factor(const PdParams& params) {
 }
 
 // BatchedPCG: the bodies (connected components), their systems from the
-// assembled matrix, and the tuned workgroup size of each size class.
+// assembled matrix, and the tuned workgroup size.
 template <class T> void PdEngine<T>::build_batch(const PdParams& params) {
     SBS_REQUIRE(system_built_, "batched solver requested before the system was assembled");
     drop_graph();
@@ -1914,12 +1782,7 @@ template <class T> void PdEngine<T>::dense_info(int* bodies, int* max_body, long
     if (iterations || ratio) dense_->last_result(iterations, ratio);
 }
 
-// LDS of one local-step workgroup: corner forces, staged q, incidence list.
-template <class T> size_t PdEngine<T>::local_lds_bytes() const {
-    const size_t b = (12 * (size_t)kChunkTets + 3 * (size_t)chunk_max_verts_) * sizeof(T) +
-                     (4 * (size_t)kChunkTets + (size_t)chunk_max_verts_) * sizeof(uint16_t);
-    return (b + 15) & ~(size_t)15;
-}
+template <class T> size_t PdEngine<T>::local_lds_bytes() const { return chunk_lds_bytes<T>(chunk_max_verts_); }
 
 template <class T> void PdEngine<T>::launch_local(const T* q, bool residual_form, const int* skip) {
     const size_t lds = local_lds_bytes();
@@ -2256,7 +2119,7 @@ template <class T> void PdEngine<T>::enqueue_step(PdData<T>& data, const PdParam
     const bool fold = pcg && cheb && params.pcg_halo && halo_groups_ > 0 && chunk_rows_.get() != nullptr;
     hipLaunchKernelGGL(ctl_init_kernel, dim3(1), dim3(64), 0, stream_, ctl);
     if (solver_ == GlobalSolver::BatchedPCG) {
-        // every body's whole step in one persistent launch per size class
+        // every body on its own, see batch_engine.hpp
         BatchParams bp;
         bp.iterations = params.num_iterations;
         bp.dt = params.dt;

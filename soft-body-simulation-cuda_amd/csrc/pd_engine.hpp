@@ -62,7 +62,7 @@ struct PdParams {
     int dense_max_iter = 8;     // DenseCholesky: refinement corrections per solve
     int pcg_halo = 1;           // 1: halo-staged PCG kernels (when the tiles could be built); 0: row gathers
     int use_graph = 0;          // replay a captured HIP graph of the step when its launch sequence is fixed
-    int batch_autotune = 1;     // BatchedPCG: time the workgroup sizes of each body-size class at prepare
+    int batch_autotune = 1;     // BatchedPCG: time the workgroup sizes at prepare
     int polar_rotation = 0;     // FP32 local step: 0 TR1690 SVD (as the reference), 1 Newton polar iteration
     double mu_n = 0.5;          // fixed-body response: normal restitution (SolverParams::muN)
     double mu_t = 0.5;          // fixed-body response: friction (SolverParams::muT)
@@ -114,10 +114,6 @@ struct KernelTime {
     double ms = 0.0;
 };
 
-#ifndef SBS_CHUNK_TETS
-#define SBS_CHUNK_TETS 256
-#endif
-constexpr int kChunkTets = SBS_CHUNK_TETS;  // tets per local-step chunk (one workgroup)
 constexpr int kMaxSolveLog = 64;  // per-step log of PCG iterations, by solve index
 constexpr int kCounterInts = 6 + kMaxSolveLog;  // step counters copied to the host
 

@@ -49,7 +49,7 @@ class SolverParams:
     muN: float = 0.5              # fixed-body response: normal restitution
     muT: float = 0.5              # fixed-body response: friction
     use_graph: bool = False       # replay the step as a captured HIP graph (needs a non-null stream)
-    batch_autotune: bool = True   # BatchedPCG: time each size class's workgroup sizes at the first update
+    batch_autotune: bool = True   # BatchedPCG: time the workgroup sizes at the first update
     polar_rotation: bool = False  # FP32 local step: Newton polar iteration instead of the TR1690 SVD
 
     def to_c(self) -> capi.SbsSolverParams:

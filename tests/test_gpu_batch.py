@@ -1,6 +1,6 @@
 """GPU parity of the batched solver (SBS_SOLVER_BATCHED_PCG): every body of a
-concatenated scene advanced with its own Jacobi-PCG + Chebyshev in one
-persistent launch per size class, against the oracle run on each body alone
+concatenated scene advanced with its own Jacobi-PCG + Chebyshev by one
+workgroup per body, against the oracle run on each body alone
 (the reference's step of that body, pdSolver.cu:141-208 with the PCG global
 solve and its per-body stop test, pcgJacobi.cu:134-135) and against one
 PdSolver per body.

@@ -190,7 +190,7 @@ __device__ __forceinline__ void batch_solve_body(const BatchArgs<T>& a, int b, i
     // 32-bit byte offset, a load needs one address register for all places
     const int B = K >= kFixedPlaces ? 1024 : blockDim.x;
     const unsigned tid = threadIdx.x;
-    const int lane = tid & 63, row = lane >> 4, comp = row < 3 ? row : 2;
+    const int lane = tid & 63, row = lane >> 4;
     const bool live = (int)(tid & ~63u) < n;  // the wavefront has rows
     const int places = K > 0 ? K : (n + B - 1) / B;
     const T o[3] = {a.origin[3 * (size_t)b], a.origin[3 * (size_t)b + 1], a.origin[3 * (size_t)b + 2]};

@@ -51,7 +51,9 @@ struct HaloTiles {
     // ascending internal rows; unused positions repeat the workgroup's first row
     std::vector<uint32_t> halo;          // internal rows
     std::vector<uint32_t> halo_vertex;   // the same entries as vertex ids
-    // entry e of the workgroup's thread t at g_eptr[g] + e * rows_per_group + t
+    // `lanes` threads share a row: entry e of the workgroup's row t at
+    // g_eptr[g] + (e / lanes) * rows_per_group * lanes + t * lanes + e % lanes,
+    // and g_width counts a thread's entries
     std::vector<uint16_t> col;           // halo-local column
     std::vector<int64_t> src;            // caller's value index of the entry; -1: padding (value 0)
 };
@@ -66,10 +68,11 @@ struct HaloTiles {
 // ascending vertex id.
 template <class Key, class ValueIndex>
 HaloTiles build_halo_tiles(int nv, const std::vector<int>& rowstart, const std::vector<uint32_t>& cols, Key key,
-                           ValueIndex value_index, int rows_per_group, int halo_stride) {
+                           ValueIndex value_index, int rows_per_group, int halo_stride, int lanes = 1) {
     if (nv <= 0) throw std::invalid_argument("halo tiles: no rows");
     if (rows_per_group <= 0 || rows_per_group % 64 != 0)
         throw std::invalid_argument("halo tiles: rows per group must be a positive multiple of 64");
+    if (lanes <= 0) throw std::invalid_argument("halo tiles: lanes per row must be positive");
     if (halo_stride <= 0 || halo_stride > 65536) throw std::invalid_argument("halo tiles: halo indices are 16-bit");
     if ((int)rowstart.size() != nv + 1 || (size_t)rowstart[nv] != cols.size())
         throw std::invalid_argument("halo tiles: malformed pattern");
@@ -150,7 +153,8 @@ HaloTiles build_halo_tiles(int nv, const std::vector<int>& rowstart, const std::
         }
         std::sort(set.begin(), set.end());
         h.g_halo_n.push_back((int)set.size());
-        h.g_width.push_back(width);
+        const int per_lane = (width + lanes - 1) / lanes, threads = rows_per_group * lanes;
+        h.g_width.push_back(per_lane);
         h.g_eptr.push_back((int)h.col.size());
         h.max_halo = std::max(h.max_halo, (int)set.size());
         h.max_width = std::max(h.max_width, width);
@@ -162,17 +166,17 @@ HaloTiles build_halo_tiles(int nv, const std::vector<int>& rowstart, const std::
         };
         h.g_own0.push_back(local((uint32_t)r));  // rows r..r+n-1 are consecutive in the sorted halo
         const size_t base = h.col.size();
-        if (base + (size_t)width * rows_per_group > (size_t)INT32_MAX)
+        if (base + (size_t)per_lane * threads > (size_t)INT32_MAX)
             throw std::invalid_argument("halo tiles: too many entries");
-        h.col.resize(base + (size_t)width * rows_per_group);
-        h.src.resize(base + (size_t)width * rows_per_group, -1);
+        h.col.resize(base + (size_t)per_lane * threads);
+        h.src.resize(base + (size_t)per_lane * threads, -1);
         for (int t = 0; t < rows_per_group; ++t) {
             const bool row = t < n;
             const uint32_t i = (uint32_t)(row ? r + t : r);
             const uint32_t v = h.row_perm[i];
             const int len = row ? rowstart[v + 1] - rowstart[v] : 0;
-            for (int e = 0; e < width; ++e) {
-                const size_t pos = base + (size_t)e * rows_per_group + t;
+            for (int e = 0; e < per_lane * lanes; ++e) {
+                const size_t pos = base + (size_t)(e / lanes) * threads + (size_t)t * lanes + e % lanes;
                 if (e < len) {
                     h.col[pos] = local(h.row_of[cols[rowstart[v] + e]]);
                     h.src[pos] = (int64_t)value_index(rowstart[v] + e);

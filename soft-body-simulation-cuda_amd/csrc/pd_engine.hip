@@ -129,25 +129,25 @@ template <class T> __device__ __forceinline__ void st_rec(T* __restrict__ base, 
 
 // Sums NQ per-thread values over the block (kTpb threads); thread k < NQ adds
 // quantity k to the block's stripe of `slot` (stripe = block id mod kStripes),
-// so no address sees more than gridDim/kStripes atomics.  Each row of 16
-// lanes reduces with DPP moves and leaves its total in LDS; the 16 row totals
-// are added in row order.  Every thread of the block calls it.
+// so no address sees more than gridDim/kStripes atomics.  A wavefront reduces
+// four quantities at a time (wave_rows4) and leaves its totals in LDS, which
+// are added in a fixed order.  Every thread of the block calls it.
 template <int NQ>
 __device__ __forceinline__ void stripe_add(const double (&vals)[NQ], double* slot) {
-    constexpr int kRows = kTpb / 16;
-    __shared__ double red[NQ][kRows];
-    const int lane = threadIdx.x & 63, rid = threadIdx.x >> 4;
+    constexpr int kGroups = (NQ + 3) / 4, kWaves = kTpb / 64;
+    static_assert(kWaves == 4, "four wavefronts' totals");
+    __shared__ double red[4 * kGroups][kWaves];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    auto q = [&](int k) { return k < NQ ? vals[k] : 0.0; };
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) {
-        const double s = row16_total(vals[k]);
-        if ((lane & 15) == 0) red[k][rid] = s;
+    for (int g = 0; g < kGroups; ++g) {
+        const double s = wave_rows4(q(4 * g), q(4 * g + 1), q(4 * g + 2), q(4 * g + 3));
+        if ((lane & 15) == 0) red[4 * g + (lane >> 4)][wv] = s;
     }
     __syncthreads();
     if (threadIdx.x < NQ) {
-        double s = 0;
-#pragma unroll
-        for (int r = 0; r < kRows; ++r) s += red[threadIdx.x][r];
-        atomicAdd(&slot[(blockIdx.x % kStripes) * kSlotQ + threadIdx.x], s);
+        const double* r = red[threadIdx.x];
+        atomicAdd(&slot[(blockIdx.x % kStripes) * kSlotQ + threadIdx.x], (r[0] + r[1]) + (r[2] + r[3]));
     }
 }
 
@@ -202,7 +202,7 @@ struct CtlBlock {
     int pad0;
     int log[kMaxSolveLog];  // iterations of solve i of the step (-its-1 when stopped early)
     int outer_done;      // local/global loop early exit (direct / PCG modes)
-    int pad1;
+    int never;           // 0: the flag of the modes without an early exit
     double err;          // last computeError value
     PcgState st[2];
 };
@@ -214,6 +214,7 @@ __global__ void ctl_init_kernel(CtlBlock* ctl) {
     for (int i = threadIdx.x; i < kCounterInts; i += blockDim.x) (&ctl->pcg_iters)[i] = 0;
     if (threadIdx.x == 0) {
         ctl->outer_done = 0;
+        ctl->never = 0;
         ctl->err = 1.0;
     }
 }
@@ -428,6 +429,21 @@ template <class T> struct RhsGather {
             ld3(dbcx, v, bx, by, bz);
             bx *= wgt; by *= wgt; bz *= wgt;
         }
+    }
+    // One component of it.
+    __device__ __forceinline__ T component(unsigned v, int k, int e0, int e1) const {
+        const T pin = dbc[v];
+        const T more = more_dbc ? more_dbc[v] : (T)0;
+        T b = c[v] * sn_old[3 * (size_t)v + k];
+        for (int e = e0; e < e1; e += kGatherBatch) {
+#pragma unroll
+            for (int j = 0; j < kGatherBatch; ++j) {
+                const T f = partial[3 * (size_t)min(e + j, e1 - 1) + k];
+                if (e + j < e1) b += f;
+            }
+        }
+        if (pin > (T)0 || more > (T)0) b = dbcx[3 * (size_t)v + k] * (pin > (T)0 ? wdbc : more);
+        return b;
     }
 };
 
@@ -723,13 +739,44 @@ template <int K0> __device__ __forceinline__ double slot_rows3(const double* slo
     return row16_total(slot_pair3<K0>(slot));
 }
 
+// What pcg_state reads: the stop flag, the stripes of launch i-1 and this
+// component's state, requested together and without a branch, so they cost
+// one memory round trip, which a caller can share with its other loads.
+struct PcgReq {
+    double vg, vd, vu, vb, thr, gamma, alpha, beta;
+    int active, done, iters, unconverged;
+};
+template <bool kFirst, class T> __device__ __forceinline__ PcgReq pcg_request(const PcgArgs<T>& a, int i) {
+    const int row = (threadIdx.x & 63) >> 4, c = row < 3 ? row : 2;
+    PcgReq q{};
+    const double* sl = iter_slot(a.slots, i - 1);
+    q.vg = slot_pair3<0>(sl);
+    q.vd = slot_pair3<3>(sl);
+    q.vu = slot_pair3<6>(sl);
+    if constexpr (kFirst) {
+        q.vb = slot_pair3<0>(a.slots + kSlotInit * kSlotSize);
+    } else {
+        const PcgState* prev = &a.ctl->st[(i - 1) & 1];
+        q.thr = prev->thr[c];
+        q.gamma = prev->gamma[c];
+        q.alpha = prev->alpha[c];
+        q.beta = prev->beta[c];
+        q.active = prev->active[c];
+        q.done = prev->done;
+        q.iters = prev->iters;
+        q.unconverged = prev->unconverged;
+    }
+    return q;
+}
+
 // Stop test and scalars of iteration i, identical in every wavefront; block 0
 // records the state for the next launch.  Component c of the three
 // right-hand sides is evaluated by row c of the wavefront (row 3 repeats
 // component 2 and is ignored), so a lane does one component's divisions;
 // alpha and beta are then read from lanes 0, 16 and 32.  Every lane of the
 // wavefront must be active.
-template <class T> __device__ __forceinline__ PcgStep pcg_state(const PcgArgs<T>& a, int i) {
+template <bool kFirst, class T>
+__device__ __forceinline__ PcgStep pcg_state(const PcgArgs<T>& a, int i, const PcgReq& q) {
     const int lane = threadIdx.x & 63, row = lane >> 4;
     const int c = row < 3 ? row : 2;
     PcgStep out;
@@ -737,49 +784,33 @@ template <class T> __device__ __forceinline__ PcgStep pcg_state(const PcgArgs<T>
     const bool writer = blockIdx.x == 0 && threadIdx.x < 64;
     bool act;
     double gamma, thr, alpha = 0.0, beta = 0.0;
-    const PcgState* prev = i > 0 ? &a.ctl->st[(i - 1) & 1] : nullptr;
-    bool carried = false;  // the solve stopped earlier: the state is carried forward
-    int c_iters = 0, c_unconverged = 0;
-    if (i == 0) {
-        const double* sl = iter_slot(a.slots, -1);
-        const double vg = slot_pair3<0>(sl), vd = slot_pair3<3>(sl), vu = slot_pair3<6>(sl);
-        const double vb = slot_pair3<0>(a.slots + kSlotInit * kSlotSize);
-        const double g = row16_total(vg), dl = row16_total(vd), uu = row16_total(vu), dd = row16_total(vb);
-        thr = fmax(a.tol2 * uu, a.floor2 * dd);
+    const PcgState* prev = kFirst ? nullptr : &a.ctl->st[(i - 1) & 1];
+    const bool carried = !kFirst && q.done != 0;  // the solve stopped earlier: the state is carried forward
+    const double g = row16_total(q.vg), dl = row16_total(q.vd), uu = row16_total(q.vu);
+    gamma = g;
+    if constexpr (kFirst) {
+        thr = fmax(a.tol2 * uu, a.floor2 * row16_total(q.vb));
         act = uu > thr;
-        gamma = g;
         alpha = (act && dl != 0.0) ? g / dl : 0.0;
     } else {
-        // The stop flag, the stripes of launch i-1 and this component's state
-        // are requested together and consumed without a branch (the scalars are
-        // formed in every case and selected), so they cost one memory round
-        // trip instead of one each.
-        const double* sl = iter_slot(a.slots, i - 1);
-        const double vg = slot_pair3<0>(sl), vd = slot_pair3<3>(sl), vu = slot_pair3<6>(sl);
-        const double pthr = prev->thr[c], pg = prev->gamma[c], pa = prev->alpha[c], pb = prev->beta[c];
-        const int pact = prev->active[c];
-        carried = prev->done != 0;
-        c_iters = prev->iters;
-        c_unconverged = prev->unconverged;
-        const double g = row16_total(vg), dl = row16_total(vd), uu = row16_total(vu);
-        thr = pthr;
-        act = !carried && pact && uu > thr;
-        const double bt = g / pg;
-        const double den = dl - bt * g / pa;
+        // the scalars are formed in every case and selected
+        thr = q.thr;
+        act = !carried && q.active && uu > thr;
+        const double bt = g / q.gamma;
+        const double den = dl - bt * (g / q.alpha);  // (the two quotients side by side)
         const double al = g / den;
-        const bool ok = act && pg != 0.0;
+        const bool ok = act && q.gamma != 0.0;
         beta = ok ? bt : 0.0;
         alpha = ok && den != 0.0 ? al : 0.0;
         if (carried) {
-            alpha = pa;
-            beta = pb;
+            alpha = q.alpha;
+            beta = q.beta;
         }
-        gamma = g;
     }
     const bool any = __ballot(act && row < 3) != 0ull;
-    out.iters = carried ? c_iters : i;
+    out.iters = carried ? q.iters : i;
     out.done = carried || !any || i >= a.max_iter;
-    out.unconverged = carried ? c_unconverged : (any && i >= a.max_iter);
+    out.unconverged = carried ? q.unconverged : (any && i >= a.max_iter);
     out.alpha[0] = readlane_f64<0>(alpha);
     out.alpha[1] = readlane_f64<16>(alpha);
     out.alpha[2] = readlane_f64<32>(alpha);
@@ -806,6 +837,10 @@ template <class T> __device__ __forceinline__ PcgStep pcg_state(const PcgArgs<T>
         }
     }
     return out;
+}
+template <class T> __device__ __forceinline__ PcgStep pcg_state(const PcgArgs<T>& a, int i) {
+    if (i == 0) return pcg_state<true>(a, i, pcg_request<true>(a, i));
+    return pcg_state<false>(a, i, pcg_request<false>(a, i));
 }
 
 #ifndef SBS_ITER_BATCH
@@ -1218,6 +1253,14 @@ __global__ void __launch_bounds__(kTpb) pcg_init2_halo_kernel(PcgArgs<T> a) {
     stripe_add<9>(vals, iter_slot(a.slots, -1));
 }
 
+// The iteration kernels' arguments, all requested at the launch's start: read
+// where they are first used, each group of them would be a memory round trip
+// of its own in the launch's chain.
+template <class T> __device__ __forceinline__ void iter_args(const PcgArgs<T>& a, int i) {
+    asm volatile("" ::"s"(a.nv), "s"(a.h.grp), "s"(a.h.halo), "s"(a.h.col), "s"(a.h.val), "s"(a.h.x), "s"(a.hrec[0]),
+                 "s"(a.hrec[1]), "s"(a.p), "s"(a.slots), "s"(a.ctl), "s"(a.skip), "s"(a.max_iter), "s"(i));
+}
+
 // One PCG iteration K(i), halo-staged.  The group descriptor and the halo's
 // row indices are requested with the reduction stripes and the state of the
 // previous launch (a launch after the solve stopped carries that state
@@ -1231,7 +1274,9 @@ __global__ void __launch_bounds__(kTpb) pcg_init2_halo_kernel(PcgArgs<T> a) {
 template <class T, bool kFirst>
 __global__ void __launch_bounds__(kTpb) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 1)))
 pcg_iter_halo_kernel(PcgArgs<T> a, int i) {
-    if (a.skip && *a.skip) return;
+    
+    iter_args(a, i);
+    
     __shared__ T lu[3][kHaloStride];
     const unsigned g = xcd_block(blockIdx.x, gridDim.x);
     const int gdl = halo_group_lane(a.h, g);
@@ -1242,7 +1287,9 @@ pcg_iter_halo_kernel(PcgArgs<T> a, int i) {
     uint32_t hidx[kHaloPer];
 #pragma unroll
     for (int k = 0; k < kHaloPer; ++k) hidx[k] = hh[t + k * kTpb];  // in bounds: kHaloStride per workgroup
-    const PcgStep st = pcg_state(a, i);
+    const PcgReq rq = pcg_request<kFirst>(a, i);
+    if (a.skip && *a.skip) return;
+    const PcgStep st = pcg_state<kFirst>(a, i, rq);
     const HaloGroup G = halo_group_bcast(gdl);
     if (st.done) return;
     const bool row = t < G.rows;
@@ -1267,6 +1314,7 @@ pcg_iter_halo_kernel(PcgArgs<T> a, int i) {
     ld3(a.h.x, ir, x0, x1, x2);
     RowBatch<T> b0, b1;
     row_batch(a.h, G.first, G.width, t, 0, b0);
+    __builtin_amdgcn_sched_barrier(0);  // b0 before the staging, b1 after it: in other orders the product waits for b1
     const T al0 = (T)st.alpha[0], al1 = (T)st.alpha[1], al2 = (T)st.alpha[2];
     const T be0 = (T)st.beta[0], be1 = (T)st.beta[1], be2 = (T)st.beta[2];
     // u_{i+1} of the halo rows: S'_i = W'_i + beta S'_{i-1}, R'_{i+1} = R'_i - alpha S'_i
@@ -1283,6 +1331,7 @@ pcg_iter_halo_kernel(PcgArgs<T> a, int i) {
     }
     // the second batch is requested once the staged halo values are out of
     // registers, so its latency overlaps the barrier and the first batch
+    __builtin_amdgcn_sched_barrier(0);
     row_batch(a.h, G.first, G.width, t, kEllBatch, b1);
     if (blockIdx.x == 0) {  // slot of launch i+1: last read by launch i-1, which has finished
         double* z = iter_slot(a.slots, i + 1);
@@ -1315,6 +1364,262 @@ pcg_iter_halo_kernel(PcgArgs<T> a, int i) {
         vals[6] = (double)un0 * un0; vals[7] = (double)un1 * un1; vals[8] = (double)un2 * un2;
     }
     stripe_add<9>(vals, iter_slot(a.slots, i));
+}
+
+// ---------------------------------------------------------------------------
+// The same kernels with four lanes per row (kQuadRows rows per workgroup of
+// kTpb threads), for systems whose 256-row workgroups would not fill the chip
+// (see kQuadMaxRows).  A row's entries are dealt to its lanes, whose partial
+// products one quad sum adds; after it lane c of the row holds component c, so
+// the row's vectors are one scalar per lane and the reductions need three
+// quantities instead of nine, and a
+// thread stages two halo rows instead of three.  A launch is one short round of loads: the halo rows, the row's own vectors and its
+// entries are requested before the scalars of the launch are formed (their
+// addresses depend on neither), so the stripes' and the vectors' latencies
+// overlap.  What bounds a launch is that chain: launch, halo indices, halo
+// rows, product, reduction.
+constexpr int kQuadRows = kTpb / 4;
+// FP64 up to this many rows (measured, a step of 10 PCG solves with 256-row
+// workgroups and with these: 336 rows 1835 -> 1430 us, 2,197 rows 2204 -> 1522,
+// 11,960 rows 2285 -> 1552, 24,389 rows 2395 -> 1928; 50,653 rows 2611 -> 2802:
+// there the chip is full and a smaller workgroup's larger share of halo rows
+// costs more).  FP32 would gain 1.1-1.25x in the same range, but a row's sum in
+// another order moves an FP32 iterate by its rounding, and a step with
+// collision handling turns that into other contact decisions now and then.
+constexpr int kQuadMaxRows = 32768;
+constexpr int kQuadStride = 2 * kTpb;  // halo entries per workgroup
+constexpr int kQuadPer = kQuadStride / kTpb;
+constexpr int kQuadBatch = 4;          // entries per lane loaded together (rows of up to 16 entries: all)
+
+__device__ __forceinline__ double quad_sum(double v) {
+    v += dpp_f64<0xB1>(v);
+    v += dpp_f64<0x4E>(v);
+    return v;
+}
+template <class T> __device__ __forceinline__ T sel3(int c, T x, T y, T z) { return c == 0 ? x : c == 1 ? y : z; }
+
+template <class T> struct QuadBatch {
+    unsigned c[kQuadBatch];
+    T m[kQuadBatch];
+};
+template <class T>
+__device__ __forceinline__ void quad_batch(const HaloView<T>& h, int first, int width, int t, int e0, QuadBatch<T>& b) {
+#pragma unroll
+    for (int j = 0; j < kQuadBatch; ++j) {
+        const unsigned o = (unsigned)min(e0 + j, width - 1) * kTpb + (unsigned)t;
+        b.c[j] = (h.col + first)[o];
+        const T mv = (h.val + first)[o];
+        b.m[j] = e0 + j < width ? mv : (T)0;
+    }
+}
+// The row's product over its four lanes: component c in lane c (lane 3 repeats
+// component 2), the diagonal in all of them.
+template <class T>
+__device__ __forceinline__ T quad_product(const HaloView<T>& h, const HaloGroup& G, int t, const QuadBatch<T>& b0,
+                                          const T (&lu)[3][kQuadStride], unsigned own, T& d) {
+    T y0 = 0, y1 = 0, y2 = 0;
+    d = 0;
+    auto apply = [&](const QuadBatch<T>& b) {
+#pragma unroll
+        for (int j = 0; j < kQuadBatch; ++j) {
+            y0 += b.m[j] * lu[0][b.c[j]];
+            y1 += b.m[j] * lu[1][b.c[j]];
+            y2 += b.m[j] * lu[2][b.c[j]];
+            d += b.c[j] == own ? b.m[j] : (T)0;
+        }
+    };
+    apply(b0);
+    for (int e0 = kQuadBatch; e0 < G.width; e0 += kQuadBatch) {
+        QuadBatch<T> b;
+        quad_batch(h, G.first, G.width, t, e0, b);
+        apply(b);
+    }
+    y0 = quad_sum(y0);
+    y1 = quad_sum(y1);
+    y2 = quad_sum(y2);
+    d = quad_sum(d);
+    return sel3(t & 3, y0, y1, y2);
+}
+// stripe_add of NQ <= 4 quantities per component, component c in the lanes of
+// that place in their quads (lane 3: 0); quantity q of component c is 3 q + c.
+template <int NQ> __device__ __forceinline__ void stripe_add_quads(const double (&vals)[NQ], double* slot) {
+    static_assert(NQ <= 4 && kTpb == 256, "a row of lanes per quantity, four wavefronts");
+    __shared__ double red[4][4][kTpb / 64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double v[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        v[q] = vals[q];
+        v[q] += dpp_f64<0x124>(v[q]);  // row_ror:4
+        v[q] += dpp_f64<0x128>(v[q]);  // row_ror:8
+    }
+    const double s = fold_rows(fold_halves(v[0], v[2]), fold_halves(v[1], v[3]));  // quantity r in row r
+    if ((lane & 15) < 4) red[lane >> 4][lane & 3][wv] = s;
+    __syncthreads();
+    if (threadIdx.x < 3 * NQ) {
+        const double* r = red[threadIdx.x / 3][threadIdx.x % 3];
+        atomicAdd(&slot[(blockIdx.x % kStripes) * kSlotQ + threadIdx.x], (r[0] + r[1]) + (r[2] + r[3]));
+    }
+}
+
+template <class T>
+__global__ void __launch_bounds__(kTpb) pcg_init1_quad_kernel(PcgArgs<T> a) {
+    if (a.skip && *a.skip) return;
+    __shared__ T lx[3][kQuadStride];
+    const unsigned g = xcd_block(blockIdx.x, gridDim.x);
+    const HaloGroup G = halo_group(a.h, g);
+    const int t = threadIdx.x, rl = t >> 2, c = min(t & 3, 2);
+    const bool row = rl < G.rows;
+    const size_t ir = (size_t)G.row0 + (row ? rl : 0);
+    const uint32_t v = a.h.perm[ir];
+    QuadBatch<T> bt;
+    T x0 = 0;
+    if (a.x0) {
+        quad_batch(a.h, G.first, G.width, t, 0, bt);
+        const uint32_t* __restrict__ hv = a.h.halo_v + (size_t)g * kQuadStride;
+#pragma unroll
+        for (int k = 0; k < kQuadPer; ++k) {
+            const int e = t + k * kTpb;
+            T q0, q1, q2;
+            ld3(a.x0, hv[e], q0, q1, q2);
+            lx[0][e] = q0; lx[1][e] = q1; lx[2][e] = q2;
+        }
+        x0 = a.x0[3 * (size_t)v + c];
+    }
+    T b;
+    if (a.gathered && a.h.vent) {
+        const uint2 rv = a.h.vent[ir];
+        b = a.g.component(v, c, (int)rv.x, (int)rv.y);
+    } else if (a.gathered) {
+        b = a.g.component(v, c, a.g.vent_ptr[v], a.g.vent_ptr[v + 1]);
+    } else {
+        b = a.b[3 * (size_t)v + c];
+    }
+    T ax = 0, d;
+    if (a.x0) {
+        __syncthreads();
+        ax = quad_product(a.h, G, t, bt, lx, (unsigned)(G.own0 + rl), d);
+    }
+    double vals[1] = {0};
+    if (row && (t & 3) < 3) {
+        a.h.x[3 * ir + c] = x0;
+        const T di = a.dinv[v];
+        planes(a.hrec[0], a.nv).r[3 * ir + c] = di * (b - ax);
+        const double db = (double)di * b;
+        vals[0] = db * db;
+    }
+    stripe_add_quads<1>(vals, a.slots + kSlotInit * kSlotSize);
+}
+
+template <class T>
+__global__ void __launch_bounds__(kTpb) pcg_init2_quad_kernel(PcgArgs<T> a) {
+    if (a.skip && *a.skip) return;
+    __shared__ T lu[3][kQuadStride];
+    const unsigned g = xcd_block(blockIdx.x, gridDim.x);
+    const HaloGroup G = halo_group(a.h, g);
+    const int t = threadIdx.x, rl = t >> 2, c = min(t & 3, 2);
+    const bool row = rl < G.rows;
+    const size_t ir = (size_t)G.row0 + (row ? rl : 0);
+    const Planes<T> P = planes(a.hrec[0], a.nv);
+    QuadBatch<T> b0;
+    quad_batch(a.h, G.first, G.width, t, 0, b0);
+    const uint32_t* __restrict__ hh = a.h.halo + (size_t)g * kQuadStride;
+#pragma unroll
+    for (int k = 0; k < kQuadPer; ++k) {
+        const int e = t + k * kTpb;
+        T q0, q1, q2;
+        ld3(P.r, hh[e], q0, q1, q2);
+        lu[0][e] = q0; lu[1][e] = q1; lu[2][e] = q2;
+    }
+    const T u = P.r[3 * ir + c];
+    __syncthreads();
+    T d;
+    const T w = quad_product(a.h, G, t, b0, lu, (unsigned)(G.own0 + rl), d);
+    double vals[3] = {0, 0, 0};
+    if (row && (t & 3) < 3) {
+        P.w[3 * ir + c] = ((T)1 / d) * w;
+        vals[0] = (double)d * u * u;
+        vals[1] = (double)w * u;
+        vals[2] = (double)u * u;
+    }
+    stripe_add_quads<3>(vals, iter_slot(a.slots, -1));
+}
+
+template <class T, bool kFirst>
+__global__ void __launch_bounds__(kTpb) pcg_iter_quad_kernel(PcgArgs<T> a, int i) {
+    iter_args(a, i);
+    __shared__ T lu[3][kQuadStride];
+    const unsigned g = xcd_block(blockIdx.x, gridDim.x);
+    const int gdl = halo_group_lane(a.h, g);
+    const int t = threadIdx.x, rl = t >> 2, c = min(t & 3, 2);
+    const Planes<T> Pi = planes(a.hrec[i & 1], a.nv), Po = planes(a.hrec[(i & 1) ^ 1], a.nv);
+    const uint32_t* __restrict__ hh = a.h.halo + (size_t)g * kQuadStride;
+    uint32_t hidx[kQuadPer];
+#pragma unroll
+    for (int k = 0; k < kQuadPer; ++k) hidx[k] = hh[t + k * kTpb];  // in bounds: kQuadStride per workgroup
+    const int skip = *(a.skip ? a.skip : &a.ctl->never);
+    const PcgReq rq = pcg_request<kFirst>(a, i);
+    const HaloGroup G = halo_group_bcast(gdl);
+    const bool row = rl < G.rows;
+    const size_t ir = (size_t)G.row0 + (row ? rl : 0), j = 3 * ir + c;
+    // every slot (the padded list holds valid rows), so the loads go out together
+    T hq[kQuadPer][9];
+#pragma unroll
+    for (int k = 0; k < kQuadPer; ++k) {
+        ld3(Pi.r, hidx[k], hq[k][0], hq[k][1], hq[k][2]);
+        ld3(Pi.w, hidx[k], hq[k][3], hq[k][4], hq[k][5]);
+        if (!kFirst) ld3(Pi.s, hidx[k], hq[k][6], hq[k][7], hq[k][8]);
+    }
+    QuadBatch<T> b0;
+    quad_batch(a.h, G.first, G.width, t, 0, b0);
+    const T r = Pi.r[j], w = Pi.w[j];
+    T so = 0, p = 0;
+    if (!kFirst) {
+        so = Pi.s[j];
+        p = a.p[j];
+    }
+    T x = a.h.x[j];
+    if (__builtin_amdgcn_readfirstlane(skip)) return;
+    const PcgStep st = pcg_state<kFirst>(a, i, rq);
+    if (st.done) return;
+    const T al0 = (T)st.alpha[0], al1 = (T)st.alpha[1], al2 = (T)st.alpha[2];
+    const T be0 = (T)st.beta[0], be1 = (T)st.beta[1], be2 = (T)st.beta[2];
+    // u_{i+1} of the halo rows, as the owner forms it
+#pragma unroll
+    for (int k = 0; k < kQuadPer; ++k) {
+        const int e = t + k * kTpb;
+        T sq0 = hq[k][3], sq1 = hq[k][4], sq2 = hq[k][5];
+        if (!kFirst) {
+            sq0 = fma(be0, hq[k][6], sq0); sq1 = fma(be1, hq[k][7], sq1); sq2 = fma(be2, hq[k][8], sq2);
+        }
+        lu[0][e] = fma(-al0, sq0, hq[k][0]);
+        lu[1][e] = fma(-al1, sq1, hq[k][1]);
+        lu[2][e] = fma(-al2, sq2, hq[k][2]);
+    }
+    if (blockIdx.x == 0) {  // slot of launch i+1: last read by launch i-1, which has finished
+        double* z = iter_slot(a.slots, i + 1);
+        for (int k = threadIdx.x; k < kSlotSize; k += kTpb) z[k] = 0.0;
+    }
+    __syncthreads();
+    T d;
+    const T y = quad_product(a.h, G, t, b0, lu, (unsigned)(G.own0 + rl), d);  // w_{i+1} = A u_{i+1}
+    double vals[3] = {0, 0, 0};
+    if (row && (t & 3) < 3) {
+        const T al = sel3(c, al0, al1, al2), be = sel3(c, be0, be1, be2);
+        const T s = kFirst ? w : fma(be, so, w);
+        p = kFirst ? r : fma(be, p, r);
+        x = fma(al, p, x);
+        const T un = fma(-al, s, r);
+        a.p[j] = p;
+        a.h.x[j] = x;
+        Po.r[j] = un;
+        Po.w[j] = ((T)1 / d) * y;
+        Po.s[j] = s;
+        vals[0] = (double)d * un * un;
+        vals[1] = (double)y * un;
+        vals[2] = (double)un * un;
+    }
+    stripe_add_quads<3>(vals, iter_slot(a.slots, i));
 }
 
 // After K(L-1): the stop test of iteration L and bookkeeping (block 0); the
@@ -1579,12 +1884,17 @@ void PdEngine<T>::build_halo(const std::vector<int>& rowstart, const std::vector
         rs[v + 1] = (int)cols.size();
     }
     HaloTiles h;
-    try {
-        h = build_halo_tiles(nv_, rs, cols, [&](int v) { return vertex_key_[v]; },
-                             [&](int k) { return vidx[k]; }, kTpb, kHaloStride);
-    } catch (const std::invalid_argument&) {
-        return;
-    }
+    auto build = [&](int rows, int stride, int lanes) {
+        try {
+            h = build_halo_tiles(nv_, rs, cols, [&](int v) { return vertex_key_[v]; },
+                                 [&](int k) { return vidx[k]; }, rows, stride, lanes);
+            return true;
+        } catch (const std::invalid_argument&) {
+            return false;
+        }
+    };
+    halo_quad_ = sizeof(T) == 8 && nv_ <= kQuadMaxRows && build(kQuadRows, kQuadStride, 4);
+    if (!halo_quad_ && !build(kTpb, kHaloStride, 1)) return;
     for (int64_t s : h.src)
         if (s > INT32_MAX || s < INT32_MIN) return;
     const int ng = (int)h.g_row0.size();
@@ -1873,7 +2183,13 @@ int PdEngine<T>::launch_pcg(int gathered, const T* b, const T* x0, T* x, bool ch
     const dim3 grid(ceil_div(nv_, kTpb)), block(kTpb), hgrid(halo ? halo_groups_ : 1);
     const int max_iter = params.pcg_max_iter;
     tick(kKPcg, true);
-    if (halo) {
+    const bool quad = halo && halo_quad_;  // FP64
+    if (quad) {
+        if constexpr (sizeof(T) == 8) {
+            hipLaunchKernelGGL(pcg_init1_quad_kernel<T>, hgrid, block, 0, stream_, a);
+            hipLaunchKernelGGL(pcg_init2_quad_kernel<T>, hgrid, block, 0, stream_, a);
+        }
+    } else if (halo) {
         hipLaunchKernelGGL(pcg_init1_halo_kernel<T>, hgrid, block, 0, stream_, a);
         hipLaunchKernelGGL(pcg_init2_halo_kernel<T>, hgrid, block, 0, stream_, a);
     } else {
@@ -1883,7 +2199,12 @@ int PdEngine<T>::launch_pcg(int gathered, const T* b, const T* x0, T* x, bool ch
     // iterations are timed as runs of back-to-back launches (an event pair per
     // launch would add its own gap to every launch)
     auto iteration = [&](int i) {
-        if (halo) {
+        if (quad) {
+            if constexpr (sizeof(T) == 8) {
+                if (i == 0) hipLaunchKernelGGL((pcg_iter_quad_kernel<T, true>), hgrid, block, 0, stream_, a, i);
+                else hipLaunchKernelGGL((pcg_iter_quad_kernel<T, false>), hgrid, block, 0, stream_, a, i);
+            }
+        } else if (halo) {
             if (i == 0) hipLaunchKernelGGL((pcg_iter_halo_kernel<T, true>), hgrid, block, 0, stream_, a, i);
             else hipLaunchKernelGGL((pcg_iter_halo_kernel<T, false>), hgrid, block, 0, stream_, a, i);
         } else {

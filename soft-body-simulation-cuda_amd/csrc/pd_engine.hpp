@@ -255,6 +255,7 @@ private:
     // halo tiles of the halo-staged PCG kernels (rows in Morton order)
     std::vector<uint32_t> vertex_key_;  // Morton code of each vertex's rest position
     int halo_groups_ = 0;
+    bool halo_quad_ = false;  // four lanes per row
     size_t halo_entries_ = 0;
     DevBuf<int> h_grp_, h_src_;
     DevBuf<uint32_t> h_halo_, h_halo_v_, h_perm_;

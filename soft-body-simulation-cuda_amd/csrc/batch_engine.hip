@@ -22,7 +22,7 @@
 namespace sbs {
 namespace {
 
-constexpr int kMaxWaves = 16;  // 1024-thread workgroups at most
+constexpr int kMaxWaves = kRowWaves;  // 1024-thread workgroups at most
 constexpr int kTpbB = 256;     // threads of the per-vertex kernels
 constexpr int kMaxNarrow = 65535 / 3 - 1;  // vertices of a body whose columns fit 16 bits
 constexpr int kFixedPlaces = 6;  // from this many rows per thread on, workgroups have 1,024 threads
@@ -76,26 +76,6 @@ template <class T> __device__ __forceinline__ T cheb(T x, T s, T prev, T omega) 
     return fma(damped - prev, omega, prev);
 }
 
-// Block sums of the three components of NG quantities: component c of
-// quantity g ends in every lane of row c of each wavefront (t[g]).  A
-// wavefront's totals go to LDS by rows (wave_rows4), one read per quantity
-// gives a row all wavefronts' totals of its component, and one 16-lane sum
-// finishes it; with a full wavefront sum and one LDS read per wavefront and
-// value the reductions were most of a small body's iteration.  `live`: the
-// wavefront has rows (uniform; the others' values are 0 and only wait).
-// `buf` alternates between two LDS buffers from one reduction to the next, so
-// one barrier suffices.
-template <int NG> __device__ __forceinline__ void block_rows(const double (&v)[NG][3], double (&t)[NG], double* buf, bool live) {
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6, row = lane >> 4, s = lane & 15;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        const double w = live ? wave_rows4(v[g][0], v[g][1], v[g][2], 0.0) : 0.0;
-        if (s == 0) buf[(4 * g + row) * kMaxWaves + wv] = w;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < NG; ++g) t[g] = row16_total(s < nw ? buf[(4 * g + row) * kMaxWaves + s] : 0.0);
-}
 // A value of lanes 0, 16 and 32 (components 0, 1, 2) as three uniform values.
 __device__ __forceinline__ void from_rows(float v, float (&o)[3]) {
     o[0] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));

@@ -180,4 +180,27 @@ __device__ __forceinline__ double wave_rows4(double q0, double q1, double q2, do
     return row16_total(fold_rows(fold_halves(q0, q2), fold_halves(q1, q3)));
 }
 
+constexpr int kRowWaves = 16;  // wavefronts of a workgroup at most
+// Block sums of the three components of NG quantities: component c of
+// quantity g ends in every lane of row c of each wavefront (t[g]).  A
+// wavefront's totals go to LDS by rows (wave_rows4), one read per quantity
+// gives a row all wavefronts' totals of its component, and one 16-lane sum
+// finishes it; with a full wavefront sum and one LDS read per wavefront and
+// value the reductions were most of a small body's iteration.  `live`: the
+// wavefront has rows (uniform; the others' values are 0 and only wait).
+// `buf` alternates between two LDS buffers from one reduction to the next, so
+// one barrier suffices.
+template <int NG>
+__device__ __forceinline__ void block_rows(const double (&v)[NG][3], double (&t)[NG], double* buf, bool live) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6, row = lane >> 4, s = lane & 15;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const double w = live ? wave_rows4(v[g][0], v[g][1], v[g][2], 0.0) : 0.0;
+        if (s == 0) buf[(4 * g + row) * kRowWaves + wv] = w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < NG; ++g) t[g] = row16_total(s < nw ? buf[(4 * g + row) * kRowWaves + s] : 0.0);
+}
+
 }  // namespace sbs

@@ -1647,6 +1647,188 @@ __global__ void __launch_bounds__(kTpb) pcg_finish_halo_kernel(PcgArgs<T> a, int
     }
 }
 
+// ---------------------------------------------------------------------------
+// A whole solve in one workgroup, for systems of up to kSmallRows rows: the
+// right-hand side, the iterations above with their stop test and what follows
+// the solve (the Chebyshev recurrence, or computeError and the early exit of
+// the local/global loop) in one launch.  A thread holds a row: its vectors and
+// its first kSmallWidth entries stay in registers, u lives in LDS, and the
+// reductions are block sums (block_rows), so an iteration costs two barriers
+// instead of a launch.  Each row's products are added in the order of the
+// halo kernels.  What bounds it is one CU's chain per iteration: LDS reads of
+// the product, the FP64 sums and three divisions.  A step of 10 solves, one
+// launch per iteration and this kernel: FP32, without and with Chebyshev, 27
+// rows 643 -> 191 and 654 -> 239 us, 336 rows 806 -> 268 and 923 -> 374, 1,000
+// rows 813 -> 398 and 941 -> 563; FP64 336 rows 1208 -> 392 and 1747 -> 607,
+// 1,000 rows 1329 -> 685 and 1940 -> 1104.  The limit is a thread per row in
+// one workgroup (two rows' entries per thread would not stay in registers).
+constexpr int kSmallRows = 1024;
+constexpr int kSmallWidth = 16;  // off-diagonal entries of a row held in registers
+
+template <class T> struct SmallEnd {
+    int cheb, outer;  // Chebyshev recurrence / computeError into sn, prev; neither: x
+    double tol;       // of the outer loop
+};
+
+template <class T>
+__global__ void __launch_bounds__(kSmallRows) pcg_small_kernel(PcgArgs<T> a, SmallEnd<T> end) {
+    if (a.skip && *a.skip) return;
+    __shared__ T lu[3][kSmallRows];
+    __shared__ double red[2][16 * kRowWaves];
+    const int t = threadIdx.x, lrow = (t & 63) >> 4;
+    const bool row = t < a.nv, live = (t & ~63) < a.nv;
+    const unsigned v = row ? t : 0;
+    const int slice = __builtin_amdgcn_readfirstlane(t / kSlice);
+    const int width = live ? __builtin_amdgcn_readfirstlane(a.slice_w[slice]) : 0;
+    const size_t base = (live ? (size_t)a.slice_ptr[slice] : 0) + (t & 63);
+    static_assert(kSlice == 64, "a wavefront per slice");
+    T m[kSmallWidth];
+    unsigned col[kSmallWidth];
+#pragma unroll
+    for (int e = 0; e < kSmallWidth; ++e) {
+        const bool in = e < width && row;
+        const size_t at = base + (size_t)min(e, max(width - 1, 0)) * kSlice;
+        m[e] = in ? a.eval[at] : (T)0;
+        col[e] = in ? a.ecol[at] : v;
+    }
+    const T d = row ? a.diagA[v] : (T)1, dinv = row ? a.dinv[v] : (T)0;
+    // y = A lu, in the order of the row's entries (diagonal first)
+    auto product = [&](T (&y)[3]) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) y[c] = d * lu[c][v];
+#pragma unroll
+        for (int e0 = 0; e0 < kSmallWidth; e0 += 4)
+            if (e0 < width)
+#pragma unroll
+                for (int e = e0; e < e0 + 4; ++e)
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) y[c] += m[e] * lu[c][col[e]];
+        if (row)
+            for (int e = kSmallWidth; e < width; ++e) {
+                const T me = a.eval[base + (size_t)e * kSlice];
+                const unsigned ce = a.ecol[base + (size_t)e * kSlice];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) y[c] += me * lu[c][ce];
+            }
+    };
+    T x[3] = {0, 0, 0}, r[3] = {0, 0, 0}, w[3], p[3] = {0, 0, 0}, s[3] = {0, 0, 0};
+    double acc[4][3] = {};  // r.u, w.u, u.u, (D^-1 b)^2
+    {
+        T ax[3] = {0, 0, 0};
+        if (a.x0) {
+            if (row) {
+                ld3(a.x0, v, x[0], x[1], x[2]);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) lu[c][t] = x[c];
+            }
+            __syncthreads();
+            product(ax);
+            __syncthreads();
+        }
+        if (row) {
+            T b[3];
+            if (a.gathered) a.g.at(v, b[0], b[1], b[2]);
+            else ld3(a.b, v, b[0], b[1], b[2]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                r[c] = dinv * (b[c] - ax[c]);
+                lu[c][t] = r[c];
+                const double db = (double)dinv * b[c];
+                acc[3][c] = db * db;
+            }
+        }
+    }
+    __syncthreads();
+    const T di = (T)1 / d;
+    product(w);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        if (row) {
+            acc[0][c] = (double)d * r[c] * r[c];
+            acc[1][c] = (double)w[c] * r[c];
+            acc[2][c] = (double)r[c] * r[c];
+        }
+        w[c] = di * w[c];
+    }
+    // component c's scalars in every lane of row c, the same in every wavefront
+    double t0[4];
+    block_rows<4>(acc, t0, red[0], live);
+    int rb = 1;
+    double gamma = t0[0];
+    const double thr = fmax(a.tol2 * t0[2], a.floor2 * t0[3]);
+    bool act = t0[2] > thr && lrow < 3;
+    double alpha = act && t0[1] != 0.0 ? gamma / t0[1] : 0.0, beta = 0.0;
+    int it = 0;
+    for (; it < a.max_iter && __ballot(act) != 0ull; ++it) {
+        const T al[3] = {(T)readlane_f64<0>(alpha), (T)readlane_f64<16>(alpha), (T)readlane_f64<32>(alpha)};
+        const T be[3] = {(T)readlane_f64<0>(beta), (T)readlane_f64<16>(beta), (T)readlane_f64<32>(beta)};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            p[c] = fma(be[c], p[c], r[c]);
+            s[c] = fma(be[c], s[c], w[c]);
+            x[c] = fma(al[c], p[c], x[c]);
+            r[c] = fma(-al[c], s[c], r[c]);
+            if (row) lu[c][t] = r[c];  // the last product's reads ended before the reduction's barrier
+        }
+        __syncthreads();
+        product(w);
+        double q[3][3] = {};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if (row) {
+                q[0][c] = (double)d * r[c] * r[c];
+                q[1][c] = (double)w[c] * r[c];
+                q[2][c] = (double)r[c] * r[c];
+            }
+            w[c] = di * w[c];
+        }
+        double tq[3];
+        block_rows<3>(q, tq, red[rb], live);
+        rb ^= 1;
+        const double bt = tq[0] / gamma, den = tq[1] - bt * (tq[0] / alpha), an = tq[0] / den;
+        act = act && tq[2] > thr;
+        const bool ok = act && gamma != 0.0;
+        beta = ok ? bt : 0.0;
+        alpha = ok && den != 0.0 ? an : 0.0;
+        gamma = tq[0];
+    }
+    const bool cut = __ballot(act) != 0ull;
+    if (t == 0) pcg_log_solve(a.ctl, it, 1, cut, it);
+    double err[1][3] = {};
+    if (row) {
+        if (end.cheb) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const size_t j = 3 * (size_t)v + c;
+                const T sn = a.sn[j], nx = cheb_update(x[c], sn, a.prev[j], a.omega);
+                a.prev[j] = sn;
+                a.sn[j] = nx;
+            }
+        } else if (end.outer) {
+            T o[3];
+            ld3(a.prev, v, o[0], o[1], o[2]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const T dx = o[c] - x[c];
+                err[0][c] = (double)(dx * dx);
+            }
+            st3(a.sn, v, x[0], x[1], x[2]);
+            st3(a.prev, v, x[0], x[1], x[2]);
+        } else {
+            st3(a.x, v, x[0], x[1], x[2]);
+        }
+    }
+    if (end.outer) {  // as outer_error_kernel and outer_decide_kernel
+        double te[1];
+        block_rows<1>(err, te, red[rb], live);
+        const double e = (readlane_f64<0>(te[0]) + readlane_f64<16>(te[0]) + readlane_f64<32>(te[0])) / (3.0 * a.nv);
+        if (t == 0) {
+            a.ctl->err = e;
+            a.ctl->outer_done = !(sqrt(e) >= end.tol);
+        }
+    }
+}
+
 // Entry values of the halo tiles from the assembled matrix: src >= 0 an
 // off-diagonal sliced-ELL position, -1 padding, <= -2 the diagonal of row -2-src.
 template <class T>
@@ -2183,6 +2365,16 @@ int PdEngine<T>::launch_pcg(int gathered, const T* b, const T* x0, T* x, bool ch
     const dim3 grid(ceil_div(nv_, kTpb)), block(kTpb), hgrid(halo ? halo_groups_ : 1);
     const int max_iter = params.pcg_max_iter;
     tick(kKPcg, true);
+    if (small_pcg(params)) {
+        SBS_REQUIRE(!defer_finish, "PCG: a solve in one workgroup is finished in it");
+        tick(kKPcgIter, true);
+        hipLaunchKernelGGL(pcg_small_kernel<T>, dim3(1), dim3(ceil_div(nv_, 64) * 64), 0, stream_, a,
+                           SmallEnd<T>{(int)cheb, (int)(skip != nullptr), params.tol});
+        tick(kKPcgIter, false, 1);
+        tick(kKPcg, false);
+        SBS_HIP(hipGetLastError());
+        return 0;
+    }
     const bool quad = halo && halo_quad_;  // FP64
     if (quad) {
         if constexpr (sizeof(T) == 8) {
@@ -2239,6 +2431,10 @@ int PdEngine<T>::launch_pcg(int gathered, const T* b, const T* x0, T* x, bool ch
     tick(kKPcg, false);
     SBS_HIP(hipGetLastError());
     return L;
+}
+
+template <class T> bool PdEngine<T>::small_pcg(const PdParams& params) const {
+    return params.pcg_halo && nv_ <= kSmallRows;
 }
 
 // Iterations of headroom over the last observed count of a solve.
@@ -2437,7 +2633,8 @@ template <class T> void PdEngine<T>::enqueue_step(PdData<T>& data, const PdParam
     // and the Chebyshev recurrence) runs inside the local step of iteration
     // i+1, which forms q from solve i's iterate; sn/prev then alternate
     // between two buffers.  The last solve keeps its finish launch.
-    const bool fold = pcg && cheb && params.pcg_halo && halo_groups_ > 0 && chunk_rows_.get() != nullptr;
+    const bool fold = pcg && cheb && params.pcg_halo && halo_groups_ > 0 && chunk_rows_.get() != nullptr &&
+                      !small_pcg(params);
     hipLaunchKernelGGL(ctl_init_kernel, dim3(1), dim3(64), 0, stream_, ctl);
     if (solver_ == GlobalSolver::BatchedPCG) {
         // every body on its own, see batch_engine.hpp
@@ -2502,7 +2699,7 @@ template <class T> void PdEngine<T>::enqueue_step(PdData<T>& data, const PdParam
                 const int L = launch_pcg(1, nullptr, sn_cur, next_.get(), cheb, omega, params, skip, i,
                                          !params.pcg_adaptive, sn_cur, prev_cur, defer);
                 if (defer) open_L = L;
-                if (!cheb) {
+                if (!cheb && !small_pcg(params)) {
                     hipLaunchKernelGGL(outer_error_kernel<T>, dim3(vb), dim3(kTpb), 0, stream_, nv_,
                                        (const T*)next_.get(), sn_.get(), prev_.get(), slots_.get(), skip);
                     hipLaunchKernelGGL(outer_decide_kernel, dim3(1), dim3(64), 0, stream_, (const double*)slots_.get(),

@@ -191,6 +191,7 @@ private:
     size_t local_lds_bytes() const;
     // sn/prev: the Chebyshev state the finish updates (null: sn_, prev_);
     // defer_finish: launch no finish (the next local step does it)
+    bool small_pcg(const PdParams& params) const;  // a solve runs in one workgroup
     int launch_pcg(int gathered, const T* b, const T* x0, T* x, bool cheb, T omega, const PdParams& params,
                    const int* skip, int solve_index, bool exact, T* sn = nullptr, T* prev = nullptr,
                    bool defer_finish = false);

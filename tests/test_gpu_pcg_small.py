@@ -1,0 +1,68 @@
+"""A PCG solve in one workgroup (systems of up to 1,024 rows) against the
+row-gather kernels: one wavefront, a part of one, the largest size of the rule
+and one past it, rows of exactly the entries held in registers and of more,
+the Chebyshev form, the early exit of the local/global loop and solves cut by
+the iteration limit.
+
+Bounds: in FP64 both sides stop at ||D^-1 r|| <= 1e-13 of its start (1e-10
+relative, the bar of the PCG tests).  In FP32 both stop by the same test and
+differ in the sums' order, so the distance to the FP64 solution may be at most
+twice the row-gather kernels' plus 1e-6 (8 units of FP32 rounding of the
+positions that are handed back)."""
+import pytest
+
+from conftest import rel_err
+from test_gpu_pcg_quads import body, fan
+from sbs_amd.pd import PdSolver, SolverData, SolverParams, SolverType
+
+pytestmark = pytest.mark.gpu
+
+
+def solve(s, precision, **kw):
+    p = SolverParams(**dict(dict(numIterations=6, dt=1.0 / 60.0, gravity=9.8, tol=0.0, rho=0.9992, pcg_max_iter=400,
+                                 pcg_tol=1e-6 if precision == 32 else 1e-13,
+                                 pcg_floor=1e-8 if precision == 32 else 0.0), **kw))
+    data = SolverData(s, precision)
+    pd = PdSolver(128, data)
+    pd.SetGlobalSolver(SolverType.PCG)
+    try:
+        for _ in range(3):
+            pd.Update(data, p)
+        pd.synchronize()
+        return data.get("X"), pd.stats()
+    finally:
+        pd.close()
+        data.free()
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("mode", ["chebyshev", "all iterations", "early exit"])
+@pytest.mark.parametrize("size", [(1, 1, 1), (3, 3, 3), (1, 4, 12), (7, 7, 15), (4, 4, 40), "fan 15", "fan 16", "fan 60"])
+def test_matches_the_row_gather_kernels(gpu, size, mode, precision):
+    s = fan(int(size.split()[1])) if isinstance(size, str) else body(*size)
+    kw = dict(pcg_chebyshev=mode == "chebyshev", tol=1e-4 if mode == "early exit" else 0.0)
+    x, st = solve(s, precision, **kw)
+    ref, sr = solve(s, 64, pcg_halo=0, **kw)
+    assert st.pcg_cap_hits == 0 and st.pcg_iterations_total > 0
+    if mode != "early exit":
+        assert st.pcg_solves_total == 18
+    if precision == 64:
+        assert st.pcg_solves_total == sr.pcg_solves_total
+        assert rel_err(x, ref) < 1e-10, rel_err(x, ref)
+    else:
+        gather, sg = solve(s, 32, pcg_halo=0, **kw)
+        assert st.pcg_solves_total == sg.pcg_solves_total
+        assert rel_err(x, ref) <= 2 * rel_err(gather, ref) + 1e-6, (rel_err(x, ref), rel_err(gather, ref))
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_iteration_limit(gpu, precision):
+    """Solves cut at 3 iterations: the same iterates as the row-gather kernels
+    (three iterations' rounding apart) and every solve counted as cut."""
+    s = body(4, 5, 6)
+    kw = dict(pcg_chebyshev=True, pcg_max_iter=3, pcg_adaptive=False)
+    x, st = solve(s, precision, **kw)
+    ref, sr = solve(s, precision, pcg_halo=0, **kw)
+    assert st.pcg_iterations_total == sr.pcg_iterations_total == 3 * 18
+    assert st.pcg_cap_hits == sr.pcg_cap_hits == 18
+    assert rel_err(x, ref) < (1e-5 if precision == 32 else 1e-12)

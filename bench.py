@@ -605,7 +605,7 @@ def main():
         run_solver_workload(args, SolverType.Jacobi, 64, "jacobi_chebyshev", "Jacobi + Chebyshev global step")
         return
     if args.workload in ("direct14", "direct27"):
-        # band factor (host) + ring-buffer band triangular solves (GPU)
+        # band factor (host), then its explicit inverse and the product with it (GPU)
         run_solver_workload(args, SolverType.CuSolverCholesky, int(args.workload[6:]), "direct_solve",
                             "band Cholesky global step")
         return

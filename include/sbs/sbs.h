@@ -401,7 +401,7 @@ typedef struct SbsIpcParams {
     double dhat;          /* barrier distance (queries kept while d^2 <= dhat)  */
     double tol;           /* Newton stop: |p|_inf / dt < tol                    */
     int max_iterations;   /* Newton iterations per step (failure beyond)        */
-    double lin_tol;       /* PCG: |r| <= lin_tol |g|                     */
+    double lin_tol;       /* PCG: |r| <= lin_tol |g|                            */
     int lin_max_iter;
 } SbsIpcParams;
 

@@ -15,8 +15,10 @@
 // Layout: per-tet Dm^-1 (row-major) and V0; per Newton iteration the 12x12
 // Hessian of every tet and of every active query (row-major, the query's or
 // tet's 4 vertices x 3 coordinates) and the gradient; the linear system
-// H p = g is solved by Jacobi-PCG applied element by element (no assembled
-// matrix), with fixed degrees of freedom as rows and columns of the identity.
+// H p = g is solved by PCG over assembled 3x3-block rows (the tets' and the
+// active queries'), preconditioned by the diagonal and by inverted blocks of
+// the vertices in contact, with fixed degrees of freedom as rows and columns of
+// the identity.
 #pragma once
 
 #include <cstdint>

@@ -163,6 +163,16 @@ int sbs_pd_set_perf(SbsPd* pd, int on);
 int sbs_pd_perf_count(SbsPd* pd, int* count);
 int sbs_pd_perf_entry(SbsPd* pd, int index, const char** name, double* ms);
 int sbs_pd_set_stream(SbsPd* pd, void* hip_stream);
+/* The Cholesky solver types hold either the band factor (triangular solves) or,
+ * where a product with it is the faster solve, the explicit inverse: the square
+ * of each body's vertices in values, kept until the handle goes (1.9 GB for
+ * 27^3 hexes in FP32).  `bytes` bounds that memory (default 4 GiB; never more
+ * than a quarter of what is free when the system is factored); 0 keeps the
+ * triangular solves.  A changed bound takes effect with the next update, which
+ * factors again.  sbs_pd_direct_info reports what the last factorisation
+ * took: bodies, half bandwidth, bytes of the inverse (0: triangular solves). */
+int sbs_pd_set_direct_memory(SbsPd* pd, long long bytes);
+int sbs_pd_direct_info(SbsPd* pd, int* systems, int* bandwidth, long long* inverse_bytes);
 /* Waits for queued work of the handle and returns its statistics. */
 int sbs_pd_stats(SbsPd* pd, SbsPdStats* out);
 

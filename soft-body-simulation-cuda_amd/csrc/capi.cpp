@@ -365,6 +365,17 @@ int sbs_pd_dense_info(SbsPd* pd, int* bodies, int* max_body, long long* inverse_
         [&] { with_engine(pd, [&](auto& e) { e.dense_info(bodies, max_body, inverse_bytes, last_iterations, last_ratio); }); });
 }
 
+int sbs_pd_set_direct_memory(SbsPd* pd, long long bytes) {
+    return guarded([&] {
+        SBS_REQUIRE(bytes >= 0, "sbs_pd_set_direct_memory: negative size");
+        with_engine(pd, [&](auto& e) { e.set_direct_memory((size_t)bytes); });
+    });
+}
+
+int sbs_pd_direct_info(SbsPd* pd, int* systems, int* bandwidth, long long* inverse_bytes) {
+    return guarded([&] { with_engine(pd, [&](auto& e) { e.direct_info(systems, bandwidth, inverse_bytes); }); });
+}
+
 int sbs_pd_batch_info(SbsPd* pd, int* num_bodies, int* num_classes) {
     return guarded([&] {
         with_engine(pd, [&](auto& e) {

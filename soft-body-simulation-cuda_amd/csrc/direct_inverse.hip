@@ -13,7 +13,6 @@ constexpr int kThreads = 256;
 constexpr int kStripCols = 64;    // columns of one inversion workgroup (one wavefront)
 constexpr int kPadTo = 4;         // rows are padded to whole 4-value loads
 constexpr size_t kScratchBytes = (size_t)4 << 30;   // FP64 columns in flight while inverting
-constexpr size_t kMaxInverseBytes = (size_t)4 << 30;
 
 // One 64-column strip of a system's inverse, one column per lane.  Rows go in
 // blocks of kBlkRows: each wavefront takes every kStripWaves-th of the rows
@@ -224,8 +223,7 @@ int padded(int n) { return (n + kPadTo - 1) / kPadTo * kPadTo; }
 // solve walks the largest system's 64-row blocks twice, about 2.2 us a block
 // and sweep (12 blocks: 77 us, 53 blocks: 227 us), with about 512 workgroups
 // (three per system) side by side.
-template <class T> bool InverseOperator<T>::suits(int bw, const std::vector<int>& sys) {
-    (void)bw;
+template <class T> bool InverseOperator<T>::suits(const std::vector<int>& sys, size_t most_bytes) {
     const int nsys = (int)sys.size() - 1;
     size_t bytes = 0;
     int longest = 0;
@@ -234,7 +232,11 @@ template <class T> bool InverseOperator<T>::suits(int bw, const std::vector<int>
         bytes += (size_t)n * padded(n) * sizeof(T);
         longest = std::max(longest, n);
     }
-    if (bytes > kMaxInverseBytes) return false;
+    // never more than a quarter of what is free: the inverse of a large body is
+    // 27 to 50 times its factor, and the caller's arrays come first
+    size_t free_bytes = 0, total_bytes = 0;
+    if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) return false;
+    if (bytes > std::min(most_bytes, free_bytes / 4)) return false;
     const double product_us = 5.0 + (double)bytes / 4.5e6;
     const double band_us = 2.2 * 2 * ceil_div((size_t)longest, 64) * ceil_div(3 * (size_t)nsys, 512);
     return product_us < band_us;

@@ -30,10 +30,13 @@ template <class T> struct OuterStep {
 template <class T> class InverseOperator {
 public:
     // Whether the product with the inverse of this factor's systems (row
-    // ranges sys[s] .. sys[s+1]) is the faster solve; see the rule's comment.
-    static bool suits(int bw, const std::vector<int>& sys);
+    // ranges sys[s] .. sys[s+1]) is the faster solve and the inverse takes no
+    // more than most_bytes nor a quarter of the free memory; see the rule's
+    // comment.
+    static bool suits(const std::vector<int>& sys, size_t most_bytes);
     void setup(const BandFactor& f, const std::vector<int>& sys, hipStream_t stream);
     bool ready() const { return n_ > 0; }
+    size_t bytes() const { return inv_.bytes(); }
     // The right-hand side's place: component c of vertex v at
     // rhs()[c * stride() + pos()[v]] (padding between systems stays 0).
     T* rhs() const { return rhs_.get(); }

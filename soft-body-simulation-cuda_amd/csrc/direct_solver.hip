@@ -209,7 +209,7 @@ template <class T> int BandCholesky<T>::max_bandwidth() {
 
 template <class T>
 void BandCholesky<T>::factor(int n, const std::vector<int>& rowptr, const std::vector<int>& col,
-                             const std::vector<T>& val, hipStream_t stream) {
+                             const std::vector<T>& val, hipStream_t stream, size_t inverse_bytes) {
     SBS_REQUIRE(n > 0, "BandCholesky: empty matrix");
     const int bw_est = band_width_estimate(n, rowptr, col);
     if (bw_est > max_bandwidth())
@@ -234,7 +234,7 @@ void BandCholesky<T>::factor(int n, const std::vector<int>& rowptr, const std::v
     bw_ = bw;
     nsys_ = (int)sys.size() - 1;
     inverse_ = InverseOperator<T>();
-    if (InverseOperator<T>::suits(bw, sys)) {
+    if (InverseOperator<T>::suits(sys, inverse_bytes)) {
         try {
             inverse_.setup(f, sys, stream);
             return;

@@ -32,9 +32,10 @@ namespace sbs {
 
 template <class T> class BandCholesky {
 public:
-    // CSR of the full symmetric matrix (both triangles, sorted columns).
+    // CSR of the full symmetric matrix (both triangles, sorted columns).  The
+    // explicit inverse may take up to inverse_bytes (0: triangular solves).
     void factor(int n, const std::vector<int>& rowptr, const std::vector<int>& col, const std::vector<T>& val,
-                hipStream_t stream);
+                hipStream_t stream, size_t inverse_bytes);
     // x = A^-1 b for 3 interleaved right-hand sides; kernels return early
     // when *skip != 0 (device flag, may be null).
     void solve(const T* b, T* x, hipStream_t stream, const int* skip) const;
@@ -42,6 +43,7 @@ public:
     // solved (null otherwise): the caller may write the right-hand side in its
     // place and take the outer loop's end with it.
     const InverseOperator<T>* inverse() const { return inverse_.ready() ? &inverse_ : nullptr; }
+    size_t inverse_bytes() const { return inverse_.ready() ? inverse_.bytes() : 0; }
     int n() const { return n_; }
     int bandwidth() const { return bw_; }
     int systems() const { return nsys_; }

@@ -2212,7 +2212,8 @@ template <class T> void PdEngine<T>::direct_factor(const PdParams& params) {
         dense_prec_ = params.dense_precision;
     } else {
         direct_ = std::make_unique<BandCholesky<T>>();
-        direct_->factor(nv_, ex.rowptr, ex.col, ex.val, stream_);
+        direct_->factor(nv_, ex.rowptr, ex.col, ex.val, stream_, direct_memory_);
+        direct_stale_ = false;
     }
 }
 
@@ -2263,6 +2264,18 @@ template <class T> void PdEngine<T>::direct_solve(const T* b, T* x, const PdPara
     }
     SBS_REQUIRE(direct_ != nullptr, "direct solve requested before factorisation");
     direct_->solve(b, x, stream_, skip);
+}
+
+template <class T> void PdEngine<T>::set_direct_memory(size_t bytes) {
+    direct_stale_ = direct_stale_ || bytes != direct_memory_;
+    direct_memory_ = bytes;
+}
+
+template <class T> void PdEngine<T>::direct_info(int* systems, int* bandwidth, long long* inverse_bytes) {
+    SBS_REQUIRE(direct_ != nullptr, "direct solver not in use (set a Cholesky global solver and run an update)");
+    if (systems) *systems = direct_->systems();
+    if (bandwidth) *bandwidth = direct_->bandwidth();
+    if (inverse_bytes) *inverse_bytes = (long long)direct_->inverse_bytes();
 }
 
 template <class T> void PdEngine<T>::dense_info(int* bodies, int* max_body, long long* bytes, int* iterations,
@@ -2493,7 +2506,7 @@ template <class T> void PdEngine<T>::update(PdData<T>& data, const PdParams& par
     SBS_REQUIRE(params.pcg_max_iter >= 1, "PdSolver: pcg_max_iter must be >= 1");
     const bool direct = is_direct();
     if (direct && ((solver_ == GlobalSolver::DenseCholesky) ? (!dense_ || dense_prec_ != params.dense_precision)
-                                                             : !direct_)) {
+                                                             : (!direct_ || direct_stale_))) {
         direct_.reset();
         dense_.reset();
         direct_factor(params);

@@ -125,6 +125,9 @@ public:
     void set_global_solver(GlobalSolver s) { solver_ = s; }
     GlobalSolver global_solver() const { return solver_; }
     void set_perf(bool on) { perf_ = on; }
+    // Device memory that the direct modes may keep for the explicit inverse.
+    void set_direct_memory(size_t bytes);
+    void direct_info(int* systems, int* bandwidth, long long* inverse_bytes);
     void set_stream(hipStream_t s) {
         if (s != stream_) drop_graph();
         stream_ = s;
@@ -277,6 +280,8 @@ private:
     long long step_caps_[2] = {-1, -1};  // cap epoch of each counter slot
     // direct solver (band Cholesky factor, GPU triangular solves) for small bodies
     std::unique_ptr<BandCholesky<T>> direct_;
+    size_t direct_memory_ = (size_t)4 << 30;  // for its explicit inverse
+    bool direct_stale_ = false;               // factored with another bound
     std::unique_ptr<DenseRefinedSolver<T>> dense_;   // per-body dense inverses (DenseCholesky)
     std::unique_ptr<BatchEngine<T>> batch_;          // per-body persistent solve (BatchedPCG)
     void build_batch(const PdParams& params);

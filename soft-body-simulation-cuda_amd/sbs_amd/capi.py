@@ -109,6 +109,8 @@ SIGNATURES = {
     "sbs_pd_perf_count": (_I, [_VP, ctypes.POINTER(_I)]),
     "sbs_pd_perf_entry": (_I, [_VP, _I, ctypes.POINTER(_CP), ctypes.POINTER(_D)]),
     "sbs_pd_set_stream": (_I, [_VP, _VP]),
+    "sbs_pd_set_direct_memory": (_I, [_VP, ctypes.c_longlong]),
+    "sbs_pd_direct_info": (_I, [_VP, ctypes.POINTER(_I), ctypes.POINTER(_I), ctypes.POINTER(ctypes.c_longlong)]),
     "sbs_pd_stats": (_I, [_VP, ctypes.POINTER(SbsPdStats)]),
     "sbs_pd_set_kernel_timing": (_I, [_VP, ctypes.c_uint]),
     "sbs_pd_kernel_time": (_I, [_VP, _I, ctypes.POINTER(_CP), ctypes.POINTER(_I), ctypes.POINTER(_D)]),

@@ -176,6 +176,16 @@ class PdSolver:
     def SetGlobalSolver(self, val: SolverType) -> None:
         capi.check(self._L.sbs_pd_set_global_solver(self.h, int(val)))
 
+    def set_direct_memory(self, nbytes: int) -> None:
+        """Bound of the device memory that the Cholesky solvers keep for an explicit inverse (0: none)."""
+        capi.check(self._L.sbs_pd_set_direct_memory(self.h, int(nbytes)))
+
+    def direct_info(self) -> dict:
+        """Bodies, half bandwidth and bytes of the explicit inverse (0: triangular solves) of the last factorisation."""
+        s, b, n = ctypes.c_int(), ctypes.c_int(), ctypes.c_longlong()
+        capi.check(self._L.sbs_pd_direct_info(self.h, ctypes.byref(s), ctypes.byref(b), ctypes.byref(n)))
+        return dict(systems=s.value, bandwidth=b.value, inverse_bytes=n.value)
+
     def Update(self, solverData: SolverData, solverParams: SolverParams) -> None:
         p = solverParams.to_c()
         capi.check(self._L.sbs_pd_update(self.h, ctypes.byref(solverData.c), ctypes.byref(p)))

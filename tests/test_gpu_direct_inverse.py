@@ -47,3 +47,34 @@ def test_solve_against_dense(name, precision):
     assert np.all(np.abs(x - ref) <= bound)
     pd.close()
     data.free()
+
+
+def test_memory_bound(gpu):
+    """The bound on the inverse's memory: below the inverse's size the factor is
+    solved by triangular solves, a changed bound takes effect with the next
+    update, and both forms give the same step to FP64 rounding (the matrix's
+    condition number, about 1e6 with the pins, times 1e-16, over 2 iterations)."""
+    scene = mesh.make_scene([dict(nx=7, ny=8, nz=6, seed=3, pin_top=True)])
+    n = scene.nv
+    size = 8 * n * ((n + 3) // 4 * 4)
+    data = SolverData(scene, 64)
+    pd = PdSolver(128, data)
+    pd.SetGlobalSolver(SolverType.CuSolverCholesky)
+    p = SolverParams(numIterations=2, dt=1.0 / 60.0, tol=0.0)
+    rest = {k: data.get(k) for k in ("X", "V", "XTilde")}
+    out = {}
+    for bound, held in ((None, size), (size - 1, 0), (size, size), (0, 0)):
+        if bound is not None:
+            before = pd.direct_info()
+            pd.set_direct_memory(bound)
+            assert pd.direct_info() == before  # until the next update
+        for k, a in rest.items():
+            data._bufs[k].upload(a)
+        pd.Update(data, p)
+        pd.synchronize()
+        assert pd.direct_info()["inverse_bytes"] == held
+        out[bound] = data.get("X")
+        assert np.abs(out[bound] - out[None]).max() <= 1e-9 * np.abs(out[None]).max()
+    assert np.array_equal(out[size], out[None]) and np.array_equal(out[size - 1], out[0])
+    pd.close()
+    data.free()

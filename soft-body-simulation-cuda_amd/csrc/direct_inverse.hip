@@ -11,6 +11,13 @@ namespace {
 constexpr int kRowsPer = 8;       // rows of the inverse per workgroup of the product
 constexpr int kThreads = 256;
 constexpr int kStripCols = 64;    // columns of one inversion workgroup (one wavefront)
+// Up to this many workgroups the product decides the early exit itself, by a
+// ticket; with more, their atomics on one word (33 ns each: 1,024 bodies of 64
+// rows 267 us an iteration) cost more than a launch (42 us).  Single bodies, an
+// iteration with the ticket and with the launch, FP32, us: 125 rows 16.1 and
+// 16.3, 343 rows (43 workgroups) 16.8 and 17.1, 729 rows (92) 18.3 and 17.5,
+// 3,360 rows (420) 34.8 and 25.5.
+constexpr unsigned kTicketGroups = 64;
 constexpr int kPadTo = 4;         // rows are padded to whole 4-value loads
 constexpr size_t kScratchBytes = (size_t)4 << 30;   // FP64 columns in flight while inverting
 
@@ -126,6 +133,12 @@ __device__ __forceinline__ float row16_sum(float v) {
 }
 __device__ __forceinline__ double row16_sum(double v) { return row16_total(v); }
 
+template <class T> __device__ __forceinline__ void outer_decide(const OuterStep<T>& o, double sum, int nv) {
+    const double err = sum / (3.0 * (double)nv);
+    *o.err = err;
+    *o.done = !(sqrt(err) >= o.tol);
+}
+
 // kRowsPer rows of a system's inverse times its three right-hand sides.  Each
 // thread takes 4 consecutive columns of every 1,024: one 4-value load per
 // row and right-hand side, kRowsPer + 3 of them in flight.  Per thread the
@@ -137,13 +150,12 @@ __device__ __forceinline__ double row16_sum(double v) { return row16_total(v); }
 template <class T, bool kOuter>
 __global__ void __launch_bounds__(kThreads) inverse_apply_kernel(
     const int4* __restrict__ job, const long long* __restrict__ job_off, const T* __restrict__ inv,
-    const T* __restrict__ rhs, int stride, const int* __restrict__ vert, T* __restrict__ x, OuterStep<T> o, int nv,
-    double* parts, unsigned* ticket, const int* __restrict__ skip) {
+    const T* __restrict__ rhs, int stride, const int* __restrict__ vert, T* __restrict__ x, OuterStep<T> o,
+    int nv, double* parts, unsigned* ticket, const int* __restrict__ skip) {
     if (skip && *skip) return;
     typedef T V4 __attribute__((ext_vector_type(4)));
     constexpr int kVals = 3 * kRowsPer, kRows16 = kThreads / 16;
     __shared__ double red[kVals][kRows16 + 1];
-    __shared__ int last;
     const int4 j = job[blockIdx.x];  // first padded position of the system, its rows, ld, first row here
     const T* __restrict__ A = inv + job_off[blockIdx.x];
     const int ld = j.z, rows = min(kRowsPer, j.y - j.w);
@@ -174,7 +186,7 @@ __global__ void __launch_bounds__(kThreads) inverse_apply_kernel(
             if ((tid & 15) == 0) red[3 * r + c][tid >> 4] = (double)s;
         }
     __syncthreads();
-    if (tid >= 64 && !kOuter) return;
+    if (tid >= 64) return;
     double sq = 0.0;
     if (tid < 3 * rows) {
         double s = 0.0;
@@ -192,54 +204,69 @@ __global__ void __launch_bounds__(kThreads) inverse_apply_kernel(
         }
     }
     if constexpr (kOuter) {
-        // the workgroup that stores its sum last adds them all, in index order
-        if (tid < 64) {
-            const double s = wave_total(sq);
-            if (tid == 0) {
-                __hip_atomic_store(&parts[blockIdx.x], s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
-            }
+        const double total = wave_total(sq);
+        if (!ticket) {  // inverse_decide_kernel adds them
+            if (tid == 0) parts[blockIdx.x] = total;
+            return;
         }
-        __syncthreads();
-        if (!last || tid >= 64) return;
+        // the workgroup that stores its sum last adds them all (kTicketGroups at
+        // most, one per lane)
+        unsigned before = 0;
+        if (tid == 0) {
+            __hip_atomic_store(&parts[blockIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            before = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (__builtin_amdgcn_readfirstlane(before) != gridDim.x - 1) return;
         double s = 0.0;
-        for (unsigned k = tid; k < gridDim.x; k += 64)
-            s += __hip_atomic_load(&parts[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((unsigned)tid < gridDim.x)
+            s = __hip_atomic_load(&parts[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s = wave_total(s);
         if (tid == 0) {
-            const double err = s / (3.0 * (double)nv);
-            *o.err = err;
-            *o.done = !(sqrt(err) >= o.tol);
+            outer_decide(o, s, nv);
             *ticket = 0;
         }
     }
+}
+
+// The outer loop's error and decision from more than kTicketGroups workgroups'
+// sums, added in a fixed order.
+template <class T>
+__global__ void __launch_bounds__(kThreads) inverse_decide_kernel(int groups, int nv, const double* __restrict__ parts,
+                                                                  OuterStep<T> o, const int* __restrict__ skip) {
+    if (skip && *skip) return;
+    __shared__ double red[kThreads / 64];
+    double s = 0.0;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < groups; k += kThreads) s += parts[k];
+    s = wave_total(s);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) outer_decide(o, (red[0] + red[1]) + (red[2] + red[3]), nv);
 }
 
 int padded(int n) { return (n + kPadTo - 1) / kPadTo * kPadTo; }
 
 }  // namespace
 
-// The product reads n_s^2 values of each system, at about 4.5 TB/s; the band
-// solve walks the largest system's 64-row blocks twice, about 2.2 us a block
-// and sweep (12 blocks: 77 us, 53 blocks: 227 us), with about 512 workgroups
-// (three per system) side by side.
-template <class T> bool InverseOperator<T>::suits(const std::vector<int>& sys, size_t most_bytes) {
-    const int nsys = (int)sys.size() - 1;
+// An iteration of the outer loop (local step, right-hand side, solve, error,
+// decision) with the triangular solves and with the product, FP32, us: one
+// body of 8 rows 20.1 and 13.3, of 1,000 rows 193 and 17.9, of 21,952 rows
+// 10,891 and 359; 1,024 bodies of 64 rows 106 and 42, of 343 rows 437 and 214,
+// of 729 rows 1,046 and 594; 128 bodies of 2,197 rows 619 and 547 (FP64: 22.3
+// and 14.3, 227 and 20.2, 19,174 and 687; 187 and 69, 967 and 440, 2,318 and
+// 1,263; 1,603 and 1,072).  The product was the faster one at every size that
+// was measured, so the memory alone decides.
+template <class T> bool InverseOperator<T>::fits(const std::vector<int>& sys, size_t most_bytes) {
     size_t bytes = 0;
-    int longest = 0;
-    for (int s = 0; s < nsys; ++s) {
+    for (size_t s = 0; s + 1 < sys.size(); ++s) {
         const int n = sys[s + 1] - sys[s];
         bytes += (size_t)n * padded(n) * sizeof(T);
-        longest = std::max(longest, n);
     }
     // never more than a quarter of what is free: the inverse of a large body is
     // 27 to 50 times its factor, and the caller's arrays come first
     size_t free_bytes = 0, total_bytes = 0;
     if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) return false;
-    if (bytes > std::min(most_bytes, free_bytes / 4)) return false;
-    const double product_us = 5.0 + (double)bytes / 4.5e6;
-    const double band_us = 2.2 * 2 * ceil_div((size_t)longest, 64) * ceil_div(3 * (size_t)nsys, 512);
-    return product_us < band_us;
+    return bytes <= std::min(most_bytes, free_bytes / 4);
 }
 
 template <class T>
@@ -333,16 +360,20 @@ template <class T> void InverseOperator<T>::apply(T* x, hipStream_t stream, cons
     hipLaunchKernelGGL((inverse_apply_kernel<T, false>), dim3(groups_), dim3(kThreads), 0, stream,
                        (const int4*)job_.get(), (const long long*)job_off_.get(), (const T*)inv_.get(),
                        (const T*)rhs_.get(), npad_, (const int*)vert_.get(), x, OuterStep<T>{}, n_, parts_.get(),
-                       ticket_.get(), skip);
+                       (unsigned*)nullptr, skip);
     SBS_HIP(hipGetLastError());
 }
 
 template <class T>
 void InverseOperator<T>::apply_outer(const OuterStep<T>& o, hipStream_t stream, const int* skip) const {
+    const bool ticket = groups_ <= kTicketGroups;
     hipLaunchKernelGGL((inverse_apply_kernel<T, true>), dim3(groups_), dim3(kThreads), 0, stream,
                        (const int4*)job_.get(), (const long long*)job_off_.get(), (const T*)inv_.get(),
                        (const T*)rhs_.get(), npad_, (const int*)vert_.get(), (T*)nullptr, o, n_, parts_.get(),
-                       ticket_.get(), skip);
+                       ticket ? ticket_.get() : nullptr, skip);
+    if (!ticket)
+        hipLaunchKernelGGL(inverse_decide_kernel<T>, dim3(1), dim3(kThreads), 0, stream, (int)groups_, n_,
+                           (const double*)parts_.get(), o, skip);
     SBS_HIP(hipGetLastError());
 }
 

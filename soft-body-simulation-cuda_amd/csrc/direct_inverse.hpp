@@ -17,8 +17,9 @@
 namespace sbs {
 
 // The outer loop's end of iteration (computeError, pdSolver.cu:243-253, and
-// the early exit, :164) done by the product itself: sum (prev - x)^2, sn and
-// prev take x, and the last workgroup decides.
+// the early exit, :164) with the product: sn and prev take x, each workgroup
+// sums its (prev - x)^2, and the last of them or a launch of its own adds the
+// sums and decides.
 template <class T> struct OuterStep {
     T* sn;
     T* prev;
@@ -29,11 +30,10 @@ template <class T> struct OuterStep {
 
 template <class T> class InverseOperator {
 public:
-    // Whether the product with the inverse of this factor's systems (row
-    // ranges sys[s] .. sys[s+1]) is the faster solve and the inverse takes no
-    // more than most_bytes nor a quarter of the free memory; see the rule's
-    // comment.
-    static bool suits(const std::vector<int>& sys, size_t most_bytes);
+    // Whether the inverse of the systems (row ranges sys[s] .. sys[s+1]) takes no
+    // more than most_bytes nor a quarter of the free memory: the rule by which
+    // the product replaces the triangular solves, see its comment.
+    static bool fits(const std::vector<int>& sys, size_t most_bytes);
     void setup(const BandFactor& f, const std::vector<int>& sys, hipStream_t stream);
     bool ready() const { return n_ > 0; }
     size_t bytes() const { return inv_.bytes(); }

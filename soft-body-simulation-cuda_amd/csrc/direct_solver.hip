@@ -234,7 +234,7 @@ void BandCholesky<T>::factor(int n, const std::vector<int>& rowptr, const std::v
     bw_ = bw;
     nsys_ = (int)sys.size() - 1;
     inverse_ = InverseOperator<T>();
-    if (InverseOperator<T>::suits(sys, inverse_bytes)) {
+    if (InverseOperator<T>::fits(sys, inverse_bytes)) {
         try {
             inverse_.setup(f, sys, stream);
             return;

@@ -18,9 +18,8 @@
 //     the band update reads the previous (next) bw rows' values from a ring
 //     of bw + 64 rows in LDS, so the limit is the bandwidth (up to the LDS a
 //     workgroup may use), not the number of rows;
-//   * where the product with the explicit inverse is faster than that chain
-//     of blocks (InverseOperator::suits), the factor only gives the inverse
-//     and a solve is that product.
+//   * where there is room for the explicit inverse (InverseOperator::fits),
+//     the factor only gives that inverse and a solve is a product with it.
 #pragma once
 
 #include <vector>

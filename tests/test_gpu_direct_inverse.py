@@ -78,3 +78,31 @@ def test_memory_bound(gpu):
     assert np.array_equal(out[size], out[None]) and np.array_equal(out[size - 1], out[0])
     pd.close()
     data.free()
+
+
+def test_error_and_early_exit_of_many_bodies(gpu):
+    """The outer loop's error and decision from 1,300 workgroups' sums: the step
+    ends after the same iteration as with the triangular solves (whose error
+    and decision are launches of their own), FP64."""
+    scene = mesh.make_scene([dict(nx=2, ny=2, nz=2, seed=i, pin_top=True, origin=(1.0 * (i % 20), 0.0, 1.0 * (i // 20)))
+                             for i in range(320)] + [dict(nx=4, ny=5, nz=6, seed=7, origin=(0.0, 3.0, 0.0))])
+    out = {}
+    for tol in (0.0, 2e-5):
+        for bound in (4 << 30, 0):
+            data = SolverData(scene, 64)
+            pd = PdSolver(128, data)
+            pd.SetGlobalSolver(SolverType.CuSolverCholesky)
+            pd.set_direct_memory(bound)
+            for _ in range(2):
+                pd.Update(data, SolverParams(numIterations=12, dt=1.0 / 60.0, tol=tol))
+            pd.synchronize()
+            info = pd.direct_info()
+            assert info["systems"] == 321 and (info["inverse_bytes"] > 0) == (bound > 0)
+            out[tol, bound > 0] = data.get("X")
+            pd.close()
+            data.free()
+    scale = np.abs(out[0.0, True]).max()
+    for tol in (0.0, 2e-5):
+        assert np.abs(out[tol, True] - out[tol, False]).max() <= 1e-9 * scale
+    # the exit was taken: an iteration more moves some vertex by more than that
+    assert np.abs(out[0.0, True] - out[2e-5, True]).max() > 1e-7 * scale

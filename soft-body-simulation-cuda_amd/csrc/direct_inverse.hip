@@ -11,13 +11,14 @@ namespace {
 constexpr int kRowsPer = 8;       // rows of the inverse per workgroup of the product
 constexpr int kThreads = 256;
 constexpr int kStripCols = 64;    // columns of one inversion workgroup (one wavefront)
-// Up to this many workgroups the product decides the early exit itself, by a
-// ticket; with more, their atomics on one word (33 ns each: 1,024 bodies of 64
-// rows 267 us an iteration) cost more than a launch (42 us).  Single bodies, an
-// iteration with the ticket and with the launch, FP32, us: 125 rows 16.1 and
-// 16.3, 343 rows (43 workgroups) 16.8 and 17.1, 729 rows (92) 18.3 and 17.5,
-// 3,360 rows (420) 34.8 and 25.5.
-constexpr unsigned kTicketGroups = 64;
+// The outer loop's decision is taken by the workgroup that passes a ticket last.
+// Past kOneTicket workgroups the ticket is a tree of kStripes, since atomics on
+// one word follow each other at 11 ns each; up to there the second level costs
+// more (an iteration of one 125-row body 16.3 us with one ticket, 17.2 with the
+// tree; 16 bodies of 729 rows 41 and 24; 1,024 of 64 rows about 130 and 40).
+constexpr unsigned kOneTicket = 64;
+constexpr unsigned kStripes = 32;
+constexpr unsigned kTicketPitch = 32;  // words: a cache line of its own per ticket
 constexpr int kPadTo = 4;         // rows are padded to whole 4-value loads
 constexpr size_t kScratchBytes = (size_t)4 << 30;   // FP64 columns in flight while inverting
 
@@ -133,10 +134,30 @@ __device__ __forceinline__ float row16_sum(float v) {
 }
 __device__ __forceinline__ double row16_sum(double v) { return row16_total(v); }
 
-template <class T> __device__ __forceinline__ void outer_decide(const OuterStep<T>& o, double sum, int nv) {
-    const double err = sum / (3.0 * (double)nv);
-    *o.err = err;
-    *o.done = !(sqrt(err) >= o.tol);
+// Called by wavefront 0 of `members` workgroups: v (the same in every lane) into
+// the slot; true in the workgroup that comes last, which may then read all
+// slots.  The exchange's result is waited for, so the slot is written where all
+// XCDs see it before the ticket counts it; a release fence in every workgroup
+// instead writes back its XCD's L2 each time (32 bodies of 2,197 rows: 616 us
+// an iteration, this form 146).
+__device__ __forceinline__ bool passed_last(double v, double* slot, unsigned* ticket, unsigned members) {
+    unsigned before = 0;
+    if (threadIdx.x == 0) {
+        double old = __hip_atomic_exchange(slot, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(old)::"memory");
+        before = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (__builtin_amdgcn_readfirstlane(before) != members - 1) return false;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (threadIdx.x == 0) *ticket = 0;  // for the next launch
+    return true;
+}
+// Sum of `members` slots, `pitch` apart, in every lane of the wavefront.
+__device__ __forceinline__ double slot_sum(const double* slots, unsigned pitch, unsigned members) {
+    double s = 0.0;
+    for (unsigned k = threadIdx.x; k < members; k += 64)
+        s += __hip_atomic_load(&slots[(size_t)k * pitch], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return wave_total(s);
 }
 
 // kRowsPer rows of a system's inverse times its three right-hand sides.  Each
@@ -205,43 +226,24 @@ __global__ void __launch_bounds__(kThreads) inverse_apply_kernel(
     }
     if constexpr (kOuter) {
         const double total = wave_total(sq);
-        if (!ticket) {  // inverse_decide_kernel adds them
-            if (tid == 0) parts[blockIdx.x] = total;
-            return;
+        // the workgroup that passes its stripe's ticket last adds the stripe's
+        // sums, and the stripe that passes the common ticket last adds those
+        // (one level up to kOneTicket workgroups), each in index order
+        const unsigned groups = gridDim.x, stripes = groups <= kOneTicket ? 1u : kStripes;
+        const unsigned st = blockIdx.x % stripes, members = (groups - st + stripes - 1) / stripes;
+        double sum = total;
+        if (!passed_last(sum, &parts[blockIdx.x], &ticket[kTicketPitch * (1 + st)], members)) return;
+        sum = slot_sum(parts + st, stripes, members);
+        if (stripes > 1) {
+            if (!passed_last(sum, &parts[groups + st], ticket, stripes)) return;
+            sum = slot_sum(parts + groups, 1, stripes);
         }
-        // the workgroup that stores its sum last adds them all (kTicketGroups at
-        // most, one per lane)
-        unsigned before = 0;
         if (tid == 0) {
-            __hip_atomic_store(&parts[blockIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            before = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (__builtin_amdgcn_readfirstlane(before) != gridDim.x - 1) return;
-        double s = 0.0;
-        if ((unsigned)tid < gridDim.x)
-            s = __hip_atomic_load(&parts[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s = wave_total(s);
-        if (tid == 0) {
-            outer_decide(o, s, nv);
-            *ticket = 0;
+            const double err = sum / (3.0 * (double)nv);
+            *o.err = err;
+            *o.done = !(sqrt(err) >= o.tol);
         }
     }
-}
-
-// The outer loop's error and decision from more than kTicketGroups workgroups'
-// sums, added in a fixed order.
-template <class T>
-__global__ void __launch_bounds__(kThreads) inverse_decide_kernel(int groups, int nv, const double* __restrict__ parts,
-                                                                  OuterStep<T> o, const int* __restrict__ skip) {
-    if (skip && *skip) return;
-    __shared__ double red[kThreads / 64];
-    double s = 0.0;
-#pragma unroll 4
-    for (int k = threadIdx.x; k < groups; k += kThreads) s += parts[k];
-    s = wave_total(s);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) outer_decide(o, (red[0] + red[1]) + (red[2] + red[3]), nv);
 }
 
 int padded(int n) { return (n + kPadTo - 1) / kPadTo * kPadTo; }
@@ -297,8 +299,8 @@ void InverseOperator<T>::setup(const BandFactor& f, const std::vector<int>& sys,
     vert_.alloc(vert.size());
     job_.alloc(job.size());
     job_off_.alloc(off.size());
-    parts_.alloc(off.size());
-    ticket_.alloc(1);
+    parts_.alloc(off.size() + kStripes);
+    ticket_.alloc(kTicketPitch * (1 + kStripes));
     SBS_HIP(hipMemsetAsync(rhs_.get(), 0, rhs_.bytes(), stream));
     SBS_HIP(hipMemsetAsync(ticket_.get(), 0, ticket_.bytes(), stream));
     SBS_HIP(hipMemcpyAsync(pos_.get(), pos.data(), pos_.bytes(), hipMemcpyHostToDevice, stream));
@@ -366,14 +368,10 @@ template <class T> void InverseOperator<T>::apply(T* x, hipStream_t stream, cons
 
 template <class T>
 void InverseOperator<T>::apply_outer(const OuterStep<T>& o, hipStream_t stream, const int* skip) const {
-    const bool ticket = groups_ <= kTicketGroups;
     hipLaunchKernelGGL((inverse_apply_kernel<T, true>), dim3(groups_), dim3(kThreads), 0, stream,
                        (const int4*)job_.get(), (const long long*)job_off_.get(), (const T*)inv_.get(),
                        (const T*)rhs_.get(), npad_, (const int*)vert_.get(), (T*)nullptr, o, n_, parts_.get(),
-                       ticket ? ticket_.get() : nullptr, skip);
-    if (!ticket)
-        hipLaunchKernelGGL(inverse_decide_kernel<T>, dim3(1), dim3(kThreads), 0, stream, (int)groups_, n_,
-                           (const double*)parts_.get(), o, skip);
+                       ticket_.get(), skip);
     SBS_HIP(hipGetLastError());
 }
 

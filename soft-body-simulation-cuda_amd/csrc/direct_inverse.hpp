@@ -17,9 +17,8 @@
 namespace sbs {
 
 // The outer loop's end of iteration (computeError, pdSolver.cu:243-253, and
-// the early exit, :164) with the product: sn and prev take x, each workgroup
-// sums its (prev - x)^2, and the last of them or a launch of its own adds the
-// sums and decides.
+// the early exit, :164) done by the product itself: sum (prev - x)^2, sn and
+// prev take x, and the last workgroup decides.
 template <class T> struct OuterStep {
     T* sn;
     T* prev;
@@ -58,8 +57,8 @@ private:
     DevBuf<int> pos_, vert_;   // vertex -> padded position; padded position -> vertex
     DevBuf<int> job_;          // per workgroup: first padded position, rows, ld, first row
     DevBuf<long long> job_off_;  // per workgroup: first value of its first row
-    DevBuf<double> parts_;     // per workgroup: its sum of squared differences
-    DevBuf<unsigned> ticket_;  // workgroups that have stored theirs
+    DevBuf<double> parts_;     // per workgroup, then per stripe: its sum of squared differences
+    DevBuf<unsigned> ticket_;  // stripes, then per stripe workgroups, that have stored theirs
 };
 
 }  // namespace sbs

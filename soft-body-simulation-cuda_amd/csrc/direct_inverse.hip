@@ -293,20 +293,6 @@ void InverseOperator<T>::setup(const BandFactor& f, const std::vector<int>& sys,
         total += (long long)n * ld;
         npad += ld;
     }
-    inv_.alloc((size_t)total);
-    rhs_.alloc(3 * (size_t)npad);
-    pos_.alloc(pos.size());
-    vert_.alloc(vert.size());
-    job_.alloc(job.size());
-    job_off_.alloc(off.size());
-    parts_.alloc(off.size() + kStripes);
-    ticket_.alloc(kTicketPitch * (1 + kStripes));
-    SBS_HIP(hipMemsetAsync(rhs_.get(), 0, rhs_.bytes(), stream));
-    SBS_HIP(hipMemsetAsync(ticket_.get(), 0, ticket_.bytes(), stream));
-    SBS_HIP(hipMemcpyAsync(pos_.get(), pos.data(), pos_.bytes(), hipMemcpyHostToDevice, stream));
-    SBS_HIP(hipMemcpyAsync(vert_.get(), vert.data(), vert_.bytes(), hipMemcpyHostToDevice, stream));
-    SBS_HIP(hipMemcpyAsync(job_.get(), job.data(), job_.bytes(), hipMemcpyHostToDevice, stream));
-    SBS_HIP(hipMemcpyAsync(job_off_.get(), off.data(), job_off_.bytes(), hipMemcpyHostToDevice, stream));
     // the factor by rows and by columns, kBlkRows zeros past the band and past the last row
     const int lw = f.bw + 1 + kBlkRows;
     std::vector<double> Lr((size_t)(f.n + kBlkRows) * lw, 0.0), Uc(Lr.size(), 0.0), ri(f.n + kBlkRows, 1.0);
@@ -318,12 +304,21 @@ void InverseOperator<T>::setup(const BandFactor& f, const std::vector<int>& sys,
             Uc[(size_t)(i - d) * lw + d] = Li[d];
         }
     }
+    // every allocation before the first copy: one that fails leaves nothing of the host's vectors in flight
+    inv_.alloc((size_t)total);
+    rhs_.alloc(3 * (size_t)npad);
+    pos_.alloc(pos.size());
+    vert_.alloc(vert.size());
+    job_.alloc(job.size());
+    job_off_.alloc(off.size());
+    parts_.alloc(off.size() + kStripes);
+    ticket_.alloc(kTicketPitch * (1 + kStripes));
     DevBuf<double> dLr(Lr.size()), dUc(Uc.size()), dri(ri.size());
-    SBS_HIP(hipMemcpyAsync(dLr.get(), Lr.data(), dLr.bytes(), hipMemcpyHostToDevice, stream));
-    SBS_HIP(hipMemcpyAsync(dUc.get(), Uc.data(), dUc.bytes(), hipMemcpyHostToDevice, stream));
-    SBS_HIP(hipMemcpyAsync(dri.get(), ri.data(), dri.bytes(), hipMemcpyHostToDevice, stream));
-    // strips in runs whose columns fit the scratch
-    const size_t most = kScratchBytes / sizeof(double);
+    DevBuf<StripJob> dstrips(strips.size());
+    // strips in runs whose columns fit the scratch, which takes a quarter of the free memory at most
+    size_t free_bytes = 0, total_bytes = 0;
+    SBS_HIP(hipMemGetInfo(&free_bytes, &total_bytes));
+    const size_t most = std::min(kScratchBytes, free_bytes / 4) / sizeof(double);
     size_t scratch = 0;
     std::vector<size_t> runs = {0};
     for (size_t k = 0; k < strips.size(); ++k) {
@@ -338,7 +333,15 @@ void InverseOperator<T>::setup(const BandFactor& f, const std::vector<int>& sys,
     }
     runs.push_back(strips.size());
     DevBuf<double> Y(scratch);
-    DevBuf<StripJob> dstrips(strips.size());
+    SBS_HIP(hipMemsetAsync(rhs_.get(), 0, rhs_.bytes(), stream));
+    SBS_HIP(hipMemsetAsync(ticket_.get(), 0, ticket_.bytes(), stream));
+    SBS_HIP(hipMemcpyAsync(pos_.get(), pos.data(), pos_.bytes(), hipMemcpyHostToDevice, stream));
+    SBS_HIP(hipMemcpyAsync(vert_.get(), vert.data(), vert_.bytes(), hipMemcpyHostToDevice, stream));
+    SBS_HIP(hipMemcpyAsync(job_.get(), job.data(), job_.bytes(), hipMemcpyHostToDevice, stream));
+    SBS_HIP(hipMemcpyAsync(job_off_.get(), off.data(), job_off_.bytes(), hipMemcpyHostToDevice, stream));
+    SBS_HIP(hipMemcpyAsync(dLr.get(), Lr.data(), dLr.bytes(), hipMemcpyHostToDevice, stream));
+    SBS_HIP(hipMemcpyAsync(dUc.get(), Uc.data(), dUc.bytes(), hipMemcpyHostToDevice, stream));
+    SBS_HIP(hipMemcpyAsync(dri.get(), ri.data(), dri.bytes(), hipMemcpyHostToDevice, stream));
     SBS_HIP(hipMemcpyAsync(dstrips.get(), strips.data(), dstrips.bytes(), hipMemcpyHostToDevice, stream));
     for (size_t k = 0; k + 1 < runs.size(); ++k) {
         hipLaunchKernelGGL(inverse_strip_kernel<T>, dim3((unsigned)(runs[k + 1] - runs[k])), dim3(64 * kStripWaves), 0,

@@ -14,7 +14,6 @@ namespace sbs {
 namespace {
 
 constexpr int kTpbL = 256;
-constexpr int kCheck = 16;  // fewest iterations launched between host reads of the control word
 
 struct LinCtl {
     double rho[2];   // r.z of iteration k, by parity of k
@@ -525,14 +524,10 @@ int CooPcgSolver<T>::solve_in(int n, const T* b, T* x, const T* A, long long nz,
             default: launch(pcg_spmv_kernel<32, true, T>); break;
         }
     };
+    looks_.begin(n, nz, guess != nullptr);
     int k = 0;
     while (k < max_iter_) {
-        // a look at the control word leaves the GPU idle for about 30 us, an
-        // iteration launched after the solve has stopped costs 5: the first
-        // look after 9/10 of this solver's previous count, then every quarter
-        // of what has been launched
-        const int want = k == 0 ? std::max(kCheck, last_iters_ * 9 / 10) : std::max(kCheck, k / 4);
-        const int chunk = std::min(want, max_iter_ - k);
+        const int chunk = std::min(looks_.next(k), max_iter_ - k);
         for (int j = 0; j < chunk; ++j, ++k) {
             const int par = k & 1;
             product(k, L.prr + par * nb, L.prz + par * nb);
@@ -545,7 +540,7 @@ int CooPcgSolver<T>::solve_in(int n, const T* b, T* x, const T* A, long long nz,
         SBS_HIP(hipStreamSynchronize(stream));
         if (hc.done) break;
     }
-    last_iters_ = hc.iters;
+    looks_.end(hc.iters, hc.done != 0);
     return hc.iters;
 }
 

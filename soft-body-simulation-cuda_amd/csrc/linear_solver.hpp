@@ -9,14 +9,14 @@
 //     rho = r.z, stop when |rho| < 1e-15, p = z (+ beta p), q = A p,
 //     alpha = rho / p.q, x += alpha p, r -= alpha q; at most max_iter.
 // Dot products accumulate in double whatever T is.  The scalars stay on the
-// device; the host reads the control word at points that follow the previous
-// solve's iteration count.
+// device; look_schedule.hpp says when the host reads the control word.
 #pragma once
 
 #include <cstddef>
 #include <cstdint>
 
 #include "common.hpp"
+#include "look_schedule.hpp"
 
 namespace sbs {
 
@@ -56,7 +56,7 @@ private:
     int max_iter_;
     double tol_;
     long long nnz_ = 0;
-    int last_iters_ = 0;  // of the previous solve: when the host first looks at this one
+    LookSchedule looks_;
     DevBuf<unsigned char> ws_;
 };
 

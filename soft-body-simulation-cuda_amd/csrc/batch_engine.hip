@@ -7,9 +7,13 @@
 //   Jacobi-PCG warm-started from sn, per component stopping when
 //   ||D^-1 r_k|| <= max(tol ||D^-1 r_0||, floor ||D^-1 b||);
 //   the Chebyshev recurrence (pdSolver.cu:196-198, pdUtil.cu:216-226);
-// the last three by one workgroup per body in one launch.  Reductions are
-// block reductions in a fixed order, so a body's result does not depend on the
-// other bodies or on scheduling.  See batch_engine.hpp.
+// the last three by one workgroup per body in one launch.  A body's forces are
+// summed in an order of its own and reductions are block reductions in a fixed
+// order, so its result does not depend on scheduling.  On the other bodies it
+// depends through two orders of summation only: the workgroup size (the
+// tuner's, or half a thread per vertex of the largest body) sets that of the
+// block sums, and the scene's box, whose Morton curve the assembly follows,
+// that of the matrix entries.  See batch_engine.hpp.
 #include "batch_engine.hpp"
 
 #include <algorithm>
@@ -129,13 +133,14 @@ template <class T> __global__ void __launch_bounds__(kTpbB) batch_end_kernel(Bat
 
 template <class T>
 __global__ void __launch_bounds__(kChunkTets) batch_local_kernel(
-    int nt, const uint2* __restrict__ lidx, const int* __restrict__ chunk_vptr,
+    int nt, const int* __restrict__ chunk_tptr, const uint2* __restrict__ lidx, const int* __restrict__ chunk_vptr,
     const uint32_t* __restrict__ chunk_verts, const uint32_t* __restrict__ entry_pos,
     const uint16_t* __restrict__ inc_codes, const uint16_t* __restrict__ inc_end, const T* __restrict__ dminv,
     const T* __restrict__ w, const T* __restrict__ q, T* __restrict__ partial, int flags) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    local_chunk<T>(xcd_block(blockIdx.x, gridDim.x), nt, lidx, chunk_vptr, chunk_verts, entry_pos, inc_codes, inc_end,
-                   dminv, w, partial, flags, smem_raw, [&](int, uint32_t g, T& x, T& y, T& z) {
+    const unsigned c = xcd_block(blockIdx.x, gridDim.x);
+    local_chunk<T>(c, chunk_tptr[c], chunk_tptr[c + 1], nt, lidx, chunk_vptr, chunk_verts, entry_pos, inc_codes,
+                   inc_end, dminv, w, partial, flags, smem_raw, [&](int, uint32_t g, T& x, T& y, T& z) {
         x = q[3 * (size_t)g];
         y = q[3 * (size_t)g + 1];
         z = q[3 * (size_t)g + 2];
@@ -623,11 +628,15 @@ template <class T> BatchEngine<T>::BatchEngine(const BatchSystem<T>& s) {
     sn_.alloc(n3); sn_old_.alloc(n3); prev_.alloc(n3); x_.alloc(n3); r_.alloc(n3); p_.alloc(n3); q_.alloc(n3);
     stats_.alloc(4 * (size_t)nb_);
     reset_stats();
-    // the tets in chunks: body by body, along a Morton curve of the
-    // rest centroids inside a body
+    // the tets in chunks: a body's tets along a Morton curve of the rest
+    // centroids, cut every kChunkTets; what is left of each body goes whole
+    // into shared chunks at the end.  So the tets whose forces a chunk sums for
+    // a vertex, and the order of a vertex's partial forces, are the body's own,
+    // whatever other bodies there are.
     std::vector<std::vector<int>> tets_of(nb_);
     for (int t = 0; t < nt_; ++t) tets_of[place[number[s.tets[4 * (size_t)t]]]].push_back(t);
-    std::vector<int> seq;
+    std::vector<int> seq, starts, rest;
+    std::vector<size_t> rest_n;
     std::vector<std::pair<uint32_t, int>> key;
     for (int b = 0; b < nb_; ++b) {
         double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
@@ -644,8 +653,23 @@ template <class T> BatchEngine<T>::BatchEngine(const BatchSystem<T>& s) {
             key.emplace_back(morton_code(cen, lo, hi), t);
         }
         std::sort(key.begin(), key.end());
-        for (const auto& q : key) seq.push_back(q.second);
+        const size_t whole = key.size() / kChunkTets * kChunkTets;
+        for (size_t i = 0; i < whole; ++i) {
+            if (i % kChunkTets == 0) starts.push_back((int)seq.size());
+            seq.push_back(key[i].second);
+        }
+        for (size_t i = whole; i < key.size(); ++i) rest.push_back(key[i].second);
+        rest_n.push_back(key.size() - whole);
     }
+    for (size_t b = 0, r = 0, room = 0; b < rest_n.size(); ++b) {  // room: of the last shared chunk
+        if (rest_n[b] > room) {
+            starts.push_back((int)seq.size());
+            room = kChunkTets;
+        }
+        room -= rest_n[b];
+        for (size_t e = r + rest_n[b]; r < e; ++r) seq.push_back(rest[r]);
+    }
+    starts.push_back((int)seq.size());
     const int nt = (int)seq.size();
     std::vector<uint32_t> tv(4 * (size_t)nt);
     std::vector<T> dm(9 * (size_t)nt), w(nt);
@@ -655,11 +679,12 @@ template <class T> BatchEngine<T>::BatchEngine(const BatchSystem<T>& s) {
         for (int k = 0; k < 9; ++k) dm[(size_t)k * nt + i] = s.dminv[9 * t + k];
         w[i] = s.w[t];
     }
-    const ChunkLists ch = build_chunk_lists(nv_, tv);
-        chunks_ = ch.chunks;
+    const ChunkLists ch = build_chunk_lists(nv_, tv, starts);
+    chunks_ = ch.chunks;
     local_lds_ = chunk_lds_bytes<T>(ch.max_verts);
     SBS_REQUIRE(local_lds_ <= 64 * 1024, "batched PD: chunk vertex list exceeds LDS");
     upload(lidx_, ch.lidx);
+    upload(chunk_tptr_, starts);
     upload(chunk_vptr_, ch.vptr);
     upload(chunk_verts_, ch.verts);
     upload(entry_pos_, ch.pos);
@@ -771,7 +796,8 @@ void BatchEngine<T>::launch_step(T* X, T* V, T* XT, const T* DBCX, const BatchPa
     T omega = 1;
     for (int i = 0; i < p.iterations; ++i) {
         if (chunks_ > 0)
-            hipLaunchKernelGGL(batch_local_kernel<T>, dim3(chunks_), dim3(kChunkTets), local_lds_, s, nt_, lidx_.get(),
+            hipLaunchKernelGGL(batch_local_kernel<T>, dim3(chunks_), dim3(kChunkTets), local_lds_, s, nt_,
+                               (const int*)chunk_tptr_.get(), lidx_.get(),
                                chunk_vptr_.get(), chunk_verts_.get(), entry_pos_.get(), inc_codes_.get(),
                                inc_end_.get(), dminv_.get(), w_.get(), (const T*)sn_.get(), partial_.get(),
                                p.polar ? kLocalPolar : 0);

@@ -90,7 +90,7 @@ private:
     int chunks_ = 0;
     size_t local_lds_ = 0;               // of a chunk's workgroup
     DevBuf<uint2> lidx_;
-    DevBuf<int> chunk_vptr_, vent_ptr_;
+    DevBuf<int> chunk_tptr_, chunk_vptr_, vent_ptr_;
     DevBuf<uint32_t> chunk_verts_, entry_pos_;
     DevBuf<uint16_t> inc_codes_, inc_end_;
     DevBuf<T> dminv_, w_, partial_;

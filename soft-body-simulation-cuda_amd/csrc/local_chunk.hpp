@@ -1,7 +1,7 @@
 // Tet chunks of the local step: the host builder of their lists and the
 // device body shared by the kernels that run computeLocal over them.
 //
-// A chunk is kChunkTets consecutive tets of some order (one workgroup).  It
+// A chunk is up to kChunkTets consecutive tets of some order (one workgroup).  It
 // lists the vertices it touches (sorted; an entry is a (chunk, vertex) pair),
 // its tets' corners as indices into that list, and per entry the (tet, corner)
 // pairs that touch it in tet order.  The forces of an entry's tets are summed
@@ -47,11 +47,12 @@ struct ChunkLists {
     std::vector<uint16_t> inc_end;      // per entry: end of its codes in the chunk's list
 };
 
-// tets: 4 vertices (below nv) per tet, in the chunks' order.
-inline ChunkLists build_chunk_lists(int nv, const std::vector<uint32_t>& tets) {
+// tets: 4 vertices (below nv) per tet, in the chunks' order; chunk c holds the
+// tets starts[c] .. starts[c + 1] (kChunkTets at most).
+inline ChunkLists build_chunk_lists(int nv, const std::vector<uint32_t>& tets, const std::vector<int>& starts) {
     ChunkLists o;
     const int nt = (int)(tets.size() / 4);
-    o.chunks = (nt + kChunkTets - 1) / kChunkTets;
+    o.chunks = (int)starts.size() - 1;
     o.vptr.assign(o.chunks + 1, 0);
     o.verts.reserve((size_t)nt * 2);
     o.lidx.resize(nt);
@@ -60,7 +61,7 @@ inline ChunkLists build_chunk_lists(int nv, const std::vector<uint32_t>& tets) {
     std::vector<uint32_t> tmp;
     std::vector<int> cnt(4 * kChunkTets), at;
     for (int c = 0; c < o.chunks; ++c) {
-        const int t0 = c * kChunkTets, t1 = std::min(nt, t0 + kChunkTets);
+        const int t0 = starts[c], t1 = starts[c + 1];
         tmp.assign(tets.begin() + 4 * (size_t)t0, tets.begin() + 4 * (size_t)t1);
         std::sort(tmp.begin(), tmp.end());
         tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
@@ -100,6 +101,15 @@ inline ChunkLists build_chunk_lists(int nv, const std::vector<uint32_t>& tets) {
     return o;
 }
 
+// Chunks of kChunkTets tets, the last one of what is left.
+inline ChunkLists build_chunk_lists(int nv, const std::vector<uint32_t>& tets) {
+    const int nt = (int)(tets.size() / 4);
+    std::vector<int> starts;
+    for (int t = 0; t < nt; t += kChunkTets) starts.push_back(t);
+    starts.push_back(nt);
+    return build_chunk_lists(nv, tets, starts);
+}
+
 // LDS of one workgroup: corner forces, staged q, incidence list.
 template <class T> size_t chunk_lds_bytes(int max_verts) {
     const size_t b = (12 * (size_t)kChunkTets + 3 * (size_t)max_verts) * sizeof(T) +
@@ -112,7 +122,8 @@ template <class T> __device__ __forceinline__ void load_dminv(const T* __restric
     for (int k = 0; k < 9; ++k) m[k] = dminv[(size_t)k * nt + t];
 }
 
-// Chunk c of the lists, by a workgroup of kChunkTets threads:
+// Chunk c of the lists, the tets t0 .. t1 (thread i the tet t0 + i), by a
+// workgroup of kChunkTets threads:
 //   1. the chunk's vertices are staged into LDS (stage(entry, vertex, x, y, z)
 //      gives the position), with the chunk's incidence list;
 //   2. one thread per tet: F = Ds Dm^-1, the rotation in registers, R (or
@@ -122,7 +133,8 @@ template <class T> __device__ __forceinline__ void load_dminv(const T* __restric
 //      force at its slot.
 // No atomics anywhere, so the result is deterministic.
 template <class T, class Stage>
-__device__ __forceinline__ void local_chunk(unsigned c, int nt, const uint2* __restrict__ lidx,
+__device__ __forceinline__ void local_chunk(unsigned c, unsigned t0, unsigned t1, int nt,
+                                            const uint2* __restrict__ lidx,
                                             const int* __restrict__ chunk_vptr,
                                             const uint32_t* __restrict__ chunk_verts,
                                             const uint32_t* __restrict__ entry_pos,
@@ -148,8 +160,8 @@ __device__ __forceinline__ void local_chunk(unsigned c, int nt, const uint2* __r
         for (int k = threadIdx.x; k < 2 * kChunkTets; k += kChunkTets) dst[k] = src[k];
     }
     __syncthreads();
-    const unsigned t = c * kChunkTets + threadIdx.x;
-    if (t < (unsigned)nt) {
+    const unsigned t = t0 + threadIdx.x;
+    if (t < t1) {
         const uint2 li = lidx[t];
         const unsigned l0 = li.x & 0xffffu, l1 = li.x >> 16, l2 = li.y & 0xffffu, l3 = li.y >> 16;
         T m[9];

@@ -1012,7 +1012,7 @@ __global__ void __launch_bounds__(kChunkTets) local_chunk_kernel(
         for (int i = threadIdx.x; i < zero_n; i += kChunkTets) zero_slots[i] = 0.0;
     }
     const unsigned c = xcd_block(blockIdx.x, gridDim.x);
-    local_chunk<T>(c, nt, lidx, chunk_vptr, chunk_verts, entry_pos, inc_codes, inc_end, dminv, w, partial, flags,
+    local_chunk<T>(c, c * kChunkTets, nt, nt, lidx, chunk_vptr, chunk_verts, entry_pos, inc_codes, inc_end, dminv, w, partial, flags,
                    smem_raw, [&](int e, uint32_t g, T& x, T& y, T& z) {
         if (kFold) {
             const uint32_t rw = fold.rows[e];

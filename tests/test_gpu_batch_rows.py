@@ -88,3 +88,28 @@ def test_rows_wider_than_the_registers(gpu, precision):
                    mass=np.full(len(X), base.mass[0]), mu=np.full(m, base.mu[0]), lam=np.full(m, base.lam[0]),
                    dbc=np.zeros(len(X)), body_vert_start=np.array([0, len(X)]), body_tet_start=np.array([0, m]))
     check([s], s, precision, tune=False)
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_result_does_not_depend_on_the_other_bodies(gpu, precision):
+    """A body's step is the same to the bit whatever bodies are beside it: bodies
+    of less than a tet chunk, of several and of several whole ones.  Two bodies
+    are in every scene at the corners of its box (the matrix is assembled in the
+    order of a Morton curve over that box) and one is the largest (the workgroup
+    size follows it)."""
+    def spec(i, n, origin):
+        return dict(nx=n[0], ny=n[1], nz=n[2], spacing=0.1, origin=origin, jitter=1e-3, nu=0.3, E=2e5,
+                    seed=i, density=1000.0, pin_top=True)
+    dims = [(1, 1, 1), (7, 7, 7), (2, 2, 2), (5, 4, 4), (8, 4, 8), (3, 4, 5), (1, 1, 1), (6, 7, 5)]
+    assert 6 * 8 * 4 * 8 % 256 == 0  # whole chunks only
+    specs = [spec(i, n, (3.0 * i, 0.0, 0.0)) for i, n in enumerate(dims)]
+    specs[0] = spec(0, dims[0], (-5.0, -5.0, -5.0))
+    specs.append(spec(8, (1, 1, 1), (30.0, 5.0, 5.0)))
+    full = mesh.make_scene(specs)
+    X, _ = solve(full, precision, SolverType.BatchedPCG, batch_autotune=False)
+    ref = [X[full.body_vert_start[i]:full.body_vert_start[i + 1]] for i in range(len(specs))]
+    for keep in ([0, 1, 8], [3, 0, 1, 8], [5, 0, 8, 1, 2], [0, 1, 7, 6, 4, 8]):
+        s = mesh.make_scene([specs[i] for i in keep])
+        x, _ = solve(s, precision, SolverType.BatchedPCG, batch_autotune=False)
+        for j, i in enumerate(keep):
+            assert np.array_equal(x[s.body_vert_start[j]:s.body_vert_start[j + 1]], ref[i]), (keep, i)

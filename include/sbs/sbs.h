@@ -116,9 +116,9 @@ typedef struct SbsSolverParams {
     double mu_t;          /* fixed-body response: friction (muT)            */
     int use_graph;        /* 1: on a non-null stream, capture the step's launches once into a
                              HIP graph and replay it while launch sequence, arrays and
-                             parameters stay the same (Jacobi, or adaptive PCG with learned
-                             caps; no collision handling, perf or kernel timing).  On MI355X
-                             a replay costs what the eager launches cost (64^3 cube: 248 vs
+                             parameters stay the same (Jacobi, or adaptive PCG, with
+                             learned caps past 1,024 vertices; no collision handling, perf
+                             or kernel timing).  On MI355X a replay costs what the eager launches cost (64^3 cube: 248 vs
                              256 steps/s; 8^3: 660 vs 654), so 0 is the usual choice */
     int batch_autotune;   /* SBS_SOLVER_BATCHED_PCG: 1 times a step with each workgroup
                              size at the first batched update (state unchanged); 0 keeps

@@ -2524,21 +2524,23 @@ template <class T> void PdEngine<T>::update(PdData<T>& data, const PdParams& par
     // A step whose launch sequence is known in advance (no host reads of the
     // device state, no timing events) is captured once into a HIP graph and
     // replayed while the sequence, its pointers and its parameters stay the
-    // same; the learned PCG caps are part of that key.
+    // same; the learned PCG caps are part of that key where solves are runs of
+    // launches (a solve in one workgroup is one launch whatever its count).
+    const bool capped = pcg && !small_pcg(params);
     bool caps_known = true;
-    if (pcg)
+    if (capped)
         for (int i = 0; i < params.num_iterations; ++i) caps_known = caps_known && cap_[i] > 0;
     const bool graph = params.use_graph && stream_ != nullptr && !perf_ && timing_mask_ == 0 && !params.handle_collision &&
                        (solver_ == GlobalSolver::Jacobi || solver_ == GlobalSolver::BatchedPCG ||
                         (pcg && params.pcg_adaptive && caps_known));
     if (graph) {
         const std::vector<uint64_t> key = step_key(data, params);
-        if (!graph_exec_ || key != graph_key_ || graph_caps_stale(pcg ? params.num_iterations : 0)) {
+        if (!graph_exec_ || key != graph_key_ || graph_caps_stale(capped ? params.num_iterations : 0)) {
             drop_graph();
             // the graph keeps its own caps, one launch above the learned ones,
             // so that counts moving by a few launches replay the same graph
             std::vector<int> learned;
-            if (pcg) {
+            if (capped) {
                 learned = cap_;
                 graph_caps_.assign(cap_.begin(), cap_.end());
                 for (int& c : graph_caps_) c = std::min(cap_max_iter_, c + 1);
@@ -2551,10 +2553,10 @@ template <class T> void PdEngine<T>::update(PdData<T>& data, const PdParams& par
             } catch (...) {
                 (void)hipStreamEndCapture(stream_, &gr);
                 if (gr) (void)hipGraphDestroy(gr);
-                if (pcg) cap_ = learned;
+                if (capped) cap_ = learned;
                 throw;
             }
-            if (pcg) cap_ = learned;
+            if (capped) cap_ = learned;
             SBS_HIP(hipStreamEndCapture(stream_, &gr));
             const hipError_t e = hipGraphInstantiate(&graph_exec_, gr, nullptr, nullptr, 0);
             (void)hipGraphDestroy(gr);

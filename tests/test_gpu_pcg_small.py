@@ -9,10 +9,12 @@ relative, the bar of the PCG tests).  In FP32 both stop by the same test and
 differ in the sums' order, so the distance to the FP64 solution may be at most
 twice the row-gather kernels' plus 1e-6 (8 units of FP32 rounding of the
 positions that are handed back)."""
+import numpy as np
 import pytest
 
 from conftest import rel_err
 from test_gpu_pcg_quads import body, fan
+from test_gpu_pd import graph_pair
 from sbs_amd.pd import PdSolver, SolverData, SolverParams, SolverType
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +68,23 @@ def test_iteration_limit(gpu, precision):
     assert st.pcg_iterations_total == sr.pcg_iterations_total == 3 * 18
     assert st.pcg_cap_hits == sr.pcg_cap_hits == 18
     assert rel_err(x, ref) < (1e-5 if precision == 32 else 1e-12)
+
+
+@pytest.mark.parametrize("mode", ["chebyshev", "early exit", "more solves than the log"])
+def test_graph_is_captured_once(gpu, mode):
+    """The launches of a step do not depend on the iteration counts, so the first
+    step is captured and replayed from then on, solves that the early exit skips
+    and solves past the 64 that the step's log holds among them."""
+    p = SolverParams(numIterations=70 if mode == "more solves than the log" else 8, dt=1.0 / 60.0, rho=0.9992,
+                     tol=1e-4 if mode == "early exit" else 0.0, pcg_tol=1e-6, pcg_floor=1e-8, pcg_max_iter=400,
+                     pcg_chebyshev=mode == "chebyshev", pcg_adaptive=True)
+
+    def check(k, xg, xe):
+        np.testing.assert_array_equal(xg, xe, err_msg=f"step {k}")  # every sum has a fixed order
+
+    sg, se = graph_pair(body(4, 5, 6), SolverType.PCG, p, 8, check)
+    assert sg.graph_captures == 1 and sg.graph_replays == 8
+    assert sg.pcg_solves_total == se.pcg_solves_total
+    if mode == "early exit":
+        assert se.pcg_solves_total < 8 * 8
+    assert se.graph_captures == 0 and se.graph_replays == 0

@@ -616,6 +616,15 @@ __global__ void __launch_bounds__(kQB) ipc_barrier_kernel(long long nq, const Qu
             H[12 * a + b] = coef * (d2 * gd[a] * gd[b] + d1 * M[(12 * a + b) * kQB + lane]);
 }
 
+// Orders the LDS accesses of a wavefront's lanes among each other, for the
+// compiler (the hardware runs a wavefront's LDS instructions in order, so this
+// costs no instruction).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // makePD (matrix.h:441-518) of the active queries' Hessians in hq, and their
 // diagonal into the Jacobi diagonal of the free vertices: cyclic Jacobi over
 // the pairs p < q, rotations skipped when |a_pq| < 1e-9, at most 20 sweeps;
@@ -655,7 +664,6 @@ __global__ void __launch_bounds__(64) ipc_barrier_pd_kernel(long long nq, const 
         bool moved = false;
         for (int p = 0; p < 12; ++p)
             for (int q = p + 1; q < 12; ++q) {
-                // (a block of one wavefront: LDS accesses keep their order)
                 double apq = 0.0, app = 0.0, aqq = 0.0, akp = 0.0, akq = 0.0, vkp = 0.0, vkq = 0.0;
                 if (run) {
                     apq = m[p][q];
@@ -668,7 +676,7 @@ __global__ void __launch_bounds__(64) ipc_barrier_pd_kernel(long long nq, const 
                 }
                 const bool turn = run && !(fabs(apq) < 1e-9);
                 if (__ballot(turn) == 0ull) continue;
-                __builtin_amdgcn_wave_barrier();
+                wave_sync();  // every lane has read before one writes
                 if (turn) {
                     moved = true;
                     // t = sign(theta) / (|theta| + sqrt(1 + theta^2)), theta = (a_qq - a_pp) / (2 a_pq)
@@ -692,7 +700,7 @@ __global__ void __launch_bounds__(64) ipc_barrier_pd_kernel(long long nq, const 
                     v[k][p] = c * vkp - s * vkq;
                     v[k][q] = s * vkp + c * vkq;
                 }
-                __builtin_amdgcn_wave_barrier();
+                wave_sync();
             }
         // a sweep without a rotation ends the query (its 12 lanes take the same decision)
         run = run && moved;

@@ -1,10 +1,12 @@
-"""The contact blocks of the IPC solver's preconditioner: one partial block
-(16 contact vertices), one full block (32) and several with a remainder (72),
-steps in contact from the start against the IPC oracle; and blocks that are
-not positive definite, which take their diagonal."""
+"""The contact blocks of the IPC solver's preconditioner: one partial block (12
+contact vertices at the start of the smallest scene) and full ones with a
+remainder (34 vertices, 56, more), steps in contact from the start against the
+IPC oracle; the preconditioned direction itself; and blocks that are not
+positive definite, which take their diagonal."""
 import numpy as np
 import pytest
 
+import oracle as O
 from sbs_amd import mesh
 from sbs_amd.ipc import IpcData, IpcParams, IpcSolver
 from test_gpu_ipc import run_pair
@@ -36,3 +38,87 @@ def test_blocks_that_are_not_positive_definite(gpu):
     assert np.all(np.isfinite(data.get("X")))
     solver.close()
     data.free()
+
+
+def newton_system(s, p, kappa):
+    """Gradient and Hessian at the rest positions (x~ there too), fixed vertices
+    eliminated, and the free vertices of active queries, from the oracle's
+    gradient, Neo-Hookean d2Psi/dF2, distance derivatives and makePD."""
+    fixed, h2 = s.dbc > 0, p.dt ** 2
+    o = O.IpcOracle(s.X, np.zeros_like(s.X), s.tet, s.tri, s.tri_fathers, s.mass, s.mu, s.lam, fixed, dt=p.dt,
+                    damp=p.damp, dhat=p.dhat, tol=p.tol, elastic="neohookean")
+    o.set_state(s.X, kappa)
+    g = o.energy(s.X, grad=True)[1].ravel()
+    H = np.diag(np.repeat(s.mass, 3))
+    for v, mu, lam in zip(s.tet.astype(int), s.mu, s.lam):
+        Dm = (s.X[v[1:]] - s.X[v[0]]).T
+        G = np.linalg.inv(Dm)
+        G = np.vstack([-G.sum(axis=0), G])               # dF[r, c] / dx[a, r]
+        B = np.zeros((9, 12))                            # vec F index 3 c + r
+        for a in range(4):
+            for r in range(3):
+                B[r::3, 3 * a + r] = G[a]
+        at = (3 * v[:, None] + np.arange(3)).ravel()
+        H[np.ix_(at, at)] += h2 * abs(np.linalg.det(Dm)) / 6 * (B.T @ O.nh_density(np.eye(3), mu, lam)[2] @ B)
+    contact = set()
+    for row, t, d in zip(*o.queries()):
+        if d > p.dhat ** 2:
+            continue
+        v = row[1:5].astype(int)
+        _, gd, Hd = O.ipc_distance(int(row[0]), int(t), s.X[v].reshape(12))
+        _, d1, d2 = O.ipc_barrier(d, p.dhat, kappa)
+        at = (3 * v[:, None] + np.arange(3)).ravel()
+        H[np.ix_(at, at)] += O.ipc_make_pd(h2 * (d2 * np.outer(gd, gd) + d1 * Hd))
+        contact.update(int(u) for u in v if not fixed[u])
+    fx = np.repeat(fixed, 3)
+    g[fx] = 0.0
+    H[fx] = 0.0
+    H[:, fx] = 0.0
+    H[fx, fx] = 1.0
+    return g, H, contact
+
+
+def morton_order(X):
+    """The vertices along a Morton curve (x highest) over cells of half the
+    box's edge per cube root of the vertex count, equal cells by vertex."""
+    cell = 0.5 * (X.max(axis=0) - X.min(axis=0)).max() / np.cbrt(len(X))
+    c = np.floor(X / cell).astype(np.int64) + (1 << 20)
+    key = [sum(((int(c[v, a]) >> b) & 1) << (3 * b + 2 - a) for b in range(21) for a in range(3)) for v in range(len(X))]
+    return sorted(range(len(X)), key=lambda v: (key[v], v))
+
+
+@pytest.mark.parametrize("stiffness", [1.0, -1.0])
+@pytest.mark.parametrize("n", [1, 2])
+def test_preconditioner(gpu, n, stiffness):
+    """One PCG iteration moves the positions along M^-1 g: with positive definite
+    blocks (one of 12 vertices; 32 and 2), their inverses on the contact vertices
+    and the diagonal elsewhere; with a negative shear modulus of the upper cube
+    the blocks are indefinite, and the diagonal everywhere.  Up to a common factor (the step length), to 1e-8: the
+    positions' rounding (1e-16 of 1e-3 moved) and the Hessian's, times the
+    blocks' condition numbers, at most 1e4."""
+    s = mesh.stack_scene(n, gap=2e-4, jitter=2e-4)
+    s.mu[s.body_tet_start[1]:] *= stiffness
+    p = IpcParams(dt=0.01, dhat=1e-3, tol=1e-3, maxIterations=1, lin_max_iter=1)
+    data = IpcData(s)
+    solver = IpcSolver(data, elastic="neohookean")
+    solver.Update(data, p)
+    st = solver.stats()
+    moved = (s.X - data.get("X")).ravel()
+    solver.close()
+    data.free()
+    g, H, contact = newton_system(s, p, st["kappa"])
+    assert st["linear_iterations"] == 2 and np.abs(moved).max() > 1e-9
+    z = g / np.diag(H)
+    order = [v for v in morton_order(s.X) if v in contact]
+    assert len(order) == len(contact) == {1: 12, 2: 34}[n]
+    for k in range(0, len(order), 32):
+        at = (3 * np.array(order[k:k + 32])[:, None] + np.arange(3)).ravel()
+        block = H[np.ix_(at, at)]
+        if stiffness > 0:
+            assert np.linalg.eigvalsh(block)[0] > 0
+            z[at] = np.linalg.solve(block, g[at])
+        else:
+            assert np.linalg.eigvalsh(block)[0] < 0
+    assert z @ H @ z > 0  # the iteration is taken
+    scale = (moved @ z) / (z @ z)
+    assert scale > 0 and np.abs(moved - scale * z).max() <= 1e-8 * np.abs(moved).max()

@@ -15,8 +15,8 @@ template <class V> void put(const char* name, const V& v) {
 }
 
 int main() {
-    int nv = 0, nnz = 0, rpg = 0, stride = 0;
-    std::cin >> nv >> nnz >> rpg >> stride;
+    int nv = 0, nnz = 0, rpg = 0, stride = 0, lanes = 0;
+    std::cin >> nv >> nnz >> rpg >> stride >> lanes;
     std::vector<int> rowstart(nv + 1);
     std::vector<uint32_t> cols(nnz);
     std::vector<double> X(3 * (size_t)nv);
@@ -32,7 +32,7 @@ int main() {
     try {
         const sbs::HaloTiles h = sbs::build_halo_tiles(
             nv, rowstart, cols, [&](int v) { return sbs::morton_code(&X[3 * (size_t)v], lo, hi); },
-            [](int k) { return (int64_t)k; }, rpg, stride);
+            [](int k) { return (int64_t)k; }, rpg, stride, lanes);
         std::printf("max_halo %d\nmax_width %d\n", h.max_halo, h.max_width);
         std::vector<uint32_t> keys(nv);
         for (int v = 0; v < nv; ++v) keys[v] = sbs::morton_code(&X[3 * (size_t)v], lo, hi);

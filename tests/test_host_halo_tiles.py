@@ -39,9 +39,9 @@ def pattern(tet, nv, diagonal=True):
     return np.cumsum(rowstart), cols
 
 
-def run(exe, rowstart, cols, X, rpg=256, stride=768):
+def run(exe, rowstart, cols, X, rpg=256, stride=768, lanes=1):
     nv = len(rowstart) - 1
-    text = f"{nv} {len(cols)} {rpg} {stride}\n" + " ".join(map(str, rowstart)) + "\n" + \
+    text = f"{nv} {len(cols)} {rpg} {stride} {lanes}\n" + " ".join(map(str, rowstart)) + "\n" + \
         " ".join(map(str, cols)) + "\n" + " ".join(repr(float(x)) for x in np.asarray(X).ravel()) + "\n"
     p = subprocess.run([exe], input=text, capture_output=True, text=True)
     if p.returncode != 0:
@@ -65,7 +65,7 @@ def morton(X):
     return code
 
 
-def check_tiles(h, rowstart, cols, X, rpg, stride):
+def check_tiles(h, rowstart, cols, X, rpg, stride, lanes=1):
     nv = len(rowstart) - 1
     perm, row_of = h["row_perm"], h["row_of"]
     assert np.array_equal(np.sort(perm), np.arange(nv))
@@ -95,10 +95,11 @@ def check_tiles(h, rowstart, cols, X, rpg, stride):
         assert (halo[g, hn[g]:] == row0[g]).all()
         own = h["g_own0"][g] + np.arange(rows[g])                        # the rows' own halo-local columns
         assert np.array_equal(halo[g, own], r)
-        assert width[g] == rl[verts].max()
+        assert width[g] == -(-rl[verts].max() // lanes)  # a thread's entries
         base = eptr[g]
         for t in range(rpg):
-            e = base + np.arange(width[g]) * rpg + t
+            k = np.arange(width[g] * lanes)  # entries of the row, dealt to its lanes
+            e = base + k // lanes * (rpg * lanes) + t * lanes + k % lanes
             if t < rows[g]:
                 v = verts[t]
                 n = rl[v]
@@ -114,7 +115,7 @@ def check_tiles(h, rowstart, cols, X, rpg, stride):
             nv_next = morton_order[row0[g] + rows[g]]
             more = np.concatenate([nb, [row_of[nv_next]], row_of[cols[rowstart[nv_next]:rowstart[nv_next + 1]]]])
             assert len(np.unique(more)) > stride, g
-    assert eptr[-1] + width[-1] * rpg == len(col) == len(src)
+    assert eptr[-1] + width[-1] * rpg * lanes == len(col) == len(src)
 
 
 def test_cube_tiles(driver):
@@ -137,6 +138,27 @@ def test_multi_body_tiles_tight_halo(driver):
     assert rc == 0
     check_tiles(h, rs, cols, s.X, 64, 90)
     assert (h["g_rows"][:-1] < 64).any()          # the capacity did cut some workgroups
+
+
+@pytest.mark.parametrize("nv", [64, 200, 1500])
+def test_four_lanes_per_row(driver, nv):
+    """Rows of entries dealt to four lanes, 64 rows and 512 halo slots per
+    workgroup: rows of every remainder of four, exactly one workgroup, a last one
+    that is partly filled, workgroups cut by their halo; no lanes are refused."""
+    rng = np.random.default_rng(nv)
+    X = rng.uniform(size=(nv, 3))
+    near = np.argsort(((X[:, None] - X[None]) ** 2).sum(-1), axis=1)[:, :13]
+    pairs = np.concatenate([np.stack([np.repeat(i, k), near[i, :k]], 1) for i, k in enumerate(rng.integers(1, 14, nv))])
+    key = np.unique(np.concatenate([pairs, pairs[:, ::-1]]) @ [nv, 1])
+    rs = np.searchsorted(key // nv, np.arange(nv + 1))
+    cols = key % nv
+    assert set(np.diff(rs) % 4) == {0, 1, 2, 3}
+    stride = 512 if nv < 1500 else 150
+    rc, h = run(driver, rs, cols, X, 64, stride, 4)
+    assert rc == 0
+    check_tiles(h, rs, cols, X, 64, stride, 4)
+    assert (nv < 1500) or (h["g_rows"][:-1] < 64).any()
+    assert run(driver, rs, cols, X, 64, stride, 0)[0] == 3
 
 
 def test_off_diagonal_pattern(driver):

@@ -35,7 +35,7 @@ constexpr int kRegWidth = 16;  // widest matrix row kept in registers
 
 template <class T> struct BatchArgs {
     const int* vptr;      // first vertex of each body
-    const int* eptr;      // first matrix entry
+    const int* eptr;      // first pair of matrix entries
     const int* ew;        // entries per row
     const int* orig;      // the caller's number of the body
     const int* vbody;     // body of each vertex
@@ -170,7 +170,7 @@ __device__ __forceinline__ void batch_solve_body(const BatchArgs<T>& a, int b, i
     constexpr int KR = K > 0 ? K : 1;
     constexpr bool kDiag = K > 0 && K * sizeof(T) <= 16;  // the diagonal and its inverse in registers
     typedef T V2 __attribute__((ext_vector_type(2)));
-    const size_t ebase = (size_t)__builtin_amdgcn_readfirstlane(a.eptr[b]);
+    const size_t ebase = 2 * (size_t)__builtin_amdgcn_readfirstlane(a.eptr[b]);
     // rows k B + tid: with the k B part in a uniform base and the thread's part a
     // 32-bit byte offset, a load needs one address register for all places
     const int B = K >= kFixedPlaces ? 1024 : blockDim.x;
@@ -579,15 +579,15 @@ template <class T> BatchEngine<T>::BatchEngine(const BatchSystem<T>& s) {
         const size_t n = (size_t)(vptr[b + 1] - vptr[b]);
         wide = wide || n > (size_t)kMaxNarrow;
         entries += n * (size_t)ew[b];
-        SBS_REQUIRE(entries < ((size_t)1 << 31), "batched PD: scene too large");
-        eptr[b + 1] = (int)entries;
+        SBS_REQUIRE(entries < ((size_t)1 << 32), "batched PD: scene too large");
+        eptr[b + 1] = (int)(entries / 2);
     }
     std::vector<uint16_t> ecol(std::max<size_t>(entries, 1));
     std::vector<uint32_t> ecol_wide(wide ? entries : 0);
     std::vector<T> eval(std::max<size_t>(entries, 1), (T)0);
     for (int b = 0; b < nb_; ++b) {
         const int n = vptr[b + 1] - vptr[b];
-        auto place_of = [&](int j, int il) { return (size_t)eptr[b] + 2 * ((size_t)(j / 2) * n + il) + (j & 1); };
+        auto place_of = [&](int j, int il) { return 2 * ((size_t)eptr[b] + (size_t)(j / 2) * n + il) + (j & 1); };
         auto set_col = [&](size_t pos, int col) {
             if (n > kMaxNarrow) ecol_wide[pos] = (uint32_t)(3 * col);
             else ecol[pos] = (uint16_t)(3 * col);

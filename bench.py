@@ -462,7 +462,7 @@ def config0_measure(steps: int = 100):
 def run_solver_workload(args, solver, n: int, kernel: str, label: str):
     """The 20-iteration PD step of an n^3 cube (the headline's body and
     parameters) on another global solver: Jacobi + Chebyshev (the reference's
-    default) or the direct band Cholesky.  The global-step kernel is timed
+    default) or the direct Cholesky solver.  The global-step kernel is timed
     with HIP events in as many steps again after the timed region."""
     scene = mesh.cube_scene(n, spacing=0.1, jitter=1e-3, seed=0, E=1e5, nu=0.3, density=1000.0, pin_top=True)
     print(f"# {label}: {scene.nv} vertices, {scene.nt} tets", file=sys.stderr, flush=True)
@@ -573,7 +573,7 @@ def main():
                     help="cube64: the headline 64^3 cube; dense256: 256 small bodies on the dense solver; "
                          "batched: 1024 uneven bodies in one engine vs per-body engines; "
                          "ipc: the FP64 IPC step on two 16^3 cubes in contact; jacobi64: the 64^3 cube on the "
-                         "Jacobi + Chebyshev global step; direct14, direct27: a 14^3 or 27^3 cube on the band Cholesky; "
+                         "Jacobi + Chebyshev global step; direct14, direct27: a 14^3 or 27^3 cube on the direct Cholesky; "
                          "collide: "
                          "two 24^3 cubes colliding, with fixed bodies")
     ap.add_argument("--per-body-sample", type=int, default=16, help="bodies timed as separate engines (batched)")
@@ -607,7 +607,7 @@ def main():
     if args.workload in ("direct14", "direct27"):
         # band factor (host), then its explicit inverse and the product with it (GPU)
         run_solver_workload(args, SolverType.CuSolverCholesky, int(args.workload[6:]), "direct_solve",
-                            "band Cholesky global step")
+                            "direct Cholesky global step")
         return
     if args.workload == "collide":
         run_collide_workload(args)

@@ -184,7 +184,8 @@ int sbs_pd_stats(SbsPd* pd, SbsPdStats* out);
 #define SBS_KERNEL_JACOBI_CHEBYSHEV 2
 #define SBS_KERNEL_DIRECT_SOLVE 3
 #define SBS_KERNEL_RHS_GATHER 4
-#define SBS_KERNEL_PCG_ITERATION 5     /* one launch per PCG iteration (+ stop probe) */
+#define SBS_KERNEL_PCG_ITERATION 5     /* one launch per PCG iteration (+ stop probe); none
+                                          up to 1,024 vertices, where a solve is one launch */
 #define SBS_KERNEL_COUNT 6
 int sbs_pd_set_kernel_timing(SbsPd* pd, unsigned mask);
 int sbs_pd_kernel_time(SbsPd* pd, int kernel_id, const char** name, int* launches, double* ms);

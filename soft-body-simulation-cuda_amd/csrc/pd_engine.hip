@@ -2380,10 +2380,8 @@ int PdEngine<T>::launch_pcg(int gathered, const T* b, const T* x0, T* x, bool ch
     tick(kKPcg, true);
     if (small_pcg(params)) {
         SBS_REQUIRE(!defer_finish, "PCG: a solve in one workgroup is finished in it");
-        tick(kKPcgIter, true);
         hipLaunchKernelGGL(pcg_small_kernel<T>, dim3(1), dim3(ceil_div(nv_, 64) * 64), 0, stream_, a,
                            SmallEnd<T>{(int)cheb, (int)(skip != nullptr), params.tol});
-        tick(kKPcgIter, false, 1);
         tick(kKPcg, false);
         SBS_HIP(hipGetLastError());
         return 0;

@@ -104,7 +104,8 @@ enum KernelId : int {
     kKJacobi,
     kKDirect,
     kKRhs,
-    kKPcgIter,  // PCG iteration launches (the stop probe and launches after convergence included), timed per run
+    kKPcgIter,  // PCG iteration launches (the stop probe and launches after convergence included), timed per run;
+                // none where a solve is one launch
     kKCount
 };
 const char* kernel_name(int id);

@@ -88,3 +88,21 @@ def test_graph_is_captured_once(gpu, mode):
     if mode == "early exit":
         assert se.pcg_solves_total < 8 * 8
     assert se.graph_captures == 0 and se.graph_replays == 0
+
+
+def test_kernel_timing_counts_solves(gpu):
+    """A solve is one launch: the timer has whole solves and no iteration launches."""
+    data = SolverData(body(4, 5, 6), 32)
+    pd = PdSolver(128, data)
+    pd.SetGlobalSolver(SolverType.PCG)
+    pd.set_kernel_timing(("local_step", "pcg_iteration", "pcg_solve"))
+    try:
+        for _ in range(2):
+            pd.Update(data, SolverParams(numIterations=5, dt=1.0 / 60.0, tol=0.0, pcg_chebyshev=True))
+        assert pd.kernel_time("local_step")[0] == 10
+        launches, ms = pd.kernel_time("pcg_solve")
+        assert launches == 10 and ms > 0
+        assert pd.kernel_time("pcg_iteration") == (0, 0.0)
+    finally:
+        pd.close()
+        data.free()

@@ -1274,9 +1274,7 @@ template <class T> __device__ __forceinline__ void iter_args(const PcgArgs<T>& a
 template <class T, bool kFirst>
 __global__ void __launch_bounds__(kTpb) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 5 : 1)))
 pcg_iter_halo_kernel(PcgArgs<T> a, int i) {
-    
     iter_args(a, i);
-    
     __shared__ T lu[3][kHaloStride];
     const unsigned g = xcd_block(blockIdx.x, gridDim.x);
     const int gdl = halo_group_lane(a.h, g);

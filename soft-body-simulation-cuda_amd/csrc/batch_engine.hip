@@ -635,8 +635,8 @@ template <class T> BatchEngine<T>::BatchEngine(const BatchSystem<T>& s) {
     // whatever other bodies there are.
     std::vector<std::vector<int>> tets_of(nb_);
     for (int t = 0; t < nt_; ++t) tets_of[place[number[s.tets[4 * (size_t)t]]]].push_back(t);
-    std::vector<int> seq, starts, rest;
-    std::vector<size_t> rest_n;
+    std::vector<int> seq, starts;
+    std::vector<std::vector<int>> rest(nb_);
     std::vector<std::pair<uint32_t, int>> key;
     for (int b = 0; b < nb_; ++b) {
         double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
@@ -658,16 +658,31 @@ template <class T> BatchEngine<T>::BatchEngine(const BatchSystem<T>& s) {
             if (i % kChunkTets == 0) starts.push_back((int)seq.size());
             seq.push_back(key[i].second);
         }
-        for (size_t i = whole; i < key.size(); ++i) rest.push_back(key[i].second);
-        rest_n.push_back(key.size() - whole);
+        for (size_t i = whole; i < key.size(); ++i) rest[b].push_back(key[i].second);
     }
-    for (size_t b = 0, r = 0, room = 0; b < rest_n.size(); ++b) {  // room: of the last shared chunk
-        if (rest_n[b] > room) {
-            starts.push_back((int)seq.size());
-            room = kChunkTets;
+    // largest rests first, each into the shared chunk with the least room that
+    // takes it (taken in body order they would leave a quarter of them idle)
+    std::vector<int> by_rest(nb_);
+    std::iota(by_rest.begin(), by_rest.end(), 0);
+    std::stable_sort(by_rest.begin(), by_rest.end(), [&](int x, int y) { return rest[x].size() > rest[y].size(); });
+    std::vector<std::vector<int>> shared, with_room(kChunkTets + 1);  // with_room[r]: shared chunks with room for r more
+    for (int b : by_rest) {
+        size_t r = rest[b].size();
+        if (r == 0) break;
+        while (r < with_room.size() && with_room[r].empty()) ++r;
+        int c = (int)shared.size();
+        if (r < with_room.size()) {
+            c = with_room[r].back();
+            with_room[r].pop_back();
+        } else {
+            shared.emplace_back();
         }
-        room -= rest_n[b];
-        for (size_t e = r + rest_n[b]; r < e; ++r) seq.push_back(rest[r]);
+        shared[c].insert(shared[c].end(), rest[b].begin(), rest[b].end());
+        with_room[kChunkTets - shared[c].size()].push_back(c);
+    }
+    for (const auto& c : shared) {
+        starts.push_back((int)seq.size());
+        seq.insert(seq.end(), c.begin(), c.end());
     }
     starts.push_back((int)seq.size());
     const int nt = (int)seq.size();

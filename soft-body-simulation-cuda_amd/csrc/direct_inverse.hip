@@ -164,10 +164,12 @@ __device__ __forceinline__ double slot_sum(const double* slots, unsigned pitch, 
 // thread takes 4 consecutive columns of every 1,024: one 4-value load per
 // row and right-hand side, kRowsPer + 3 of them in flight.  Per thread the
 // products are summed in the solve precision (n / 1024 of them), then 16
-// lanes, then the 16 row totals in double.  HBM / MALL bound: 45 MB for 3,360
-// rows in 8.0 us (5.6 TB/s; the band solve 227 us), 2.1 MB for 729 rows in
-// 5.1 us (77 us).  With the outer loop's error and decision taken along (two
-// launches of 4 us each before), an iteration is three launches.
+// lanes, then the 16 row totals in double.  A launch that runs (not skipped by
+// the early exit): 2.1 MB for 729 rows in 7.7 us, 45 MB for 3,360 rows in 13.7
+// (3.3 TB/s), 1.9 GB for 21,952 rows in 340 (5.7 TB/s: HBM bound there, below
+// it the launch, one round of loads and the ticket).  With the outer loop's
+// error and decision taken along (two launches of 4 us each before), an
+// iteration is three launches.
 template <class T, bool kOuter>
 __global__ void __launch_bounds__(kThreads) inverse_apply_kernel(
     const int4* __restrict__ job, const long long* __restrict__ job_off, const T* __restrict__ inv,

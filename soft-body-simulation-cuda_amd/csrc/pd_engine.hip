@@ -1377,8 +1377,9 @@ pcg_iter_halo_kernel(PcgArgs<T> a, int i) {
 // overlap.  What bounds a launch is that chain: launch, halo indices, halo
 // rows, product, reduction.
 constexpr int kQuadRows = kTpb / 4;
-// FP64 up to this many rows (measured, a step of 10 PCG solves with 256-row
-// workgroups and with these: 336 rows 1835 -> 1430 us, 2,197 rows 2204 -> 1522,
+// FP64 from kSmallRows (whose systems one workgroup solves) up to this many rows
+// (measured, a step of 10 PCG solves with 256-row workgroups and with these:
+// 336 rows 1835 -> 1430 us, 2,197 rows 2204 -> 1522,
 // 11,960 rows 2285 -> 1552, 24,389 rows 2395 -> 1928; 50,653 rows 2611 -> 2802:
 // there the chip is full and a smaller workgroup's larger share of halo rows
 // costs more).  FP32 would gain 1.1-1.25x in the same range, but a row's sum in
